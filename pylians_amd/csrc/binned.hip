@@ -14,6 +14,8 @@
 //             cell sum is exact to float64, the "compensated" accumulator) the stencil weights that
 //             fall inside the tile, from its own particles and from those of its 7 lower neighbours
 //             whose class reaches it, then writes every cell once with one rounding.
+// The grid edge need not be a multiple of TILE: a ragged edge N is cut into nt = ceil(N / TILE) tiles of
+// nearly equal width (TILE / 2 to TILE cells), tile t of cell c being floor(c nt / N).
 // Output modes: accumulate into the existing grid (MAS_library.MA semantics), overwrite, or the
 // overdensity delta = rho * a - 1 (a = N^3 / mass) evaluated in float64 before the single rounding.
 #include <math.h>
@@ -149,14 +151,18 @@ __device__ __forceinline__ int wrapN(double b, int N) {
 }
 
 
+// ceil(2^32 nt / N): c * tile_mul(N, nt) >> 32 = floor(c nt / N) for 0 <= c < N + 4 and N < 65536 (the
+// rounding of the factor adds less than (N + 4) / 2^32 < 1 / N, the smallest distance below an integer)
+static unsigned tile_mul(int N, int nt) { return (unsigned)((((unsigned long long)nt << 32) + N - 1) / N); }
+
 template <int S>
 __device__ __forceinline__ int halo_class(int bx, int by, int bz) {
     return ((bx % TILE) > TILE - S ? 1 : 0) | ((by % TILE) > TILE - S ? 2 : 0) | ((bz % TILE) > TILE - S ? 4 : 0);
 }
 
 // AGG: 0 every lane counts itself, 1 runs of equal keys are counted once, 2 a.agg decides (batched
-// launches, whose jobs differ)
-template <int S, bool HASW, int AGG>
+// launches, whose jobs differ; ragged grids).  RAG: the grid edge is no multiple of TILE.
+template <int S, bool HASW, int AGG, bool RAG>
 __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
     constexpr int R = HASW ? 4 : 3;
     constexpr long long PS = (long long)BT * KP;   // particles per step
@@ -166,7 +172,10 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
     __shared__ int hused[BT * KP];   // slots that hold a key this step, in insertion order
     __shared__ unsigned nused;
     __shared__ int scap[8], scofs[8];
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x;
+    const bool grouped = a.sel && *a.sel;
+    const float* __restrict__ pos = grouped ? a.spos : a.pos;
+    const float* __restrict__ W = grouped ? a.sw : a.W;
     if (tid < 8) {
         scap[tid] = a.cap[tid];
         scofs[tid] = a.cofs[tid];
@@ -185,7 +194,7 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
         for (int k = 0; k < KP; ++k) {
             const long long p = step * PS + k * BT + tid;
             if (p < a.n) {
-                float c[3] = {a.pos[3 * p], a.pos[3 * p + 1], a.pos[3 * p + 2]};
+                float c[3] = {pos[3 * p], pos[3 * p + 1], pos[3 * p + 2]};
                 if (a.rsd.vel) {
                     const int ax = a.rsd.axis;
                     c[ax] = rsd_shift(c[ax], a.rsd.vel[3 * p + ax], a.rsd.fac, a.rsd.box);
@@ -193,7 +202,7 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
                 px[k] = c[0];
                 py[k] = c[1];
                 pz[k] = c[2];
-                pw[k] = HASW ? a.W[p] : 0.f;
+                pw[k] = HASW ? W[p] : 0.f;
             }
         }
     };
@@ -234,7 +243,17 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
                 const int bx = wrapN(Axis<S>::eval((double)x[k] * a.inv, ww), a.N);
                 const int by = wrapN(Axis<S>::eval((double)y[k] * a.inv, ww), a.N);
                 const int bz = wrapN(Axis<S>::eval((double)z[k] * a.inv, ww), a.N);
-                key[k] = (((bx / TILE) * a.nt + by / TILE) * a.nt + bz / TILE) * 8 + halo_class<S>(bx, by, bz);
+                if (RAG) {
+                    // the stencil reaches into the next tile when its last cell lies there (tile nt
+                    // past the periodic edge)
+                    const unsigned m = a.tmul;
+                    const int tx = __umulhi(bx, m), ty = __umulhi(by, m), tz = __umulhi(bz, m);
+                    const int hc = (int)__umulhi(bx + S - 1, m) - tx + 2 * ((int)__umulhi(by + S - 1, m) - ty) +
+                                   4 * ((int)__umulhi(bz + S - 1, m) - tz);
+                    key[k] = ((tx * a.nt + ty) * a.nt + tz) * 8 + hc;
+                } else {
+                    key[k] = (((bx / TILE) * a.nt + by / TILE) * a.nt + bz / TILE) * 8 + halo_class<S>(bx, by, bz);
+                }
             }
             // at most BT * KP distinct keys per step in HT slots: the probe always ends
             auto probe = [&](int kk) {
@@ -309,13 +328,13 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
     }
 }
 
-template <int S, bool HASW, int AGG>
-__global__ __launch_bounds__(BT) void k_bin(BinArgs a) { bin_body<S, HASW, AGG>(a, own_blk()); }
+template <int S, bool HASW, int AGG, bool RAG>
+__global__ __launch_bounds__(BT) void k_bin(BinArgs a) { bin_body<S, HASW, AGG, RAG>(a, own_blk()); }
 template <int S, bool HASW>
 __global__ __launch_bounds__(BT) void k_bin_b(const BinArgs* __restrict__ tab,
                                                  const unsigned* __restrict__ start, int nj) {
     PYL_BATCH_BLK(start, nj);
-    bin_body<S, HASW, 2>(tab[bj_], blk_);
+    bin_body<S, HASW, 2, false>(tab[bj_], blk_);
 }
 
 // overflow grouping: count per tile, exclusive scan, scatter (records copied from the inputs)
@@ -368,17 +387,21 @@ template <bool HASW>
 __device__ __forceinline__ void ov_scatter_body(const OvArgs& a, Blk B) {
     constexpr int R = HASW ? 4 : 3;
     const long long n = *a.ov_count;
+    if (n == 0) return;
+    const bool sel = a.sel && *a.sel;
+    const float* __restrict__ pos = sel ? a.spos : a.pos;
+    const float* __restrict__ W = sel ? a.sw : a.W;
     for (long long i = (long long)B.x * blockDim.x + threadIdx.x; i < n; i += (long long)B.gx * blockDim.x) {
         const unsigned key = a.ov_key[i], t = key >> 3;
         const long long p = a.ov_idx[i];
         const unsigned s = a.ooff[t] + atomicAdd(&a.ocur[t], 1u);
         float* r = a.grouped + (long long)s * R;
-        float c[3] = {a.pos[3 * p], a.pos[3 * p + 1], a.pos[3 * p + 2]};
+        float c[3] = {pos[3 * p], pos[3 * p + 1], pos[3 * p + 2]};
         if (a.rsd.vel) c[a.rsd.axis] = rsd_shift(c[a.rsd.axis], a.rsd.vel[3 * p + a.rsd.axis], a.rsd.fac, a.rsd.box);
         r[0] = c[0];
         r[1] = c[1];
         r[2] = c[2];
-        if (HASW) r[3] = a.W[p];
+        if (HASW) r[3] = W[p];
         a.gcls[s] = key & 7u;
     }
 }
@@ -403,15 +426,20 @@ __device__ __forceinline__ void put(G* __restrict__ grid, long long g, double rh
 }
 
 
-// the stencil weights of one particle that fall inside the tile with lowest cell (ox, oy, oz)
+// lowest cell and width (cells, at most TILE) of a tile along each axis
+struct TileBox {
+    int ox, oy, oz, ex, ey, ez;
+};
+
+// the stencil weights of one particle that fall inside the tile t
 // (CLIP = false: a particle of the tile itself whose stencil stays inside it)
 template <int S, bool HASW, bool CLIP, bool UNIT>
-__device__ __forceinline__ void accumulate(double* acc, const float* r, int N, int ox, int oy, int oz, double inv,
+__device__ __forceinline__ void accumulate(double* acc, const float* r, int N, const TileBox& t, double inv,
                                            double mult) {
     double w0[S], w1[S], w2[S];
-    int l0 = wrapN(Axis<S>::eval((double)r[0] * inv, w0), N) - ox;
-    int l1 = wrapN(Axis<S>::eval((double)r[1] * inv, w1), N) - oy;
-    int l2 = wrapN(Axis<S>::eval((double)r[2] * inv, w2), N) - oz;
+    int l0 = wrapN(Axis<S>::eval((double)r[0] * inv, w0), N) - t.ox;
+    int l1 = wrapN(Axis<S>::eval((double)r[1] * inv, w1), N) - t.oy;
+    int l2 = wrapN(Axis<S>::eval((double)r[2] * inv, w2), N) - t.oz;
     // a particle of the lower neighbour across the periodic boundary
     if (l0 >= TILE) l0 -= N;
     if (l1 >= TILE) l1 -= N;
@@ -420,17 +448,17 @@ __device__ __forceinline__ void accumulate(double* acc, const float* r, int N, i
 #pragma unroll
     for (int l = 0; l < S; ++l) {
         const int c0 = l0 + l;
-        if (CLIP && (c0 < 0 || c0 >= TILE)) continue;
+        if (CLIP && (unsigned)c0 >= (unsigned)t.ex) continue;
 #pragma unroll
         for (int m = 0; m < S; ++m) {
             const int c1 = l1 + m;
-            if (CLIP && (c1 < 0 || c1 >= TILE)) continue;
+            if (CLIP && (unsigned)c1 >= (unsigned)t.ey) continue;
             const double wlm = UNIT ? w0[l] * w1[m] : w0[l] * w1[m] * ww;   // UNIT: no weights, mult == 1
             double* row = acc + (c0 * TILE + c1) * TROW;
 #pragma unroll
             for (int q = 0; q < S; ++q) {
                 const int c2 = l2 + q;
-                if (!CLIP || (c2 >= 0 && c2 < TILE)) atomicAdd(row + c2, wlm * w2[q]);
+                if (!CLIP || (unsigned)c2 < (unsigned)t.ez) atomicAdd(row + c2, wlm * w2[q]);
             }
         }
     }
@@ -439,12 +467,12 @@ __device__ __forceinline__ void accumulate(double* acc, const float* r, int N, i
 // accumulate() with the 1-D weights and their products in float32 (Axis32); each contribution is
 // added to the float64 LDS cell
 template <int S, bool HASW, bool CLIP, bool UNIT>
-__device__ __forceinline__ void accumulate32(double* acc, const float* r, int N, int ox, int oy, int oz, double inv,
+__device__ __forceinline__ void accumulate32(double* acc, const float* r, int N, const TileBox& t, double inv,
                                              float mult) {
     float w0[S], w1[S], w2[S];
-    int l0 = wrapN(Axis32<S>::eval((double)r[0] * inv, w0), N) - ox;
-    int l1 = wrapN(Axis32<S>::eval((double)r[1] * inv, w1), N) - oy;
-    int l2 = wrapN(Axis32<S>::eval((double)r[2] * inv, w2), N) - oz;
+    int l0 = wrapN(Axis32<S>::eval((double)r[0] * inv, w0), N) - t.ox;
+    int l1 = wrapN(Axis32<S>::eval((double)r[1] * inv, w1), N) - t.oy;
+    int l2 = wrapN(Axis32<S>::eval((double)r[2] * inv, w2), N) - t.oz;
     if (l0 >= TILE) l0 -= N;
     if (l1 >= TILE) l1 -= N;
     if (l2 >= TILE) l2 -= N;
@@ -452,17 +480,17 @@ __device__ __forceinline__ void accumulate32(double* acc, const float* r, int N,
 #pragma unroll
     for (int l = 0; l < S; ++l) {
         const int c0 = l0 + l;
-        if (CLIP && (c0 < 0 || c0 >= TILE)) continue;
+        if (CLIP && (unsigned)c0 >= (unsigned)t.ex) continue;
 #pragma unroll
         for (int m = 0; m < S; ++m) {
             const int c1 = l1 + m;
-            if (CLIP && (c1 < 0 || c1 >= TILE)) continue;
+            if (CLIP && (unsigned)c1 >= (unsigned)t.ey) continue;
             const float wlm = UNIT ? w0[l] * w1[m] : w0[l] * w1[m] * ww;
             double* row = acc + (c0 * TILE + c1) * TROW;
 #pragma unroll
             for (int q = 0; q < S; ++q) {
                 const int c2 = l2 + q;
-                if (!CLIP || (c2 >= 0 && c2 < TILE)) atomicAdd(row + c2, (double)(wlm * w2[q]));
+                if (!CLIP || (unsigned)c2 < (unsigned)t.ez) atomicAdd(row + c2, (double)(wlm * w2[q]));
             }
         }
     }
@@ -541,7 +569,15 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
     }
     __syncthreads();
     const unsigned tot = sstart[NE];
-    const int ox = tx * TILE, oy = ty * TILE, oz = tz * TILE;
+    TileBox box{tx * TILE, ty * TILE, tz * TILE, TILE, TILE, TILE};
+    if (a.rag) {
+        box.ox = (tx * a.N + nt - 1) / nt;
+        box.oy = (ty * a.N + nt - 1) / nt;
+        box.oz = (tz * a.N + nt - 1) / nt;
+        box.ex = ((tx + 1) * a.N + nt - 1) / nt - box.ox;
+        box.ey = ((ty + 1) * a.N + nt - 1) / nt - box.oy;
+        box.ez = ((tz + 1) * a.N + nt - 1) / nt - box.oz;
+    }
     // RP records per thread per step; the records of the next step load while those of this step
     // accumulate.  The loads are unconditional (an exhausted slot reads record 0 and class word 0,
     // both always allocated) and their values are first used a step later, so only they stay in
@@ -624,9 +660,9 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
             for (int k = 0; k < RG; ++k) {
                 if (g * RG + k >= n0) break;
                 double w0[S], w1[S], w2[S];
-                int l0 = wrapN(Axis<S>::eval((double)gr[k][0] * a.inv, w0), a.N) - ox;
-                int l1 = wrapN(Axis<S>::eval((double)gr[k][1] * a.inv, w1), a.N) - oy;
-                int l2 = wrapN(Axis<S>::eval((double)gr[k][2] * a.inv, w2), a.N) - oz;
+                int l0 = wrapN(Axis<S>::eval((double)gr[k][0] * a.inv, w0), a.N) - box.ox;
+                int l1 = wrapN(Axis<S>::eval((double)gr[k][1] * a.inv, w1), a.N) - box.oy;
+                int l2 = wrapN(Axis<S>::eval((double)gr[k][2] * a.inv, w2), a.N) - box.oz;
                 if (l0 >= TILE) l0 -= a.N;
                 if (l1 >= TILE) l1 -= a.N;
                 if (l2 >= TILE) l2 -= a.N;
@@ -686,9 +722,9 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
             for (int j = 0; j < RP; ++j) {
                 if (f + j * TT >= n0) break;
                 if (ACC == ACC_F32W)
-                    accumulate32<S, HASW, false, UNIT>(acc, cr[j], a.N, ox, oy, oz, a.inv, (float)a.mult);
+                    accumulate32<S, HASW, false, UNIT>(acc, cr[j], a.N, box, a.inv, (float)a.mult);
                 else
-                    accumulate<S, HASW, false, UNIT>(acc, cr[j], a.N, ox, oy, oz, a.inv, a.mult);
+                    accumulate<S, HASW, false, UNIT>(acc, cr[j], a.N, box, a.inv, a.mult);
             }
         }
     }
@@ -705,9 +741,9 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
             const unsigned d = (unsigned)(ej / 9);
             const bool ok = ej >= 0 && (ej % 9 < 8 || (cg[j] & d) == d);
             if (ACC == ACC_F32W) {
-                if (ok) accumulate32<S, HASW, true, UNIT>(acc, cr[j], a.N, ox, oy, oz, a.inv, (float)a.mult);
+                if (ok) accumulate32<S, HASW, true, UNIT>(acc, cr[j], a.N, box, a.inv, (float)a.mult);
             } else if (ok) {
-                accumulate<S, HASW, true, UNIT>(acc, cr[j], a.N, ox, oy, oz, a.inv, a.mult);
+                accumulate<S, HASW, true, UNIT>(acc, cr[j], a.N, box, a.inv, a.mult);
             }
         }
         advance();
@@ -718,7 +754,8 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
     const long long N = a.N;
     for (int idx = tid; idx < TILE * TILE * TILE; idx += TT) {
         const int i = idx / (TILE * TILE), j = (idx / TILE) % TILE, k = idx % TILE;
-        const long long g = (((long long)ox + i) * N + oy + j) * N + oz + k;
+        if (a.rag && (i >= box.ex || j >= box.ey || k >= box.ez)) continue;
+        const long long g = (((long long)box.ox + i) * N + box.oy + j) * N + box.oz + k;
         put<G, MODE>(grid, g, acc[(i * TILE + j) * TROW + k], am);
     }
 }
@@ -741,6 +778,8 @@ __global__ __launch_bounds__(TT) void k_tile_b(const TileArgs* __restrict__ tab,
 // then reads the grouped copy, where neighbouring particles share keys as in an ordered input.
 constexpr int PT = 512;   // presort kernels: threads per workgroup
 constexpr int PKP = 8;    // k_sup_scatter: particles per thread per step
+// particles from which the device looks for a spatial order (PRESORT_PROBE)
+constexpr int64_t PROBE_MIN = 1 << 20;
 
 
 __device__ __forceinline__ void sup_load(const SupArgs& a, long long p, float& x, float& y, float& z) {
@@ -764,9 +803,29 @@ __device__ __forceinline__ int sup_of(const SupArgs& a, float x, float y, float 
     return (((bx / TILE) * a.nt + by / TILE) * a.nt + bz / TILE) / a.tps;
 }
 
+// a.sel: the particles are grouped only when they are in no spatial order.  Every workgroup looks at
+// the same PT pairs of consecutive particles (read from L2 after the first) and takes them for unordered
+// when more than half of the pairs lie in different tiles (lattice order: 1 pair in TILE, or a few with large
+// displacements; unordered: all but one in ntiles).  Returns whether to group; workgroup 0 notes it.
+__device__ __forceinline__ bool sup_probe(const SupArgs& a, Blk B) {
+    if (!a.sel) return true;
+    const long long p = (a.n - 1) * (long long)threadIdx.x / PT;   // pair (p, p + 1), p < n - 1
+    const float inv = (float)a.inv;
+    bool diff = false;
+    if (p + 1 < a.n) {
+        const float* r = a.pos + 3 * p;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) diff |= sup_cell(r[c], inv, a.N) / TILE != sup_cell(r[3 + c], inv, a.N) / TILE;
+    }
+    const bool group = 2 * __syncthreads_count(diff) > PT;
+    if (B.x == 0 && threadIdx.x == 0) *a.sel = group ? 1u : 0u;
+    return group;
+}
+
 template <int S>
 __device__ __forceinline__ void sup_count_body(const SupArgs& a, Blk B) {
     __shared__ unsigned h[SUPMAX];
+    if (!sup_probe(a, B)) return;
     for (int i = threadIdx.x; i < a.nsup; i += PT) h[i] = 0u;
     __syncthreads();
     for (long long p = (long long)B.x * PT + threadIdx.x; p < a.n; p += (long long)B.gx * PT) {
@@ -790,7 +849,7 @@ __global__ __launch_bounds__(PT) void k_sup_count_b(const SupArgs* __restrict__ 
 
 // exclusive scan of the nsup <= SUPMAX counts (one workgroup of SUPMAX threads)
 __device__ __forceinline__ void sup_scan_body(const unsigned* __restrict__ cnt, unsigned* __restrict__ off, int nsup) {
-    __shared__ unsigned wsum[SUPMAX / 64];
+    __shared__ unsigned wsum[SUPMAX / 64];   // (nothing was grouped: scans zeros)
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const unsigned c = tid < nsup ? cnt[tid] : 0u;
     unsigned v = c;
@@ -820,6 +879,7 @@ __device__ __forceinline__ void sup_scatter_body(const SupArgs& a, Blk B) {
     constexpr long long PS = (long long)PT * PKP;
     __shared__ unsigned lc[SUPMAX], lb[SUPMAX];
     const int tid = threadIdx.x;
+    if (a.sel && !*a.sel) return;
     for (int i = tid; i < a.nsup; i += PT) lc[i] = 0u;
     __syncthreads();
     const long long nstep = (a.n + PS - 1) / PS;
@@ -874,6 +934,15 @@ __global__ __launch_bounds__(PT) void k_sup_scatter_b(const SupArgs* __restrict_
 
 // ------------------------------------------------------------------ host side
 bool binned_supported(int axes, int dims) { return axes == 3 && dims % TILE == 0 && dims >= 2 * TILE; }
+// grids whose edge is no multiple of TILE (see tile_mul for the upper limit)
+bool binned_ragged(int axes, int dims) { return axes == 3 && dims % TILE != 0 && dims >= 2 * TILE && dims < 32768; }
+
+// A grouped copy of the particles and the device word that tells whether it was made
+struct Presort {
+    const unsigned* sel = nullptr;
+    const float* pos = nullptr;
+    const float* W = nullptr;
+};
 
 // Bucket layout of one deposit: class segment capacities of twice the expected count of a uniform
 // distribution plus slack, and the bytes of the counters, buckets and overflow area.
@@ -886,10 +955,10 @@ struct Layout {
 
 static int layout_of(int64_t n, int dims, int S, bool hasw, Layout* L) {
     const int R = hasw ? 4 : 3;
-    L->nt = dims / TILE;
+    L->nt = (dims + TILE - 1) / TILE;
     L->ntiles = (long long)L->nt * L->nt * L->nt;
     const double avg = (double)n / (double)L->ntiles;
-    const double ph = (double)(S - 1) / TILE, p0 = 1.0 - ph;
+    const double ph = (double)(S - 1) * L->nt / dims, p0 = 1.0 - ph;
     L->CT = 0;
     for (int c = 0; c < 8; ++c) {
         const double f = ((c & 1) ? ph : p0) * ((c & 2) ? ph : p0) * ((c & 4) ? ph : p0);
@@ -909,12 +978,13 @@ static int layout_of(int64_t n, int dims, int S, bool hasw, Layout* L) {
 
 template <int S, typename G, bool HASW, int MODE>
 static int run_binned(const float* pos, const float* W, int64_t n, int dims, double BoxSize, double mult, void* grid,
-                      const double* dmass, double mass, hipStream_t st, const Rsd& rsd, int acc) {
+                      const double* dmass, double mass, hipStream_t st, const Rsd& rsd, int acc, const Presort& ps) {
     int rc = OK;
     Layout L;
     rc = layout_of(n, dims, S, HASW, &L);
     if (rc) return rc;
     const int nt = L.nt;
+    const bool rag = dims % TILE != 0;
     const long long ntiles = L.ntiles, CT = L.CT;
     const int *cap = L.cap, *cofs = L.cofs;
     const size_t ncnt = L.ncnt;
@@ -936,6 +1006,10 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
         StageTimer tm("deposit_bin", st);
         BinArgs ba{pos, W, (long long)n, dims, nt, dims / BoxSize, fill, bucket, CT, {}, {}, ov_count, ov_idx, ov_key, rsd};
         ba.agg = bin_agg(n, dims);
+        ba.tmul = tile_mul(dims, nt);
+        ba.sel = ps.sel;
+        ba.spos = ps.pos;
+        ba.sw = ps.W;
         for (int c = 0; c < 8; ++c) {
             ba.cofs[c] = cofs[c];
             ba.cap[c] = cap[c];
@@ -943,15 +1017,18 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
         long long blocks = (n + (long long)BT * KP - 1) / ((long long)BT * KP);
         if (blocks > 2048) blocks = 2048;
         blocks = (blocks + XCDS - 1) / XCDS * XCDS;
-        if (ba.agg)
-            hipLaunchKernelGGL((k_bin<S, HASW, 1>), dim3((unsigned)blocks), dim3(BT), 0, st, ba);
+        if (rag)
+            hipLaunchKernelGGL((k_bin<S, HASW, 2, true>), dim3((unsigned)blocks), dim3(BT), 0, st, ba);
+        else if (ba.agg)
+            hipLaunchKernelGGL((k_bin<S, HASW, 1, false>), dim3((unsigned)blocks), dim3(BT), 0, st, ba);
         else
-            hipLaunchKernelGGL((k_bin<S, HASW, 0>), dim3((unsigned)blocks), dim3(BT), 0, st, ba);
+            hipLaunchKernelGGL((k_bin<S, HASW, 0, false>), dim3((unsigned)blocks), dim3(BT), 0, st, ba);
         PYL_HIP(hipGetLastError());
     }
     {
         StageTimer tm("deposit_overflow", st);
-        const OvArgs oa{ov_count, ov_idx, ov_key, ocnt, ooff, ocur, pos, W, grouped, gcls, rsd, (int)ntiles};
+        const OvArgs oa{ov_count, ov_idx, ov_key, ocnt, ooff, ocur, pos, W, grouped, gcls, rsd, (int)ntiles,
+                        ps.sel, ps.pos, ps.W};
         hipLaunchKernelGGL(k_ov_count, dim3(256), dim3(256), 0, st, oa);
         hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, oa);
         hipLaunchKernelGGL((k_ov_scatter<HASW>), dim3(256), dim3(256), 0, st, oa);
@@ -960,7 +1037,7 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
     {
         StageTimer tm("deposit_tiles", st);
         TileArgs ta{bucket, fill, CT, {}, {}, grouped, gcls, ooff, ocnt, dims, nt, dims / BoxSize, mult, grid, dmass,
-                    mass};
+                    mass, rag ? 1 : 0};
         for (int c = 0; c < 8; ++c) {
             ta.cofs[c] = cofs[c];
             ta.cap[c] = cap[c];
@@ -987,19 +1064,20 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
 
 template <int S, typename G, int MODE>
 static int dispatch_w(const float* pos, const float* W, int64_t n, int dims, double BoxSize, double mult, void* grid,
-                      const double* dmass, double mass, hipStream_t st, const Rsd& rsd, int acc) {
-    return W ? run_binned<S, G, true, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc)
-             : run_binned<S, G, false, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc);
+                      const double* dmass, double mass, hipStream_t st, const Rsd& rsd, int acc, const Presort& ps) {
+    return W ? run_binned<S, G, true, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc, ps)
+             : run_binned<S, G, false, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc, ps);
 }
 
 template <typename G, int MODE>
 static int dispatch_s(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, double mult,
-                      void* grid, const double* dmass, double mass, hipStream_t st, const Rsd& rsd, int acc) {
+                      void* grid, const double* dmass, double mass, hipStream_t st, const Rsd& rsd, int acc,
+                      const Presort& ps) {
     switch (scheme) {
-        case 1: return dispatch_w<1, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc);
-        case 2: return dispatch_w<2, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc);
-        case 3: return dispatch_w<3, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc);
-        case 4: return dispatch_w<4, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc);
+        case 1: return dispatch_w<1, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc, ps);
+        case 2: return dispatch_w<2, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc, ps);
+        case 3: return dispatch_w<3, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc, ps);
+        case 4: return dispatch_w<4, G, MODE>(pos, W, n, dims, BoxSize, mult, grid, dmass, mass, st, rsd, acc, ps);
         default: set_error("unknown scheme %d", scheme); return E_ARG;
     }
 }
@@ -1014,25 +1092,26 @@ static void launch_presort(const SupArgs& a, bool hasw, unsigned blocks, unsigne
         hipLaunchKernelGGL((k_sup_scatter<S, false>), dim3(sblocks), dim3(PT), 0, st, a);
 }
 
-// groups the particles by supertile into library workspaces (*spos, *sw); the redshift-space shift
-// is applied on the way, so the grouped copy is deposited without it
+// groups the particles by supertile into library workspaces (ps->pos, ps->W); the redshift-space shift
+// is applied on the way, so the grouped copy is deposited without it.  probe: only when they are in no
+// spatial order, which the device decides (ps->sel)
 static int presort(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, const Rsd& rsd,
-                   hipStream_t st, const float** spos, const float** sw) {
+                   bool probe, hipStream_t st, Presort* ps) {
     int rc = OK;
-    const int nt = dims / TILE;
+    const int nt = (dims + TILE - 1) / TILE;
     const long long ntiles = (long long)nt * nt * nt;
     // supertiles of whole tile columns (nt tiles along z), about 128 of them and never more than SUPMAX
     long long tps = nt * std::max(1LL, (ntiles + 128LL * nt - 1) / (128LL * nt));
     while ((ntiles + tps - 1) / tps > SUPMAX) tps += nt;
     const int nsup = (int)((ntiles + tps - 1) / tps);
-    unsigned* cnt = (unsigned*)workspace(WS_SUP, sizeof(unsigned) * 3 * SUPMAX, &rc);
+    unsigned* cnt = (unsigned*)workspace(WS_SUP, sizeof(unsigned) * (3 * SUPMAX + 4), &rc);
     if (rc) return rc;
     float* sp = (float*)workspace(WS_STAGE, sizeof(float) * (size_t)n * (W ? 4 : 3) + 64, &rc);
     if (rc) return rc;
     rc = zero_fill(cnt, sizeof(unsigned) * 3 * SUPMAX, st);
     if (rc) return rc;
     SupArgs a{pos, W, (long long)n, dims, nt, (int)tps, nsup, dims / BoxSize, rsd, cnt, cnt + SUPMAX,
-              cnt + 2 * SUPMAX, sp, W ? sp + 3 * n : nullptr};
+              cnt + 2 * SUPMAX, sp, W ? sp + 3 * n : nullptr, probe ? cnt + 3 * SUPMAX : nullptr};
     long long blocks = (n + PT - 1) / PT;
     if (blocks > 2048) blocks = 2048;
     long long sblocks = (n + (long long)PT * PKP - 1) / ((long long)PT * PKP);
@@ -1046,8 +1125,9 @@ static int presort(const float* pos, const float* W, int64_t n, int dims, double
         default: set_error("unknown scheme %d", scheme); return E_ARG;
     }
     PYL_HIP(hipGetLastError());
-    *spos = sp;
-    *sw = a.sw;
+    ps->sel = a.sel;
+    ps->pos = sp;
+    ps->W = a.sw;
     return OK;
 }
 
@@ -1055,30 +1135,36 @@ static int presort(const float* pos, const float* W, int64_t n, int dims, double
 // accumulation of a float32 grid (ACC_F64 / ACC_F32W; float64 grids always use ACC_F64)
 int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, bool f64,
                    int mode, double mult, void* grid, const double* dmass, double mass, hipStream_t st,
-                   const Rsd& rsd_in, bool sorted, int acc) {
+                   const Rsd& rsd_in, int sorted, int acc) {
     PYL_CHECK(!rsd_in.vel || (rsd_in.axis >= 0 && rsd_in.axis <= 2), E_ARG, "redshift-space axis must be 0, 1 or 2");
-    PYL_CHECK(binned_supported(3, dims), E_UNSUPPORTED, "binned deposit needs 3-D grids with dims %% %d == 0", TILE);
+    PYL_CHECK(binned_supported(3, dims) || binned_ragged(3, dims), E_UNSUPPORTED,
+              "binned deposit needs 3-D grids of at least %d cells an edge", 2 * TILE);
     PYL_CHECK(n > 0, E_ARG, "binned deposit needs particles");
     PYL_CHECK(n < (1LL << 31), E_UNSUPPORTED, "binned deposit: at most 2^31 particles per call");
     Rsd rsd = rsd_in;
+    Presort ps;
+    if (sorted == PRESORT_PROBE && (rsd.vel || n < PROBE_MIN)) sorted = PRESORT_NO;
     if (sorted) {
-        const float *sp = nullptr, *sw = nullptr;
-        int rc = presort(pos, W, n, dims, BoxSize, scheme, rsd_in, st, &sp, &sw);
-        if (rc) return rc;
-        pos = sp;
-        W = sw;
-        rsd = Rsd();
+        const int rc = presort(pos, W, n, dims, BoxSize, scheme, rsd_in, sorted == PRESORT_PROBE, st, &ps);
+        if (rc && !(sorted == PRESORT_PROBE && rc == E_ALLOC)) return rc;
+        if (rc) ps = Presort();   // no room for the grouped copy: deposit the particles as they are
+        if (!rc && sorted == PRESORT_YES) {
+            pos = ps.pos;
+            W = ps.W;
+            rsd = Rsd();
+            ps = Presort();
+        }
     }
     if (f64) {
         const int a64 = dense_acc(ACC_F64, scheme, n, dims);
-        if (mode == OUT_ACC) return dispatch_s<double, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64);
-        if (mode == OUT_SET) return dispatch_s<double, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64);
-        return dispatch_s<double, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64);
+        if (mode == OUT_ACC) return dispatch_s<double, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, ps);
+        if (mode == OUT_SET) return dispatch_s<double, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, ps);
+        return dispatch_s<double, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, ps);
     }
     acc = dense_acc(acc, scheme, n, dims);
-    if (mode == OUT_ACC) return dispatch_s<float, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc);
-    if (mode == OUT_SET) return dispatch_s<float, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc);
-    return dispatch_s<float, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc);
+    if (mode == OUT_ACC) return dispatch_s<float, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc, ps);
+    if (mode == OUT_SET) return dispatch_s<float, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc, ps);
+    return dispatch_s<float, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc, ps);
 }
 
 // ------------------------------------------------------------------ batched deposit

@@ -24,6 +24,11 @@ struct BinArgs {
     unsigned* ov_key;    // [n]
     Rsd rsd;             // redshift-space shift of the positions (rsd.vel == nullptr: none)
     int agg = 0;         // runs of equal keys in consecutive lanes counted once (bin_agg)
+    unsigned tmul = 0;   // ragged grids: tile of cell c = c * tmul >> 32 (tile_mul)
+    // presort decided on the device: when sel is set and *sel != 0, the grouped copy is read instead
+    const unsigned* sel = nullptr;
+    const float* spos = nullptr;
+    const float* sw = nullptr;
 };
 
 struct TileArgs {
@@ -41,6 +46,7 @@ struct TileArgs {
     void* grid;
     const double* dmass;  // device mass (nullable) for OUT_DELTA
     double mass;
+    int rag = 0;          // ragged grid (N % TILE != 0): tile t holds the cells [ceil(t N / nt), ceil((t + 1) N / nt))
 };
 
 struct OvArgs {
@@ -56,6 +62,9 @@ struct OvArgs {
     unsigned* gcls;             // class of each grouped record
     Rsd rsd;
     int ntiles;
+    const unsigned* sel = nullptr;   // as in BinArgs
+    const float* spos = nullptr;
+    const float* sw = nullptr;
 };
 
 struct SupArgs {
@@ -70,6 +79,7 @@ struct SupArgs {
     unsigned* cur;   // [nsup] slots handed out so far
     float* spos;     // [n * 3] grouped positions (redshift-space shift applied)
     float* sw;       // [n] grouped weights (HASW)
+    unsigned* sel = nullptr;   // [1] nullable: written by the count, 1 = the particles were grouped
 };
 
 // One job of a batched binned deposit (overdensity output): the arguments of every stage and

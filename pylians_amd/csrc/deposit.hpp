@@ -55,11 +55,15 @@ int delta_round(const double* rho, float* out, int64_t n, const double* dmass, d
 // delta = rho * n / M - 1 in place on a float64 grid of n cells (M: dmass[0] when given, else mass)
 int delta_inplace(double* g, int64_t n, const double* dmass, double mass, hipStream_t st);
 
-// Cell-binned LDS deposit (3-D grids with dims % 16 == 0).  mode: 0 = grid += rho, 1 = grid = rho,
+// Cell-binned LDS deposit (3-D grids with dims % 16 == 0, or ragged ones of at least 32 cells an edge).  mode: 0 = grid += rho, 1 = grid = rho,
 // 2 = grid = rho * N^3 / mass - 1 with mass = dmass[0] when dmass != nullptr, else `mass`.
+// sorted: PRESORT_NO, PRESORT_YES (group the particles by supertile first), PRESORT_PROBE (group them when
+// they are many and in no spatial order, decided on the device).
 bool binned_supported(int axes, int dims);
+bool binned_ragged(int axes, int dims);
+enum { PRESORT_NO = 0, PRESORT_YES = 1, PRESORT_PROBE = 2 };
 int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, bool f64,
                    int mode, double mult, void* grid, const double* dmass, double mass, hipStream_t st,
-                   const Rsd& rsd = Rsd(), bool sorted = false, int acc = 0);
+                   const Rsd& rsd = Rsd(), int sorted = PRESORT_NO, int acc = 0);
 
 }  // namespace pyl

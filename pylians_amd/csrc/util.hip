@@ -2,7 +2,9 @@
 #include <stdarg.h>
 
 #include <map>
+#include <memory>
 #include <mutex>
+#include <vector>
 
 #include "common.hpp"
 #include "util.hpp"
@@ -107,6 +109,7 @@ static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc) {
     }
     size_t want = bytes < 256 ? 256 : bytes;
     if (hipMalloc(&e.first, want) != hipSuccess) {
+        (void)hipGetLastError();
         e.first = nullptr;
         set_error("workspace allocation of %zu bytes failed", want);
         *rc = E_ALLOC;
@@ -247,6 +250,52 @@ size_t ws_arena_bytes(const WsArena* a) {
     if (a)
         for (auto& kv : a->slots) s += kv.second.second;
     return s;
+}
+
+// Workspaces of the deposits that may run on several streams at once (stream_ws).  At most STREAM_WS
+// sets are kept; a further stream takes the place of the one used longest ago.
+constexpr size_t STREAM_WS = 4;
+struct StreamWs {
+    int dev;
+    hipStream_t st;
+    std::mutex mu;   // held while a call queues its kernels
+    WsArena* arena;
+    StreamWs(int d, hipStream_t s) : dev(d), st(s), arena(ws_arena_create()) {}
+    ~StreamWs() { ws_arena_destroy(arena); }
+};
+
+static std::shared_ptr<StreamWs> stream_ws(hipStream_t st) {
+    static std::mutex mu;
+    static std::vector<std::shared_ptr<StreamWs>>* sets = new std::vector<std::shared_ptr<StreamWs>>();
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    std::shared_ptr<StreamWs> old;   // freed (and its work waited for) after the lock is given back
+    std::lock_guard<std::mutex> lk(mu);
+    for (size_t i = 0; i < sets->size(); ++i)
+        if ((*sets)[i]->dev == dev && (*sets)[i]->st == st) {
+            std::shared_ptr<StreamWs> w = (*sets)[i];
+            sets->erase(sets->begin() + (long)i);
+            sets->push_back(w);
+            return w;
+        }
+    if (sets->size() >= STREAM_WS) {
+        old = sets->front();
+        sets->erase(sets->begin());
+    }
+    sets->push_back(std::make_shared<StreamWs>(dev, st));
+    return sets->back();
+}
+
+StreamScope::StreamScope(hipStream_t st) {
+    if (t_arena) return;   // a graph's or a fixed arena: that one
+    ws = stream_ws(st);
+    ws->mu.lock();
+    t_arena = ws->arena;
+}
+StreamScope::~StreamScope() {
+    if (!ws) return;
+    t_arena = nullptr;
+    ws->mu.unlock();
 }
 
 ArenaScope::ArenaScope(WsArena* a) : prev(t_arena) { t_arena = a; }

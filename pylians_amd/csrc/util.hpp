@@ -1,5 +1,7 @@
 // Zero-fill and workspace helpers.
 #pragma once
+#include <memory>
+
 #include "common.hpp"
 
 namespace pyl {
@@ -53,6 +55,16 @@ struct ArenaScope {
     explicit ArenaScope(WsArena* a);
     ~ArenaScope();
     WsArena* prev;
+};
+// While a StreamScope is alive on a thread, workspace() serves buffers that belong to the stream: for
+// calls that needed no workspace before (and so could run on several streams and threads at once).
+// Calls on one stream queue their kernels one after the other; the buffers of at most four streams are
+// kept, those of the stream used longest ago being freed for another one's.
+struct StreamWs;
+struct StreamScope {
+    explicit StreamScope(hipStream_t st);
+    ~StreamScope();
+    std::shared_ptr<StreamWs> ws;
 };
 
 }  // namespace pyl
