@@ -82,7 +82,7 @@ template <typename A> struct Table {
 struct DepClass {
     int scheme, prec, acc;
     bool hasw, sorted;
-    Table<SupArgs> sup, ssc;
+    Table<SupArgs> sup;
     Table<BinArgs> bin;
     Table<OvArgs> ov;
     Table<TileArgs> tile;
@@ -271,7 +271,6 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
                              J.kind == DK_SORTED, J.dep, &J.bj);
         if (rc) return rc;
         B->zero.add(ZeroArgs{J.bj.cnt, J.bj.cnt_bytes}, 0);
-        if (J.bj.scnt) B->zero.add(ZeroArgs{J.bj.scnt, J.bj.scnt_bytes}, 0);
         const int acc = dense_acc(f64 ? 0 : acc_mode(j.flags), j.scheme, j.n, j.dims);
         auto key = std::make_tuple(j.scheme, j.prec, acc, j.W ? 1 : 0, J.kind == DK_SORTED ? 1 : 0);
         DepClass& D = B->dep[key];
@@ -280,17 +279,14 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
         D.acc = acc;
         D.hasw = j.W != nullptr;
         D.sorted = J.kind == DK_SORTED;
-        if (D.sorted) {
-            D.sup.add(J.bj.sup, J.bj.sup_blocks);
-            D.ssc.add(J.bj.sup, J.bj.sup_sblocks);
-        }
+        if (D.sorted) D.sup.add(J.bj.sup, J.bj.sup_blocks);
         D.bin.add(J.bj.bin, J.bj.bin_blocks);
         D.ov.add(J.bj.ov, 0);
         D.tile.add(J.bj.tile, J.bj.tile_blocks);
     }
     // 4. device tables (a workspace slot of their own), uploaded now, before any capture
     size_t tb = B->zero.bytes();
-    for (auto& kv : B->dep) tb += kv.second.sup.bytes() + kv.second.ssc.bytes() + kv.second.bin.bytes() +
+    for (auto& kv : B->dep) tb += kv.second.sup.bytes() + kv.second.bin.bytes() +
                                   kv.second.ov.bytes() + kv.second.tile.bytes();
     for (auto& kv : B->fft32) tb += kv.second.r2c.bytes() + kv.second.cols.bytes();
     for (auto& kv : B->fft64) tb += kv.second.r2c.bytes() + kv.second.cols.bytes();
@@ -309,11 +305,10 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
     for (auto& kv : B->dep) {
         DepClass& D = kv.second;
         p = D.sup.place(p);
-        p = D.ssc.place(p);
         p = D.bin.place(p);
         p = D.ov.place(p);
         p = D.tile.place(p);
-        if ((rc = D.sup.upload()) || (rc = D.ssc.upload()) || (rc = D.bin.upload()) || (rc = D.ov.upload()) ||
+        if ((rc = D.sup.upload()) || (rc = D.bin.upload()) || (rc = D.ov.upload()) ||
             (rc = D.tile.upload()))
             return rc;
     }
@@ -363,9 +358,8 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
     for (auto& kv : B->dep) {
         DepClass* D = &kv.second;
         B->steps.push_back([D](hipStream_t st) {
-            BinnedTables t{D->bin.nj(), D->sup.dev, D->sup.dstart, D->ssc.dstart, D->sup.total(), D->ssc.total(),
-                           D->bin.dev, D->bin.dstart, D->bin.total(), D->ov.dev, D->tile.dev, D->tile.dstart,
-                           D->tile.total()};
+            BinnedTables t{D->bin.nj(), D->sup.dev, D->sup.dstart, D->sup.total(), D->bin.dev,
+                           D->bin.dstart, D->bin.total(), D->ov.dev, D->tile.dev, D->tile.dstart, D->tile.total()};
             return binned_batch_launch(D->scheme, D->hasw, D->prec == PYL_F64, D->acc, D->sorted, t, st);
         });
     }

@@ -160,6 +160,22 @@ __device__ __forceinline__ int halo_class(int bx, int by, int bz) {
     return ((bx % TILE) > TILE - S ? 1 : 0) | ((by % TILE) > TILE - S ? 2 : 0) | ((bz % TILE) > TILE - S ? 4 : 0);
 }
 
+// exclusive sums of one value a thread over the workgroup (wsum: a word of LDS per wave; synchronises once)
+__device__ __forceinline__ unsigned block_exscan(unsigned x, unsigned* wsum) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    unsigned v = x;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned u = __shfl_up(v, o, 64);
+        if (lane >= o) v += u;
+    }
+    if (lane == 63) wsum[wv] = v;
+    __syncthreads();
+    unsigned run = v - x;
+    for (int j = 0; j < wv; ++j) run += wsum[j];
+    return run;
+}
+
 // AGG: 0 every lane counts itself, 1 runs of equal keys are counted once, 2 a.agg decides (batched
 // launches, whose jobs differ; ragged grids).  RAG: the grid edge is no multiple of TILE.
 template <int S, bool HASW, int AGG, bool RAG>
@@ -515,7 +531,7 @@ int dense_acc(int acc, int scheme, int64_t n, int dims) {
 constexpr double AGG_PPC = 2.0;
 int bin_agg(int64_t n, int dims) { return (double)n >= AGG_PPC * (double)dims * dims * dims ? 1 : 0; }
 
-template <int S, typename G, bool HASW, int MODE, bool UNIT, int ACC>
+template <int S, typename G, bool HASW, int MODE, bool UNIT, int ACC, bool RAG>
 __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
     constexpr int R = HASW ? 4 : 3;
     constexpr int NE = 72;   // 8 neighbours (d = 0 own) x (8 class segments + 1 overflow group)
@@ -570,7 +586,7 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
     __syncthreads();
     const unsigned tot = sstart[NE];
     TileBox box{tx * TILE, ty * TILE, tz * TILE, TILE, TILE, TILE};
-    if (a.rag) {
+    if (RAG) {
         box.ox = (tx * a.N + nt - 1) / nt;
         box.oy = (ty * a.N + nt - 1) / nt;
         box.oz = (tz * a.N + nt - 1) / nt;
@@ -754,33 +770,40 @@ __device__ __forceinline__ void tile_body(const TileArgs& a, Blk B) {
     const long long N = a.N;
     for (int idx = tid; idx < TILE * TILE * TILE; idx += TT) {
         const int i = idx / (TILE * TILE), j = (idx / TILE) % TILE, k = idx % TILE;
-        if (a.rag && (i >= box.ex || j >= box.ey || k >= box.ez)) continue;
+        if (RAG && (i >= box.ex || j >= box.ey || k >= box.ez)) continue;
         const long long g = (((long long)box.ox + i) * N + box.oy + j) * N + box.oz + k;
         put<G, MODE>(grid, g, acc[(i * TILE + j) * TROW + k], am);
     }
 }
 
-template <int S, typename G, bool HASW, int MODE, bool UNIT, int ACC>
+// RAG: the grid edge is no multiple of TILE: tile t holds the cells [ceil(t N / nt), ceil((t + 1) N / nt))
+template <int S, typename G, bool HASW, int MODE, bool UNIT, int ACC, bool RAG>
 __global__ __launch_bounds__(TT) void k_tile(TileArgs a) {
-    tile_body<S, G, HASW, MODE, UNIT, ACC>(a, own_blk());
+    tile_body<S, G, HASW, MODE, UNIT, ACC, RAG>(a, own_blk());
 }
 template <int S, typename G, bool HASW, int MODE, bool UNIT, int ACC>
 __global__ __launch_bounds__(TT) void k_tile_b(const TileArgs* __restrict__ tab,
                                                   const unsigned* __restrict__ start, int nj) {
     PYL_BATCH_BLK(start, nj);
-    tile_body<S, G, HASW, MODE, UNIT, ACC>(tab[bj_], blk_);
+    tile_body<S, G, HASW, MODE, UNIT, ACC, false>(tab[bj_], blk_);
 }
 
 // ------------------------------------------------------------------ presort for unordered inputs
 // Particles in no spatial order give k_bin one key per particle: one global atomic each and 12-byte
-// scattered records.  The presort first groups them by supertile (tps consecutive tiles, at most
-// SUPMAX groups) with an exact count, a scan and a scatter whose per-step chunks are contiguous; k_bin
-// then reads the grouped copy, where neighbouring particles share keys as in an ordered input.
-constexpr int PT = 512;   // presort kernels: threads per workgroup
-constexpr int PKP = 8;    // k_sup_scatter: particles per thread per step
+// scattered records.  The presort first groups them by supertile (whole columns of tiles, at most SUPMAX
+// groups): k_sup_count counts the groups of every workgroup's particles, k_sup_scan turns the counts into
+// each workgroup's first slot per group, and k_sup_scatter copies the particles there.  No global atomics:
+// with one global reservation per group and step instead, 3 M weighted particles took 46 + 46 us, most of
+// it in atomics on a hundred addresses.
+// k_bin then reads the grouped copy, where neighbouring particles share keys as in an ordered input.
+constexpr int PT = 1024;   // presort kernels: threads per workgroup
+constexpr int PKP = 8;    // particles per thread per step
 // particles from which the device looks for a spatial order (PRESORT_PROBE)
 constexpr int64_t PROBE_MIN = 1 << 20;
-
+// groups aimed at: more give k_bin fewer keys a step (3 M particles onto 320^3: 60 us with 128, 40 with 256, 29
+// with 512), fewer give the scatter longer runs (24 / 24 / 25 us)
+constexpr int SUPGROUPS = 512;
+constexpr int SUPBLOCKS = 256;   // most workgroups of the count and the scatter
 
 __device__ __forceinline__ void sup_load(const SupArgs& a, long long p, float& x, float& y, float& z) {
     float c[3] = {a.pos[3 * p], a.pos[3 * p + 1], a.pos[3 * p + 2]};
@@ -796,11 +819,16 @@ __device__ __forceinline__ void sup_load(const SupArgs& a, long long p, float& x
 __device__ __forceinline__ int sup_cell(float x, float inv, int N) {
     return (int)fminf(fmaxf(x * inv, 0.0f), (float)(N - 1));
 }
-template <int S>
-__device__ __forceinline__ int sup_of(const SupArgs& a, float x, float y, float z) {
+__device__ __forceinline__ int sup_of(const SupArgs& a, float x, float y) {
     const float inv = (float)a.inv;
-    const int bx = sup_cell(x, inv, a.N), by = sup_cell(y, inv, a.N), bz = sup_cell(z, inv, a.N);
-    return (((bx / TILE) * a.nt + by / TILE) * a.nt + bz / TILE) / a.tps;
+    const unsigned v = (unsigned)((sup_cell(x, inv, a.N) / TILE) * a.nt + sup_cell(y, inv, a.N) / TILE);
+    return (int)(a.cmul ? __umulhi(v, a.cmul) : v);
+}
+// the steps of PT * PKP particles that workgroup B.x of a.nb owns
+__device__ __forceinline__ void sup_range(const SupArgs& a, unsigned bx, long long& s0, long long& s1) {
+    const long long nstep = (a.n + PT * PKP - 1) / (PT * PKP), per = (nstep + a.nb - 1) / a.nb;
+    s0 = min(nstep, (long long)bx * per);
+    s1 = min(nstep, s0 + per);
 }
 
 // a.sel: the particles are grouped only when they are in no spatial order.  Every workgroup looks at
@@ -822,114 +850,166 @@ __device__ __forceinline__ bool sup_probe(const SupArgs& a, Blk B) {
     return group;
 }
 
-template <int S>
 __device__ __forceinline__ void sup_count_body(const SupArgs& a, Blk B) {
     __shared__ unsigned h[SUPMAX];
-    if (!sup_probe(a, B)) return;
-    for (int i = threadIdx.x; i < a.nsup; i += PT) h[i] = 0u;
+    if (!sup_probe(a, B) || (int)B.x >= a.nb) return;
+    const int tid = threadIdx.x;
+    for (int i = tid; i < a.nsup; i += PT) h[i] = 0u;
     __syncthreads();
-    for (long long p = (long long)B.x * PT + threadIdx.x; p < a.n; p += (long long)B.gx * PT) {
-        float x, y, z;
-        sup_load(a, p, x, y, z);
-        atomicAdd(&h[sup_of<S>(a, x, y, z)], 1u);
+    long long s0, s1;
+    sup_range(a, B.x, s0, s1);
+    for (long long step = s0; step < s1; ++step) {
+        int sp[PKP];
+#pragma unroll
+        for (int k = 0; k < PKP; ++k) {
+            const long long p = (step * PKP + k) * PT + tid;
+            sp[k] = -1;
+            if (p < a.n) {
+                float x, y, z;
+                sup_load(a, p, x, y, z);
+                sp[k] = sup_of(a, x, y);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < PKP; ++k)
+            if (sp[k] >= 0) atomicAdd(&h[sp[k]], 1u);
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < a.nsup; i += PT)
-        if (h[i]) atomicAdd(&a.cnt[i], h[i]);
+    for (int i = tid; i < a.nsup; i += PT) a.cnt[(long long)B.x * a.nsup + i] = h[i];
 }
 
-template <int S>
-__global__ __launch_bounds__(PT) void k_sup_count(SupArgs a) { sup_count_body<S>(a, own_blk()); }
-template <int S>
+__global__ __launch_bounds__(PT) void k_sup_count(SupArgs a) { sup_count_body(a, own_blk()); }
 __global__ __launch_bounds__(PT) void k_sup_count_b(const SupArgs* __restrict__ tab,
+                                                     const unsigned* __restrict__ start, int nj) {
+    PYL_BATCH_BLK(start, nj);
+    sup_count_body(tab[bj_], blk_);
+}
+
+// columns [64 bx, 64 bx + 64) of cnt: exclusive sums down the rows in place, and the column totals; the rows
+// are split over the 16 waves
+__device__ __forceinline__ void sup_scan_body(const SupArgs& a, unsigned bx) {
+    __shared__ unsigned wsum[16][64];
+    if (a.sel && !*a.sel) return;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int c = (int)bx * 64 + lane;
+    const int per = (a.nb + 15) / 16, r0 = min(a.nb, wv * per), r1 = min(a.nb, r0 + per);
+    constexpr int PER = SUPBLOCKS / 16;   // all rows of a wave are loaded before the first is used
+    unsigned s = 0u, v[PER];
+#pragma unroll
+    for (int j = 0; j < PER; ++j) v[j] = c < a.nsup && r0 + j < r1 ? a.cnt[(long long)(r0 + j) * a.nsup + c] : 0u;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) s += v[j];
+    wsum[wv][lane] = s;
+    __syncthreads();
+    if (c >= a.nsup) return;
+    unsigned run = 0u;
+    for (int j = 0; j < wv; ++j) run += wsum[j][lane];
+    if (wv == 15) a.tot[c] = run + s;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        if (r0 + j < r1) a.cnt[(long long)(r0 + j) * a.nsup + c] = run;
+        run += v[j];
+    }
+}
+__global__ __launch_bounds__(1024) void k_sup_scan(SupArgs a) { sup_scan_body(a, blockIdx.x); }
+// batched: job blockIdx.y
+__global__ __launch_bounds__(1024) void k_sup_scan_b(const SupArgs* __restrict__ tab) {
+    const SupArgs& a = tab[blockIdx.y];
+    sup_scan_body(a, blockIdx.x);
+}
+
+// A step's particles are put in group order in LDS and leave in runs of consecutive addresses (one store of
+// 12 bytes a lane to as many lines kept the store path busy: 10 M weighted particles 161 -> 70 us).
+template <bool HASW>
+__device__ __forceinline__ void sup_scatter_body(const SupArgs& a, Blk B) {
+    constexpr int PS = PT * PKP, R = HASW ? 4 : 3;
+    __shared__ float rec[PS * R];
+    __shared__ unsigned short grp[PS];
+    __shared__ unsigned lc[SUPMAX];   // the step's particles per group
+    __shared__ unsigned lo[SUPMAX];   // first of them in rec
+    __shared__ unsigned gd[SUPMAX];   // where rec[i] of the group goes: gd + i
+    __shared__ unsigned wsum[PT / 64];
+    static_assert(SUPMAX == PT && PS <= 65536, "one group a thread");
+    const int tid = threadIdx.x;
+    if ((a.sel && !*a.sel) || (int)B.x >= a.nb) return;
+    // thread g's cursor: the first slot of group g (exclusive sum of the totals) plus what the workgroups before
+    // this one put there
+    unsigned cur = block_exscan(tid < a.nsup ? a.tot[tid] : 0u, wsum);
+    if (tid < a.nsup) cur += a.cnt[(long long)B.x * a.nsup + tid];
+    lc[tid] = 0u;
+    long long s0, s1;
+    sup_range(a, B.x, s0, s1);
+    float nx[PKP], ny[PKP], nz[PKP], nw[PKP];
+    auto load = [&](long long step) {
+#pragma unroll
+        for (int k = 0; k < PKP; ++k) {
+            const long long p = (step * PKP + k) * PT + tid;
+            if (p < a.n) {
+                sup_load(a, p, nx[k], ny[k], nz[k]);
+                nw[k] = HASW ? a.W[p] : 0.f;
+            }
+        }
+    };
+    if (s0 < s1) load(s0);
+    __syncthreads();
+    for (long long step = s0; step < s1; ++step) {
+        float x[PKP], y[PKP], z[PKP], w[PKP];
+        int g[PKP];
+        unsigned r[PKP];
+#pragma unroll
+        for (int k = 0; k < PKP; ++k) {
+            x[k] = nx[k];
+            y[k] = ny[k];
+            z[k] = nz[k];
+            w[k] = nw[k];
+        }
+        if (step + 1 < s1) load(step + 1);   // in flight during this step
+#pragma unroll
+        for (int k = 0; k < PKP; ++k) {
+            g[k] = -1;
+            if ((step * PKP + k) * PT + tid < a.n) {
+                g[k] = sup_of(a, x[k], y[k]);
+                r[k] = atomicAdd(&lc[g[k]], 1u);
+            }
+        }
+        __syncthreads();   // (also: every thread has stored the previous step's records)
+        const unsigned c = lc[tid];
+        lc[tid] = 0u;
+        const unsigned o = block_exscan(c, wsum);
+        lo[tid] = o;
+        gd[tid] = cur - o;
+        cur += c;
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < PKP; ++k) {
+            if (g[k] < 0) continue;
+            const unsigned i = lo[g[k]] + r[k];
+            rec[i * R] = x[k];
+            rec[i * R + 1] = y[k];
+            rec[i * R + 2] = z[k];
+            if (HASW) rec[i * R + 3] = w[k];
+            grp[i] = (unsigned short)g[k];
+        }
+        __syncthreads();
+        const int m = (int)min((long long)PS, a.n - step * PS);
+        for (int i = tid; i < m; i += PT) {
+            const long long d = gd[grp[i]] + (unsigned)i;
+            if (d >= a.n) continue;   // unreachable: the count pass gave every particle its slot
+            a.spos[3 * d] = rec[i * R];
+            a.spos[3 * d + 1] = rec[i * R + 1];
+            a.spos[3 * d + 2] = rec[i * R + 2];
+            if (HASW) a.sw[d] = rec[i * R + 3];
+        }
+    }
+}
+
+template <bool HASW>
+__global__ __launch_bounds__(PT) void k_sup_scatter(SupArgs a) { sup_scatter_body<HASW>(a, own_blk()); }
+template <bool HASW>
+__global__ __launch_bounds__(PT) void k_sup_scatter_b(const SupArgs* __restrict__ tab,
                                                        const unsigned* __restrict__ start, int nj) {
     PYL_BATCH_BLK(start, nj);
-    sup_count_body<S>(tab[bj_], blk_);
-}
-
-// exclusive scan of the nsup <= SUPMAX counts (one workgroup of SUPMAX threads)
-__device__ __forceinline__ void sup_scan_body(const unsigned* __restrict__ cnt, unsigned* __restrict__ off, int nsup) {
-    __shared__ unsigned wsum[SUPMAX / 64];   // (nothing was grouped: scans zeros)
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    const unsigned c = tid < nsup ? cnt[tid] : 0u;
-    unsigned v = c;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const unsigned u = __shfl_up(v, o, 64);
-        if (lane >= o) v += u;
-    }
-    if (lane == 63) wsum[wv] = v;
-    __syncthreads();
-    unsigned before = 0u;
-    for (int j = 0; j < wv; ++j) before += wsum[j];
-    if (tid < nsup) off[tid] = before + v - c;
-}
-__global__ __launch_bounds__(SUPMAX) void k_sup_scan(const unsigned* __restrict__ cnt, unsigned* __restrict__ off,
-                                                     int nsup) {
-    sup_scan_body(cnt, off, nsup);
-}
-// batched: one workgroup per job
-__global__ __launch_bounds__(SUPMAX) void k_sup_scan_b(const SupArgs* __restrict__ tab) {
-    const SupArgs& a = tab[blockIdx.x];
-    sup_scan_body(a.cnt, a.off, a.nsup);
-}
-
-template <int S, bool HASW>
-__device__ __forceinline__ void sup_scatter_body(const SupArgs& a, Blk B) {
-    constexpr long long PS = (long long)PT * PKP;
-    __shared__ unsigned lc[SUPMAX], lb[SUPMAX];
-    const int tid = threadIdx.x;
-    if (a.sel && !*a.sel) return;
-    for (int i = tid; i < a.nsup; i += PT) lc[i] = 0u;
-    __syncthreads();
-    const long long nstep = (a.n + PS - 1) / PS;
-    for (long long step = B.x; step < nstep; step += B.gx) {
-        float x[PKP], y[PKP], z[PKP], w[PKP];
-        int sp[PKP];
-        unsigned rank[PKP];
-#pragma unroll
-        for (int k = 0; k < PKP; ++k) {
-            const long long p = step * PS + k * PT + tid;
-            sp[k] = -1;
-            rank[k] = 0u;
-            if (p < a.n) {
-                sup_load(a, p, x[k], y[k], z[k]);
-                w[k] = HASW ? a.W[p] : 0.f;
-                sp[k] = sup_of<S>(a, x[k], y[k], z[k]);
-                rank[k] = atomicAdd(&lc[sp[k]], 1u);
-            }
-        }
-        __syncthreads();
-        // one reservation per supertile present in the step; the counters are cleared for the next
-        // step, whose insertions every thread makes only after its stores below
-        for (int i = tid; i < a.nsup; i += PT) {
-            const unsigned c = lc[i];
-            if (c) {
-                lb[i] = a.off[i] + atomicAdd(&a.cur[i], c);
-                lc[i] = 0u;
-            }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < PKP; ++k) {
-            if (sp[k] < 0) continue;
-            const long long d = (long long)lb[sp[k]] + rank[k];
-            if (d >= a.n) continue;   // unreachable: the count pass gave every particle its slot
-            a.spos[3 * d] = x[k];
-            a.spos[3 * d + 1] = y[k];
-            a.spos[3 * d + 2] = z[k];
-            if (HASW) a.sw[d] = w[k];
-        }
-    }
-}
-
-template <int S, bool HASW>
-__global__ __launch_bounds__(PT) void k_sup_scatter(SupArgs a) { sup_scatter_body<S, HASW>(a, own_blk()); }
-template <int S, bool HASW>
-__global__ __launch_bounds__(PT) void k_sup_scatter_b(const SupArgs* __restrict__ tab,
-                                                         const unsigned* __restrict__ start, int nj) {
-    PYL_BATCH_BLK(start, nj);
-    sup_scatter_body<S, HASW>(tab[bj_], blk_);
+    sup_scatter_body<HASW>(tab[bj_], blk_);
 }
 
 // ------------------------------------------------------------------ host side
@@ -1037,24 +1117,30 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
     {
         StageTimer tm("deposit_tiles", st);
         TileArgs ta{bucket, fill, CT, {}, {}, grouped, gcls, ooff, ocnt, dims, nt, dims / BoxSize, mult, grid, dmass,
-                    mass, rag ? 1 : 0};
+                    mass};
         for (int c = 0; c < 8; ++c) {
             ta.cofs[c] = cofs[c];
             ta.cap[c] = cap[c];
         }
         const dim3 tg((unsigned)((ntiles + XCDS - 1) / XCDS * XCDS));
         const bool unit = !HASW && mult == 1.0;
-#define PYL_TILE_LAUNCH(U, A) hipLaunchKernelGGL((k_tile<S, G, HASW, MODE, U, A>), tg, dim3(TT), 0, st, ta)
-        if constexpr (S == 2) {
-            if (acc == ACC_RUN) {
-                if (unit) PYL_TILE_LAUNCH(true, ACC_RUN); else PYL_TILE_LAUNCH(false, ACC_RUN);
+#define PYL_TILE_LAUNCH(U, A, G_) hipLaunchKernelGGL((k_tile<S, G, HASW, MODE, U, A, G_>), tg, dim3(TT), 0, st, ta)
+        if (rag) {
+            // (never the overdensity; ACC_F32W allows float32 weights, and gets float64 ones)
+            if constexpr (MODE != OUT_DELTA) {
+                if constexpr (S == 2) {
+                    if (acc == ACC_RUN) PYL_TILE_LAUNCH(!HASW, ACC_RUN, true);
+                }
+                if (acc != ACC_RUN) PYL_TILE_LAUNCH(!HASW, ACC_F64, true);
             }
-        }
-        if (acc == ACC_RUN) {
+        } else if (acc == ACC_RUN) {
+            if constexpr (S == 2) {
+                if (unit) PYL_TILE_LAUNCH(true, ACC_RUN, false); else PYL_TILE_LAUNCH(false, ACC_RUN, false);
+            }
         } else if (acc == ACC_F32W) {
-            if (unit) PYL_TILE_LAUNCH(true, ACC_F32W); else PYL_TILE_LAUNCH(false, ACC_F32W);
+            if (unit) PYL_TILE_LAUNCH(true, ACC_F32W, false); else PYL_TILE_LAUNCH(false, ACC_F32W, false);
         } else {
-            if (unit) PYL_TILE_LAUNCH(true, ACC_F64); else PYL_TILE_LAUNCH(false, ACC_F64);
+            if (unit) PYL_TILE_LAUNCH(true, ACC_F64, false); else PYL_TILE_LAUNCH(false, ACC_F64, false);
         }
 #undef PYL_TILE_LAUNCH
         PYL_HIP(hipGetLastError());
@@ -1082,48 +1168,54 @@ static int dispatch_s(const float* pos, const float* W, int64_t n, int dims, dou
     }
 }
 
-template <int S>
-static void launch_presort(const SupArgs& a, bool hasw, unsigned blocks, unsigned sblocks, hipStream_t st) {
-    hipLaunchKernelGGL(k_sup_count<S>, dim3(blocks), dim3(PT), 0, st, a);
-    hipLaunchKernelGGL(k_sup_scan, dim3(1), dim3(SUPMAX), 0, st, a.cnt, a.off, a.nsup);
-    if (hasw)
-        hipLaunchKernelGGL((k_sup_scatter<S, true>), dim3(sblocks), dim3(PT), 0, st, a);
-    else
-        hipLaunchKernelGGL((k_sup_scatter<S, false>), dim3(sblocks), dim3(PT), 0, st, a);
+// supertiles: m whole tile columns (nt tiles along z) each, about SUPGROUPS of them and never more than
+// SUPMAX; sup_fill sets the geometry of a presort (everything but the buffers), sup_words the unsigned words
+// of its counters (counts, totals, the order word)
+static void sup_fill(SupArgs* a, int64_t n, int dims) {
+    a->nt = (dims + TILE - 1) / TILE;
+    const long long cols = (long long)a->nt * a->nt;
+    long long m = std::max(1LL, (cols + SUPGROUPS - 1) / SUPGROUPS);
+    while ((cols + m - 1) / m > SUPMAX) ++m;
+    // v * ceil(2^32 / m) >> 32 = v / m for v < cols: the rounding adds less than cols / 2^32 < 1 / m
+    a->cmul = m == 1 ? 0u : (unsigned)(((1ULL << 32) + m - 1) / m);
+    a->nsup = (int)((cols + m - 1) / m);
+    a->N = dims;
+    a->n = n;
+    a->nb = (int)std::max<int64_t>(1, std::min<int64_t>(SUPBLOCKS, (n + PT * PKP - 1) / (PT * PKP)));
+}
+static size_t sup_words(const SupArgs& a) { return (size_t)(a.nb + 1) * a.nsup + 4; }
+static void sup_carve(SupArgs* a, unsigned* w) {
+    a->cnt = w;
+    a->tot = w + (size_t)a->nb * a->nsup;
 }
 
 // groups the particles by supertile into library workspaces (ps->pos, ps->W); the redshift-space shift
 // is applied on the way, so the grouped copy is deposited without it.  probe: only when they are in no
 // spatial order, which the device decides (ps->sel)
-static int presort(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, const Rsd& rsd,
-                   bool probe, hipStream_t st, Presort* ps) {
+static int presort(const float* pos, const float* W, int64_t n, int dims, double BoxSize, const Rsd& rsd, bool probe,
+                   hipStream_t st, Presort* ps) {
     int rc = OK;
-    const int nt = (dims + TILE - 1) / TILE;
-    const long long ntiles = (long long)nt * nt * nt;
-    // supertiles of whole tile columns (nt tiles along z), about 128 of them and never more than SUPMAX
-    long long tps = nt * std::max(1LL, (ntiles + 128LL * nt - 1) / (128LL * nt));
-    while ((ntiles + tps - 1) / tps > SUPMAX) tps += nt;
-    const int nsup = (int)((ntiles + tps - 1) / tps);
-    unsigned* cnt = (unsigned*)workspace(WS_SUP, sizeof(unsigned) * (3 * SUPMAX + 4), &rc);
+    SupArgs a{};
+    sup_fill(&a, n, dims);
+    unsigned* words = (unsigned*)workspace(WS_SUP, sizeof(unsigned) * sup_words(a), &rc);
     if (rc) return rc;
     float* sp = (float*)workspace(WS_STAGE, sizeof(float) * (size_t)n * (W ? 4 : 3) + 64, &rc);
     if (rc) return rc;
-    rc = zero_fill(cnt, sizeof(unsigned) * 3 * SUPMAX, st);
-    if (rc) return rc;
-    SupArgs a{pos, W, (long long)n, dims, nt, (int)tps, nsup, dims / BoxSize, rsd, cnt, cnt + SUPMAX,
-              cnt + 2 * SUPMAX, sp, W ? sp + 3 * n : nullptr, probe ? cnt + 3 * SUPMAX : nullptr};
-    long long blocks = (n + PT - 1) / PT;
-    if (blocks > 2048) blocks = 2048;
-    long long sblocks = (n + (long long)PT * PKP - 1) / ((long long)PT * PKP);
-    if (sblocks > 2048) sblocks = 2048;
+    sup_carve(&a, words);
+    a.pos = pos;
+    a.W = W;
+    a.inv = dims / BoxSize;
+    a.rsd = rsd;
+    a.spos = sp;
+    a.sw = W ? sp + 3 * n : nullptr;
+    a.sel = probe ? a.tot + a.nsup : nullptr;
     StageTimer tm("deposit_presort", st);
-    switch (scheme) {
-        case 1: launch_presort<1>(a, W != nullptr, (unsigned)blocks, (unsigned)sblocks, st); break;
-        case 2: launch_presort<2>(a, W != nullptr, (unsigned)blocks, (unsigned)sblocks, st); break;
-        case 3: launch_presort<3>(a, W != nullptr, (unsigned)blocks, (unsigned)sblocks, st); break;
-        case 4: launch_presort<4>(a, W != nullptr, (unsigned)blocks, (unsigned)sblocks, st); break;
-        default: set_error("unknown scheme %d", scheme); return E_ARG;
-    }
+    hipLaunchKernelGGL(k_sup_count, dim3((unsigned)a.nb), dim3(PT), 0, st, a);
+    hipLaunchKernelGGL(k_sup_scan, dim3((unsigned)((a.nsup + 63) / 64)), dim3(1024), 0, st, a);
+    if (W)
+        hipLaunchKernelGGL((k_sup_scatter<true>), dim3((unsigned)a.nb), dim3(PT), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_sup_scatter<false>), dim3((unsigned)a.nb), dim3(PT), 0, st, a);
     PYL_HIP(hipGetLastError());
     ps->sel = a.sel;
     ps->pos = sp;
@@ -1139,13 +1231,15 @@ int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double
     PYL_CHECK(!rsd_in.vel || (rsd_in.axis >= 0 && rsd_in.axis <= 2), E_ARG, "redshift-space axis must be 0, 1 or 2");
     PYL_CHECK(binned_supported(3, dims) || binned_ragged(3, dims), E_UNSUPPORTED,
               "binned deposit needs 3-D grids of at least %d cells an edge", 2 * TILE);
+    PYL_CHECK(binned_supported(3, dims) || (mode != OUT_DELTA && mult == 1.0), E_UNSUPPORTED,
+              "binned deposit: overdensities need dims %% %d == 0", TILE);
     PYL_CHECK(n > 0, E_ARG, "binned deposit needs particles");
     PYL_CHECK(n < (1LL << 31), E_UNSUPPORTED, "binned deposit: at most 2^31 particles per call");
     Rsd rsd = rsd_in;
     Presort ps;
     if (sorted == PRESORT_PROBE && (rsd.vel || n < PROBE_MIN)) sorted = PRESORT_NO;
     if (sorted) {
-        const int rc = presort(pos, W, n, dims, BoxSize, scheme, rsd_in, sorted == PRESORT_PROBE, st, &ps);
+        const int rc = presort(pos, W, n, dims, BoxSize, rsd_in, sorted == PRESORT_PROBE, st, &ps);
         if (rc && !(sorted == PRESORT_PROBE && rc == E_ALLOC)) return rc;
         if (rc) ps = Presort();   // no room for the grouped copy: deposit the particles as they are
         if (!rc && sorted == PRESORT_YES) {
@@ -1173,20 +1267,15 @@ int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double
 // job j sit in device tables and its blocks are the range [start[j], start[j+1]) of the launch.
 static size_t al256(size_t b) { return (b + 255) / 256 * 256; }
 
-static void sup_geometry(int dims, int* tps, int* nsup) {
-    const int nt = dims / TILE;
-    const long long ntiles = (long long)nt * nt * nt;
-    long long t = nt * std::max(1LL, (ntiles + 128LL * nt - 1) / (128LL * nt));
-    while ((ntiles + t - 1) / t > SUPMAX) t += nt;
-    *tps = (int)t;
-    *nsup = (int)((ntiles + t - 1) / t);
-}
-
 size_t binned_job_bytes(int64_t n, int dims, int scheme, bool hasw, bool sorted) {
     Layout L;
     if (!binned_supported(3, dims) || layout_of(n, dims, scheme, hasw, &L) != OK) return 0;
     size_t b = al256(L.cnt_bytes) + al256(L.bucket_bytes) + al256(L.ov_bytes);
-    if (sorted) b += al256(sizeof(unsigned) * 3 * SUPMAX) + al256(sizeof(float) * (size_t)n * (hasw ? 4 : 3) + 64);
+    if (sorted) {
+        SupArgs a{};
+        sup_fill(&a, n, dims);
+        b += al256(sizeof(unsigned) * sup_words(a)) + al256(sizeof(float) * (size_t)n * (hasw ? 4 : 3) + 64);
+    }
     return b;
 }
 
@@ -1217,23 +1306,22 @@ int binned_job_plan(const float* pos, const float* W, int64_t n, int dims, doubl
     const float* bpos = pos;
     const float* bW = W;
     j->sup = SupArgs{};
-    j->sup_blocks = j->sup_sblocks = 0;
-    j->scnt = nullptr;
-    j->scnt_bytes = 0;
+    j->sup_blocks = 0;
     if (sorted) {
-        unsigned* sc = (unsigned*)p;
-        p += al256(sizeof(unsigned) * 3 * SUPMAX);
+        SupArgs& a = j->sup;
+        sup_fill(&a, n, dims);
+        sup_carve(&a, (unsigned*)p);
+        p += al256(sizeof(unsigned) * sup_words(a));
         float* sp = (float*)p;
-        int tps = 0, nsup = 0;
-        sup_geometry(dims, &tps, &nsup);
-        j->sup = SupArgs{pos, W, (long long)n, dims, L.nt, tps, nsup, inv, Rsd(), sc, sc + SUPMAX, sc + 2 * SUPMAX,
-                         sp, hasw ? sp + 3 * n : nullptr};
-        j->sup_blocks = (unsigned)std::min<long long>(2048, (n + PT - 1) / PT);
-        j->sup_sblocks = (unsigned)std::min<long long>(2048, (n + (long long)PT * PKP - 1) / ((long long)PT * PKP));
-        j->scnt = sc;
-        j->scnt_bytes = sizeof(unsigned) * 3 * SUPMAX;
+        a.pos = pos;
+        a.W = W;
+        a.inv = inv;
+        a.spos = sp;
+        a.sw = hasw ? sp + 3 * n : nullptr;
+        // a batched launch gives every job a multiple of XCDS blocks; those past a.nb have no particles
+        j->sup_blocks = (unsigned)((a.nb + XCDS - 1) / XCDS * XCDS);
         bpos = sp;
-        bW = j->sup.sw;
+        bW = a.sw;
     }
     (void)R;
     j->bin = BinArgs{bpos, bW, (long long)n, dims, L.nt, inv, fill, bucket, L.CT, {}, {}, ov_count, ov_idx, ov_key,
@@ -1259,9 +1347,9 @@ static int batch_launch_s(bool sorted, const BinnedTables& t, hipStream_t st) {
     const unsigned nj = (unsigned)t.nj;
     if (sorted) {
         StageTimer tm("deposit_presort", st);
-        hipLaunchKernelGGL((k_sup_count_b<S>), dim3(t.sup_total), dim3(PT), 0, st, t.sup, t.sup_start, t.nj);
-        hipLaunchKernelGGL(k_sup_scan_b, dim3(nj), dim3(SUPMAX), 0, st, t.sup);
-        hipLaunchKernelGGL((k_sup_scatter_b<S, HASW>), dim3(t.ssc_total), dim3(PT), 0, st, t.sup, t.ssc_start, t.nj);
+        hipLaunchKernelGGL(k_sup_count_b, dim3(t.sup_total), dim3(PT), 0, st, t.sup, t.sup_start, t.nj);
+        hipLaunchKernelGGL(k_sup_scan_b, dim3(SUPMAX / 64, nj), dim3(1024), 0, st, t.sup);
+        hipLaunchKernelGGL((k_sup_scatter_b<HASW>), dim3(t.sup_total), dim3(PT), 0, st, t.sup, t.sup_start, t.nj);
         PYL_HIP(hipGetLastError());
     }
     {

@@ -46,7 +46,6 @@ struct TileArgs {
     void* grid;
     const double* dmass;  // device mass (nullable) for OUT_DELTA
     double mass;
-    int rag = 0;          // ragged grid (N % TILE != 0): tile t holds the cells [ceil(t N / nt), ceil((t + 1) N / nt))
 };
 
 struct OvArgs {
@@ -71,12 +70,14 @@ struct SupArgs {
     const float* pos;
     const float* W;
     long long n;
-    int N, nt, tps, nsup;
+    int N, nt;
+    unsigned cmul;   // supertile of tile column v = tx * nt + ty: v * cmul >> 32 (cmul = 0: v itself)
+    int nsup;
+    int nb;          // workgroups of the count and of the scatter; each owns a contiguous range of the particles
     double inv;
     Rsd rsd;
-    unsigned* cnt;   // [nsup] particles per supertile
-    unsigned* off;   // [nsup] first slot of each supertile
-    unsigned* cur;   // [nsup] slots handed out so far
+    unsigned* cnt;   // [nb][nsup] particles of each workgroup per supertile, then their exclusive sums down a column
+    unsigned* tot;   // [nsup] particles per supertile
     float* spos;     // [n * 3] grouped positions (redshift-space shift applied)
     float* sw;       // [n] grouped weights (HASW)
     unsigned* sel = nullptr;   // [1] nullable: written by the count, 1 = the particles were grouped
@@ -84,18 +85,16 @@ struct SupArgs {
 
 // One job of a batched binned deposit (overdensity output): the arguments of every stage and
 // the block count of each 1-D launch.  binned_job_bytes gives the device memory one job needs;
-// binned_job_plan carves it from `mem` and fills the arguments.  cnt / scnt: counters to zero
-// before the deposit.
+// binned_job_plan carves it from `mem` and fills the arguments.  cnt: counters to zero before the
+// deposit.
 struct BinnedJob {
     BinArgs bin;
     TileArgs tile;
     OvArgs ov;
     SupArgs sup;
-    unsigned bin_blocks, tile_blocks, sup_blocks, sup_sblocks;
+    unsigned bin_blocks, tile_blocks, sup_blocks;
     void* cnt;
     size_t cnt_bytes;
-    void* scnt;
-    size_t scnt_bytes;
 };
 size_t binned_job_bytes(int64_t n, int dims, int scheme, bool hasw, bool sorted);
 int binned_job_plan(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, void* grid,
@@ -105,8 +104,8 @@ int binned_job_plan(const float* pos, const float* W, int64_t n, int dims, doubl
 struct BinnedTables {
     int nj;
     const SupArgs* sup;
-    const unsigned *sup_start, *ssc_start;
-    unsigned sup_total, ssc_total;
+    const unsigned* sup_start;
+    unsigned sup_total;
     const BinArgs* bin;
     const unsigned* bin_start;
     unsigned bin_total;

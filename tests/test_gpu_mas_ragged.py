@@ -30,7 +30,7 @@ def _particles(n, dims, L, order, seed):
 @pytest.mark.parametrize("dims", [33, 47, 49, 63, 65, 100])
 def test_ragged_grid(gpu, dims, scheme, weighted, order):
     from pylians_amd import MAS_library
-    L, n = 310.0, 900001
+    L, n = 310.0, 2400001 if scheme == "NGP" else 900001
     pos = _particles(n, dims, L, order, dims)
     W = np.random.default_rng(3).random(n, dtype=np.float32) + np.float32(0.25) if weighted else None
     start = np.random.default_rng(4).random((dims,) * 3).astype(np.float32)
