@@ -206,8 +206,9 @@ int deposit(const float* pos, const float* W, int64_t n, int axes, int dims, dou
         const bool whole = binned_supported(axes, dims);
         const bool ragged = !(flags & (DEP_BINNED | DEP_SORTED)) && binned_ragged(axes, dims) && n < (1LL << 31) &&
                             ragged_worth(n, dims, scheme);
+        const bool map = !(flags & (DEP_BINNED | DEP_SORTED)) && axes == 2 && map_supported(n, dims, scheme);
         bool capturing = false;
-        if (ragged || (whole && !(flags & (DEP_BINNED | DEP_SORTED)))) {
+        if (ragged || map || (whole && !(flags & (DEP_BINNED | DEP_SORTED)))) {
             hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
             PYL_HIP(hipStreamIsCapturing(st, &cs));
             capturing = cs != hipStreamCaptureStatusNone;
@@ -220,6 +221,14 @@ int deposit(const float* pos, const float* W, int64_t n, int axes, int dims, dou
                                                                    : PRESORT_PROBE;
             return deposit_binned(pos, W, n, dims, BoxSize, scheme, f64, mode, 1.0, grid, nullptr, 0.0, st, rsd, sorted,
                                   acc_mode(flags));
+        }
+        if (map && !capturing) {
+            const bool dup = flags & DEP_DUP2D;
+            StreamScope scope(st);
+            const int rc = deposit_map(pos, W, n, dims, BoxSize, scheme, f64, (flags & DEP_ZERO) != 0,
+                                       dup ? (double)scheme : 1.0,
+                                       dup && (flags & DEP_RENORM2D) && scheme > 1 ? (double)scheme : 0.0, grid, st);
+            if (rc != E_ALLOC) return rc;   // no room for the records: the direct kernel
         }
         if (ragged && !capturing) {
             StreamScope scope(st);

@@ -66,4 +66,11 @@ int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double
                    int mode, double mult, void* grid, const double* dmass, double mass, hipStream_t st,
                    const Rsd& rsd = Rsd(), int sorted = PRESORT_NO, int acc = 0);
 
+
+// 2-D deposit without global atomics (binned2d.hip), in the stream's own workspaces: grid (+)= mult * rho, then
+// grid /= div when div != 0, each rounded to the grid type.  map_supported: whether a call should take it.
+bool map_supported(int64_t n, int dims, int scheme);
+int deposit_map(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, bool f64, bool zero,
+                double mult, double div, void* grid, hipStream_t st);
+
 }  // namespace pyl
