@@ -1,6 +1,7 @@
 // 3-D real FFT passes for gfx950: rows r2c/c2r (pass Z) and column passes (Y, X).
 #include <math.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -106,6 +107,9 @@ __global__ __launch_bounds__(T) void k_r2c_rows_b(const R2cArgs<R>* __restrict__
 // x[2j] = Re z[j], x[2j+1] = Im z[j].  The inverse is computed as conj(FFT(conj(Z'))).
 // store: 0 = no output, 1 = x, 2 = x * aux.  Optional fused float64 reductions: each workgroup
 // writes its sum x^2 and sum x*aux to part[2 * block + 0 / 1] (k_c2r_partsum adds them up).
+// Persistent blocks walk row blocks; the spectrum rows of the next one load into registers while the present one
+// is transformed.  A thread takes the pair X[k], X[M-k] (each read once) for Z'[k] and Z'[M-k].  With blocks of one row block each and no loads in flight across the transform a 512^3 float32 field
+// took 409 us.
 template <typename R, int M, int NL, int T>
 __global__ __launch_bounds__(T) void k_c2r_rows(const cplx<R>* __restrict__ in, R* __restrict__ out,
                                                  long long nrows, long long P,
@@ -113,58 +117,96 @@ __global__ __launch_bounds__(T) void k_c2r_rows(const cplx<R>* __restrict__ in, 
                                                  const R* __restrict__ aux, double* __restrict__ part, int K) {
     constexpr int N = 2 * M;
     constexpr int ES = NL + 1;
+    constexpr int H = M / 2;                   // pairs per row
+    constexpr int NP = NL * H;
+    constexpr int V = (NP + T - 1) / T;        // pairs per thread per row block
     // whole wavefronts only: the float64 sums below reduce across all 64 lanes of every wave
     static_assert(T % 64 == 0, "k_c2r_rows needs a multiple of 64 threads");
+    static_assert(M % 2 == 0, "pairs of an even row");
     __shared__ cplx<R> s[M * ES];
     __shared__ cplx<R> tw[N];
     __shared__ double red[2][T / 64];
     const int tid = threadIdx.x;
-    const long long row0 = (long long)blockIdx.x * NL;
     for (int i = tid; i < N; i += T) tw[i] = twg[i];
-    __syncthreads();
-    for (int idx = tid; idx < NL * M; idx += T) {
-        const int r = idx / M, k = idx % M;
-        const long long row = row0 + r;
-        cplx<R> v = mk<R>(0, 0);
-        if (row < nrows) {
-            // entries kz >= K are known zeros (K = M + 1: the whole row) and are not read
-            cplx<R> A = k < K ? in[row * P + k] : mk<R>(0, 0);
-            cplx<R> B = M - k < K ? conjg(in[row * P + (M - k)]) : mk<R>(0, 0);
-            // the imaginary parts of the DC and Nyquist terms of a row do not exist in a real
-            // transform: drop them, as numpy's irfftn and FFTW's c2r do for non-Hermitian input
-            if (k == 0) {
-                A.y = (R)0;
-                B.y = (R)0;
-            }
-            const cplx<R> e = A + B;
-            const cplx<R> o = cmul(A - B, conjg(tw[k]));
-            v = conjg(e + mul_pi(o));
+    const long long nrb = (nrows + NL - 1) / NL;
+    cplx<R> na[V], nb[V], nm;
+    // Loads without branches, so that all of a block's are in flight at once: entries kz >= K are known zeros
+    // (K = M + 1: the whole row) and read entry K - 1, rows past the end the last one.
+    auto load = [&](long long rb) {
+        const long long left = nrows - 1 - rb * NL;
+        const cplx<R>* p = in + rb * NL * P;
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            const int idx = NP % T == 0 ? tid + q * T : min(tid + q * T, NP - 1);
+            const int r = idx / H, k = idx % H;
+            const cplx<R>* pr = p + min((long long)r, left) * P;
+            na[q] = pr[min(k, K - 1)];
+            nb[q] = pr[min(M - k, K - 1)];
         }
-        s[k * ES + r] = v;
-    }
-    __syncthreads();
-    lds_fft<R, M, NL, ES, T, 2>(s, tw, tid);
+        nm = p[min((long long)(tid % NL), left) * P + min(H, K - 1)];
+    };
+    // Z'[k] of the row from X[k] and X[M-k], conjugated for the forward transform
+    auto pack = [&](cplx<R> A, cplx<R> X, int k) {
+        const cplx<R> B = conjg(X);
+        const cplx<R> e = A + B;
+        const cplx<R> o = cmul(A - B, conjg(tw[k]));
+        return conjg(e + mul_pi(o));
+    };
     double a0 = 0.0, a1 = 0.0;
-    for (int idx = tid; idx < NL * M; idx += T) {
-        const int r = idx / M, j = idx % M;
-        const long long row = row0 + r;
-        if (row >= nrows) continue;
-        const cplx<R> z = s[j * ES + r];
-        const R x0 = z.x * sc, x1 = -z.y * sc;
-        R q0 = (R)0, q1 = (R)0;
-        if (aux) {
-            const R* q = aux + row * N + 2 * j;
-            q0 = q[0];
-            q1 = q[1];
+    long long rb = blockIdx.x;
+    if (rb < nrb) load(rb);
+    for (; rb < nrb; rb += gridDim.x) {
+        cplx<R> xa[V], xb[V];
+        const cplx<R> xm = H < K ? nm : mk<R>(0, 0);
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            const int k = (tid + q * T) % H;
+            xa[q] = k < K ? na[q] : mk<R>(0, 0);
+            xb[q] = M - k < K ? nb[q] : mk<R>(0, 0);
         }
-        if (store) {
-            R* p = out + row * N + 2 * j;
-            p[0] = store == 2 ? x0 * q0 : x0;
-            p[1] = store == 2 ? x1 * q1 : x1;
+        if (rb + gridDim.x < nrb) load(rb + gridDim.x);
+        __syncthreads();   // the previous row block's outputs have been read from s (and tw is filled)
+#pragma unroll
+        for (int q = 0; q < V; ++q) {
+            const int idx = tid + q * T;
+            if (NP % T == 0 || idx < NP) {
+                const int r = idx / H, k = idx % H;
+                if (k == 0) {   // no partner: Z'[M] does not exist
+                    // the imaginary parts of the DC and Nyquist terms of a row do not exist in a real
+                    // transform: drop them, as numpy's irfftn and FFTW's c2r do for non-Hermitian input
+                    xa[q].y = (R)0;
+                    xb[q].y = (R)0;
+                } else {
+                    s[(M - k) * ES + r] = pack(xb[q], xa[q], M - k);
+                }
+                s[k * ES + r] = pack(xa[q], xb[q], k);
+            }
         }
-        if (part) {
-            a0 += (double)x0 * x0 + (double)x1 * x1;
-            a1 += (double)x0 * q0 + (double)x1 * q1;
+        if (tid < NL) s[H * ES + tid] = pack(xm, xm, H);
+        __syncthreads();
+        lds_fft<R, M, NL, ES, T, 2>(s, tw, tid);
+        const long long row0 = rb * NL;
+        for (int idx = tid; idx < NL * M; idx += T) {
+            const int r = idx / M, j = idx % M;
+            const long long row = row0 + r;
+            if (row >= nrows) continue;
+            const cplx<R> z = s[j * ES + r];
+            const R x0 = z.x * sc, x1 = -z.y * sc;
+            R q0 = (R)0, q1 = (R)0;
+            if (aux) {
+                const R* q = aux + row * N + 2 * j;
+                q0 = q[0];
+                q1 = q[1];
+            }
+            if (store) {
+                R* p = out + row * N + 2 * j;
+                p[0] = store == 2 ? x0 * q0 : x0;
+                p[1] = store == 2 ? x1 * q1 : x1;
+            }
+            if (part) {
+                a0 += (double)x0 * x0 + (double)x1 * x1;
+                a1 += (double)x0 * q0 + (double)x1 * q1;
+            }
         }
     }
     if (part) {
@@ -250,40 +292,25 @@ __device__ __forceinline__ void cols_body(const ColArgs<R>& A, Blk B) {
         valid = c < ncols && (int)(c % PW) < W;   // kz = c % PW; columns kz >= W are row padding
         return valid ? (c / CW) * CS + (c % CW) : 0;
     };
+    // loads without conditions or arithmetic on their results, so that they stay in flight until the values are
+    // needed (a conjugation here made every prefetch wait: inverse 384^3 float64 390 us against 236 forward); columns
+    // of padding read column 0 and are not stored
+    auto load = [&](long long cb, cplx<R> (&x)[F::B][F::RAD]) {
+        bool v;
+        const cplx<R>* p = src + col_base(cb, v);
+        first_load<R, N, NL, T>(x, [&](int j, int) { return p[j * EST]; }, tid);
+    };
     cplx<R> nxt[F::B][F::RAD];
     long long cb = B.x;
-    if (PREFETCH && cb < nblk) {
-        bool v;
-        const long long b = col_base(cb, v);
-        first_load<R, N, NL, T>(nxt, [&](int j, int) {
-            const cplx<R> x = v ? src[b + j * EST] : mk<R>(0, 0);
-            return INV ? conjg(x) : x;
-        }, tid);
-    }
+    if (PREFETCH && cb < nblk) load(cb, nxt);
     for (; cb < nblk; cb += B.gx) {
         cplx<R> cur[F::B][F::RAD];
-        if (PREFETCH) {
+        if (!PREFETCH) load(cb, nxt);
 #pragma unroll
-            for (int b = 0; b < F::B; ++b)
+        for (int b = 0; b < F::B; ++b)
 #pragma unroll
-                for (int m = 0; m < F::RAD; ++m) cur[b][m] = nxt[b][m];
-        } else {
-            bool v;
-            const long long b = col_base(cb, v);
-            first_load<R, N, NL, T>(cur, [&](int j, int) {
-                const cplx<R> x = v ? src[b + j * EST] : mk<R>(0, 0);
-                return INV ? conjg(x) : x;
-            }, tid);
-        }
-        const long long cbn = cb + B.gx;
-        if (PREFETCH && cbn < nblk) {
-            bool v;
-            const long long b = col_base(cbn, v);
-            first_load<R, N, NL, T>(nxt, [&](int j, int) {
-                const cplx<R> x = v ? src[b + j * EST] : mk<R>(0, 0);
-                return INV ? conjg(x) : x;
-            }, tid);
-        }
+            for (int m = 0; m < F::RAD; ++m) cur[b][m] = INV ? conjg(nxt[b][m]) : nxt[b][m];
+        if (PREFETCH && cb + B.gx < nblk) load(cb + B.gx, nxt);
         bool valid;
         const long long base = col_base(cb, valid);
         auto store = [&](int k, int, cplx<R> x) {
@@ -320,10 +347,6 @@ __global__ __launch_bounds__(T) void k_cols_b(const ColArgs<R>* __restrict__ tab
 }
 
 // ----------------------------------------------------------------------- dispatch
-#define PYL_FFT_SIZES(X) \
-    X(8) X(12) X(16) X(20) X(24) X(32) X(40) X(48) X(64) X(80) X(96) X(128) X(160) X(192) X(256) \
-    X(320) X(384) X(512) X(640) X(768) X(1024)
-
 bool fft_size_supported(int N) {
     switch (N) {
 #define PYL_CASE(n) case n:
@@ -346,6 +369,16 @@ int cu_count() {
             n = 256;
     }
     return n;
+}
+
+// Persistent grid for `units` equal pieces of work with at most `most` resident workgroups a CU.  A round takes about
+// as long with fewer workgroups a CU (rows of 320 points: 16.0 us a round with 6, 15.1 with 5), so: as few rounds
+// as `most` allows, and no more workgroups than those need.
+long long persistent_blocks(long long units, int most) {
+    const long long cu = cu_count();
+    if (units <= cu * most) return units;
+    const long long rounds = (units + cu * most - 1) / (cu * most);
+    return cu * ((units + cu * rounds - 1) / (cu * rounds));
 }
 
 // host table exp(-2 pi i t / N), t < N, rounded once from long double; cached per N
@@ -394,8 +427,9 @@ template const cplx<double>* twiddles<double>(int);
 template <typename R, int N> struct R2cShape {
     static constexpr int M = N / 2;
     static constexpr int NL = Geo<R>::NL;
-    // rows with a radix-3 factor: 8 instead of 16 complex values per thread measured faster
-    static constexpr int T = threads_for(M, NL) * ((M % 3 == 0 && M >= 96) ? 2 : 1);
+    // 8 complex values per thread, whole wavefronts (16, with 80 or 160 threads for rows of 160 or 320 points: 320^3
+    // float32 115 -> 86 us, float64 236 -> 114)
+    static constexpr int T = (2 * threads_for(M, NL) + 63) / 64 * 64;
     static constexpr int LDS = (M * (NL + 1) + N) * (int)sizeof(cplx<R>);
 };
 
@@ -407,9 +441,9 @@ static int r2c_job_n(const R* in, cplx<R>* out, long long nrows, int64_t P, bool
     PYL_CHECK(tw, E_ALLOC, "twiddle table allocation failed");
     int per_cu = (160 * 1024) / (SH::LDS + 1024);
     per_cu = per_cu < 1 ? 1 : (per_cu > 8 ? 8 : per_cu);
-    long long nb = (long long)cu_count() * per_cu;
+    // as the inverse (launch_c2r_rows): float64 one row block each (384^3 218 -> 160 us, 512^3 416 -> 372)
     const long long nrb = (nrows + SH::NL - 1) / SH::NL;
-    if (nb > nrb) nb = nrb;
+    const long long nb = sizeof(R) == 8 ? nrb : persistent_blocks(nrb, per_cu);
     *a = R2cArgs<R>{in, out, nrows, (long long)P, tw, affine ? 1 : 0, dmass, mass, (double)N * N * N};
     *blocks = (unsigned)nb;
     return OK;
@@ -441,12 +475,17 @@ static int launch_c2r_rows(const cplx<R>* in, R* out, long long nrows, int64_t P
                            const R* aux, double* acc, hipStream_t st, int K) {
     constexpr int M = N / 2;
     constexpr int NL = Geo<R>::NL;
-    // as pass Z forward, rounded up to whole wavefronts (the fused sums reduce over full waves):
-    // M = 80 or 160 points would otherwise give 80 or 160 threads
-    constexpr int T = (threads_for(M, NL) * ((M % 3 == 0 && M >= 96) ? 2 : 1) + 63) / 64 * 64;
+    // 8 complex values per thread (16: 256^3 float32 43 -> 30 us with twice the threads), whole wavefronts
+    constexpr int T = (2 * threads_for(M, NL) + 63) / 64 * 64;
     const cplx<R>* tw = twiddles<R>(N);
     PYL_CHECK(tw, E_ALLOC, "twiddle table allocation failed");
-    const long long nb = (nrows + NL - 1) / NL;
+    constexpr int LDS = (M * (NL + 1) + N) * (int)sizeof(cplx<R>);
+    int per_cu = (160 * 1024) / (LDS + 1024);
+    per_cu = per_cu < 1 ? 1 : (per_cu > 8 ? 8 : per_cu);
+    // float64: one row block each (the hardware keeps the CUs full better than rounds of persistent blocks do: 384^3
+    // 200 -> 162 us, 512^3 465 -> 420); float32: persistent (512^3 225 -> 210)
+    const long long nrb = (nrows + NL - 1) / NL;
+    const long long nb = sizeof(R) == 8 ? nrb : persistent_blocks(nrb, per_cu);
     double* part = nullptr;
     if (acc) {
         int rc = OK;
@@ -460,13 +499,6 @@ static int launch_c2r_rows(const cplx<R>* in, R* out, long long nrows, int64_t P
     PYL_HIP(hipGetLastError());
     return OK;
 }
-
-template <typename R, int N> struct ColShape {
-    static constexpr int NL = (N >= 1024 && sizeof(R) == 4) ? 8 : Geo<R>::NL;   // 1024-point lines: 8 per block
-    // 16 elements per thread (the prefetch doubles the first stage's registers)
-    static constexpr int T = clamp_i(N * NL / 16, 64, 512);
-    static constexpr int LDS = (N * NL + N) * (int)sizeof(cplx<R>);
-};
 
 template <typename R, int N>
 static int cols_job_n(const cplx<R>* src, cplx<R>* dst, int64_t P, int axis, R sc, int K, ColArgs<R>* a,

@@ -8,10 +8,17 @@
 
 namespace pyl {
 
+// the transform lengths
+#define PYL_FFT_SIZES(X) \
+    X(8) X(12) X(16) X(20) X(24) X(32) X(40) X(48) X(64) X(80) X(96) X(128) X(160) X(192) X(256) \
+    X(320) X(384) X(512) X(640) X(768) X(1024)
+
 bool fft_size_supported(int N);
 
 // compute units of the current device (cached)
 int cu_count();
+// workgroups of a persistent launch over `units` pieces of work, at most `most` resident a CU
+long long persistent_blocks(long long units, int most);
 
 // twiddle table exp(-2 pi i t/N), t in [0, N), cached per (N, precision); device pointer
 template <typename R> const cplx<R>* twiddles(int N);
@@ -68,6 +75,34 @@ template <typename R>
 int cols_job(const cplx<R>* src, cplx<R>* dst, int N, int64_t P, int axis, ColArgs<R>* a, unsigned* blocks);
 template <typename R>
 int cols_batch(int N, const ColArgs<R>* tab, const unsigned* start, int nj, unsigned total, hipStream_t st);
+
+// Row pitch of a library-owned spectrum: N / 2 + 1 rounded up to 128 bytes, so that the strided column passes read
+// whole cache lines
+template <typename R> inline int64_t padded_pitch(int N) {
+    constexpr int64_t A = 128 / (int64_t)sizeof(cplx<R>);
+    return (half_len(N) + A - 1) / A * A;
+}
+
+// Operation on the modes of a half spectrum, applied inside the pass along x (fft_pass_x_op)
+enum { XOP_FILTER = 0, XOP_WINDOW = 1, XOP_POWER = 2, XOP_GRAD = 3 };
+template <typename R> struct XOp {
+    int kind;
+    // XOP_FILTER: v *= filt (half spectrum of row pitch FP), products rounded one by one
+    const cplx<R>* filt = nullptr;
+    long long FP = 0;
+    // XOP_WINDOW: v *= W of the independent modes; XOP_POWER: v = (|W v|^2, 0)
+    const double* win = nullptr;
+    // XOP_GRAD: v *= H of the power spectrum's adjoint (adjoint.hip): weights w[nb] of the bins, their mode counts n3
+    const double* w = nullptr;
+    int nb = 0;
+    const unsigned long long* n3 = nullptr;
+    double unit = 0.0, post = 0.0;
+};
+// XOP_FILTER, XOP_WINDOW, XOP_POWER: forward transform along x, the operation, inverse transform along x, in one pass
+// over the spectrum; XOP_GRAD: the operation, then the inverse transform along x.  src (row pitch SP) -> dst (row
+// pitch P; may alias when SP == P).  FILTER and GRAD: float32.
+template <typename R>
+int fft_pass_x_op(const cplx<R>* src, int64_t SP, cplx<R>* dst, int N, int64_t P, const XOp<R>& op, hipStream_t st);
 
 // full transforms; with K > 0 only the modes kz < K of the r2c are complete (the column passes
 // skip the others, which keep the pass-Z values)

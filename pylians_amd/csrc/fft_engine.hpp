@@ -257,4 +257,12 @@ constexpr int clamp_i(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi
 // threads per block for NL lines of length N: about 16 elements per thread
 constexpr int threads_for(int N, int NL) { return clamp_i(N * NL / 16, 64, 256); }
 
+// launch shape of the column passes
+template <typename R, int N> struct ColShape {
+    static constexpr int NL = (N >= 1024 && sizeof(R) == 4) ? 8 : Geo<R>::NL;   // 1024-point lines: 8 per block
+    // 16 elements per thread (the prefetch doubles the first stage's registers)
+    static constexpr int T = clamp_i(N * NL / 16, 64, 512);
+    static constexpr int LDS = (N * NL + N) * (int)sizeof(cplx<R>);
+};
+
 }  // namespace pyl

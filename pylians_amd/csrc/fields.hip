@@ -24,52 +24,6 @@ namespace pyl {
 
 const double* pk_window_table(int N, int p);
 
-// ------------------------------------------------------------------ half-spectrum mode kernels
-// v *= (float)(W_x W_y W_z); optionally only the independent modes; optionally v = (|v|^2, 0)
-template <typename R>
-__global__ __launch_bounds__(256) void k_modes(cplx<R>* __restrict__ spec, int N, long long P,
-                                               const double* __restrict__ win, int indep_only, int square) {
-#pragma clang fp contract(off)
-    const int W = N / 2 + 1, middle = N / 2;
-    const bool even = (N % 2) == 0;
-    const long long total = (long long)N * N * W;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-         i += (long long)gridDim.x * blockDim.x) {
-        const int x = (int)(i / ((long long)N * W)), y = (int)((i / W) % N), kz = (int)(i % W);
-        if (indep_only && (kz == 0 || (kz == middle && even))) {
-            const int kx = kfreq(x, N), ky = kfreq(y, N);
-            if (kx < 0 || ((kx == 0 || (kx == middle && even)) && ky < 0)) continue;
-        }
-        const R f = (R)(win[x] * win[y] * win[kz]);
-        cplx<R>* v = spec + ((long long)x * N + y) * P + kz;
-        cplx<R> a = *v;
-        a.x = a.x * f;
-        a.y = a.y * f;
-        if (square) {
-            const R re = a.x * a.x, im = a.y * a.y;
-            a.x = re + im;
-            a.y = (R)0;
-        }
-        *v = a;
-    }
-}
-
-// spec *= filt (complex multiply in the field precision); both with row pitch P
-template <typename R>
-__global__ __launch_bounds__(256) void k_cmul(cplx<R>* __restrict__ spec, const cplx<R>* __restrict__ filt, int N,
-                                              long long P) {
-#pragma clang fp contract(off)
-    const int W = N / 2 + 1;
-    const long long total = (long long)N * N * W;
-    for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < total;
-         i += (long long)gridDim.x * blockDim.x) {
-        const long long row = i / W, kz = i % W;
-        const cplx<R> a = spec[row * P + kz], b = filt[row * P + kz];
-        const R ac = a.x * b.x, bd = a.y * b.y, ad = a.x * b.y, bc = a.y * b.x;
-        spec[row * P + kz] = mk(ac - bd, ad + bc);
-    }
-}
-
 // ------------------------------------------------------------------ Xi binning
 // One wavefront per row (x, y); lane l owns the z pairs u in [l*EU, (l+1)*EU) (z = u and N-u).
 // LDS bins (kmax+1) x {sum r, sum xi L0, sum xi L2, sum xi L4, count}; per-block rows of partials.
@@ -212,44 +166,38 @@ static int check_dims(int dims, int prec) {
     return OK;
 }
 
+// field -> r2c -> operation on the modes -> 1/N^3-normalised c2r: rows, y, (x forward, operation, x inverse), y, rows
+template <typename R>
+static int through_modes(const R* in, R* out, int N, const XOp<R>& op, hipStream_t st) {
+    int rc = OK;
+    const int64_t P = padded_pitch<R>(N);
+    cplx<R>* spec = (cplx<R>*)workspace(WS_SPEC, sizeof(cplx<R>) * (size_t)N * N * P, &rc);
+    if (rc) return rc;
+    if ((rc = fft_pass_z_r2c<R>(in, spec, N, P, false, nullptr, 1.0, st))) return rc;
+    if ((rc = fft_pass_cols<R>(spec, spec, N, P, 1, false, (R)1, st))) return rc;
+    if ((rc = fft_pass_x_op<R>(spec, P, spec, N, P, op, st))) return rc;
+    if ((rc = fft_pass_cols<R>(spec, spec, N, P, 1, true, (R)1, st))) return rc;
+    return fft_pass_z_c2r<R>(spec, out, N, P, (R)(1.0 / ((double)N * N * N)), 1, nullptr, nullptr, st);
+}
+
 template <typename R>
 static int correct_mas_run(const R* in, R* out, int N, int p, hipStream_t st) {
-    int rc = OK;
-    const int64_t P = half_len(N);
-    const size_t nspec = (size_t)N * N * P;
-    cplx<R>* spec = (cplx<R>*)workspace(WS_SPEC, sizeof(cplx<R>) * nspec, &rc);
-    if (rc) return rc;
-    cplx<R>* ws = (cplx<R>*)workspace(WS_SPEC2, sizeof(cplx<R>) * nspec, &rc);
-    if (rc) return rc;
-    const double* win = pk_window_table(N, p);
-    PYL_CHECK(win, E_ALLOC, "window table allocation failed");
-    rc = fft3d_r2c<R>(in, spec, N, P, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_modes<R>, dim3(grid_for((long long)nspec)), dim3(256), 0, st, spec, N, (long long)P, win, 1, 0);
-    PYL_HIP(hipGetLastError());
-    return fft3d_c2r<R>(spec, out, ws, N, P, (R)(1.0 / ((double)N * N * N)), st);
+    XOp<R> op{XOP_WINDOW};
+    op.win = pk_window_table(N, p);
+    PYL_CHECK(op.win, E_ALLOC, "window table allocation failed");
+    return through_modes<R>(in, out, N, op, st);
 }
 
 template <typename R>
 static int xi_run(const R* in, int N, double BoxSize, int p, int axis, double* out, hipStream_t st) {
     int rc = OK;
-    const int64_t P = half_len(N);
-    const size_t nspec = (size_t)N * N * P;
     const size_t ncell = (size_t)N * N * N;
-    cplx<R>* spec = (cplx<R>*)workspace(WS_SPEC, sizeof(cplx<R>) * nspec, &rc);
-    if (rc) return rc;
-    cplx<R>* ws = (cplx<R>*)workspace(WS_SPEC2, sizeof(cplx<R>) * nspec, &rc);
-    if (rc) return rc;
     R* fxi = (R*)workspace(WS_GRID, sizeof(R) * ncell, &rc);
     if (rc) return rc;
-    const double* win = pk_window_table(N, p);
-    PYL_CHECK(win, E_ALLOC, "window table allocation failed");
-    rc = fft3d_r2c<R>(in, spec, N, P, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_modes<R>, dim3(grid_for((long long)nspec)), dim3(256), 0, st, spec, N, (long long)P, win, 0, 1);
-    PYL_HIP(hipGetLastError());
-    rc = fft3d_c2r<R>(spec, fxi, ws, N, P, (R)(1.0 / ((double)N * N * N)), st);
-    if (rc) return rc;
+    XOp<R> op{XOP_POWER};
+    op.win = pk_window_table(N, p);
+    PYL_CHECK(op.win, E_ALLOC, "window table allocation failed");
+    if ((rc = through_modes<R>(in, fxi, N, op, st))) return rc;
     const int middle = N / 2;
     int kmax = 0;
     while ((long long)(kmax + 1) * (kmax + 1) <= 3LL * middle * middle) ++kmax;
@@ -354,18 +302,10 @@ extern "C" int pyl_field_smoothing(const void* field, const void* filter_k, void
     if (rc) return rc;
     PYL_CHECK(field && filter_k && out, E_ARG, "null pointer");
     hipStream_t st = (hipStream_t)stream;
-    const int64_t P = half_len(dims);
-    const size_t nspec = (size_t)dims * dims * P;
-    cplx<float>* spec = (cplx<float>*)workspace(WS_SPEC, sizeof(cplx<float>) * nspec, &rc);
-    if (rc) return rc;
-    cplx<float>* ws = (cplx<float>*)workspace(WS_SPEC2, sizeof(cplx<float>) * nspec, &rc);
-    if (rc) return rc;
-    rc = fft3d_r2c<float>((const float*)field, spec, dims, P, st);
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_cmul<float>, dim3(grid_for((long long)nspec)), dim3(256), 0, st, spec,
-                       (const cplx<float>*)filter_k, dims, (long long)P);
-    PYL_HIP(hipGetLastError());
-    return fft3d_c2r<float>(spec, (float*)out, ws, dims, P, (float)(1.0 / ((double)dims * dims * dims)), st);
+    XOp<float> op{XOP_FILTER};
+    op.filt = (const cplx<float>*)filter_k;
+    op.FP = half_len(dims);
+    return through_modes<float>((const float*)field, (float*)out, dims, op, st);
 }
 
 extern "C" int pyl_field_div_sub(void* field, int64_t n, double div, double sub, int prec, void* stream) {

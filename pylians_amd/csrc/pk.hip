@@ -463,9 +463,9 @@ __device__ __forceinline__ void last_bin_body(const LastBinArgs<R>& A, Blk B) {
     auto fetch = [&](int it, cplx<R> (&v)[F::B][F::RAD]) {
         int u, kzz;
         item(it, u, kzz);
-        const bool ok = kzz < W;
-        const long long b = (long long)u * UST + kzz;
-        first_load<R, N, NL, T>(v, [&](int j, int) { return ok ? src[b + j * EST] : mk<R>(0, 0); }, tid);
+        // unconditional, so that the loads stay in flight: columns past kz = N/2 read column 0 and are not binned
+        const cplx<R>* p = src + (kzz < W ? (long long)u * UST + kzz : 0);
+        first_load<R, N, NL, T>(v, [&](int j, int) { return p[j * EST]; }, tid);
     };
     cplx<R> nxt[F::B][F::RAD];
     if (nit > 0) fetch(0, nxt);
