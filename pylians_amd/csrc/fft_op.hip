@@ -1,7 +1,7 @@
 // The pass along x of a transform pair with an operation on the modes between its two halves: the column is
 // transformed forward, multiplied and transformed back while it is in LDS.  As separate passes (forward, product,
 // inverse) a 512^3 float32 field took 270 + 412 + 350 us; the spectrum is now read and written once (with the filter,
-// 1.6 GB): 475 us.
+// 1.6 GB): 443 us.
 #include <math.h>
 
 #include <algorithm>
@@ -70,6 +70,30 @@ template <int N, int NL, int T> struct Last {
     static constexpr int B = (NBF + T - 1) / T;
 };
 
+// Keeps the compiler from rearranging what made v with what uses it.  The contraction of a butterfly's products into
+// fused multiply-adds depends on its surroundings; with its outputs settled the pass rounds as the plain one does.
+template <typename R> __device__ __forceinline__ cplx<R> settle(cplx<R> v) {
+    asm volatile("" : "+v"(v.x), "+v"(v.y));
+    return v;
+}
+
+// The radix-5 butterfly of fft_engine.hpp with the fused operations of its two sums written out, as the plain passes
+// have them (left to the compiler, the other product was fused here)
+template <typename R> __device__ __forceinline__ void dft5(cplx<R>* a) {
+    const R c1 = (R)0.30901699437494742410229341718282, c2 = (R)-0.80901699437494742410229341718282;
+    const R s1 = (R)0.95105651629515357211643933337938, s2 = (R)0.58778525229247312916870595463907;
+    const cplx<R> p1 = a[1] + a[4], d1 = a[1] - a[4], p2 = a[2] + a[3], d2 = a[2] - a[3];
+    const cplx<R> m1 = mk(a[0].x + c1 * p1.x + c2 * p2.x, a[0].y + c1 * p1.y + c2 * p2.y);
+    const cplx<R> m2 = mk(a[0].x + c2 * p1.x + c1 * p2.x, a[0].y + c2 * p1.y + c1 * p2.y);
+    const cplx<R> r1 = mul_mi(mk((R)fma(s1, d1.x, s2 * d2.x), (R)fma(s1, d1.y, s2 * d2.y)));
+    const cplx<R> r2 = mul_mi(mk(s2 * d1.x - s1 * d2.x, s2 * d1.y - s1 * d2.y));
+    a[0] = a[0] + p1 + p2;
+    a[1] = m1 + r1;
+    a[4] = m1 - r1;
+    a[2] = m2 + r2;
+    a[3] = m2 - r2;
+}
+
 // Last stage of a forward transform in LDS, each output handed to f(k, value, b, m) and its result left in LDS in
 // natural order, conjugated for the inverse transform.
 template <typename R, int N, int NL, int T, class FN>
@@ -84,6 +108,14 @@ __device__ __forceinline__ void last_stage_op(cplx<R>* s, const cplx<R>* tw, FN&
             const int l = g % NL, j = g / NL;
 #pragma unroll
             for (int m = 0; m < RAD; ++m) v[b][m] = s[(j + m * NS) * NL + l];
+#pragma unroll
+            for (int m = 1; m < RAD; ++m) v[b][m] = cmul(v[b][m], tw[m * j * (N / (NS * RAD))]);
+            if constexpr (RAD == 5)
+                dft5(v[b]);
+            else
+                Dft<R, RAD>::run(v[b]);
+#pragma unroll
+            for (int m = 0; m < RAD; ++m) v[b][m] = settle(v[b][m]);
         }
     }
     __syncthreads();
@@ -92,9 +124,6 @@ __device__ __forceinline__ void last_stage_op(cplx<R>* s, const cplx<R>* tw, FN&
         const int g = tid + b * T;
         if (NBF % T == 0 || g < NBF) {
             const int l = g % NL, j = g / NL;
-#pragma unroll
-            for (int m = 1; m < RAD; ++m) v[b][m] = cmul(v[b][m], tw[m * j * (N / (NS * RAD))]);
-            Dft<R, RAD>::run(v[b]);
 #pragma unroll
             for (int m = 0; m < RAD; ++m) s[(j + m * NS) * NL + l] = conjg(f(j + m * NS, v[b][m], b, m));
         }
@@ -170,7 +199,7 @@ __global__ __launch_bounds__(T) void k_cols_op(XArgs<R> A) {
             } else {
                 using L = Last<N, NL, T>;
                 first_stage_regs<R, N, NL, NL, T>(s, cur, tid);
-                // the filter values of the thread's outputs load during the middle stages (512^3: 535 -> 475 us)
+                // the filter values of the thread's outputs load during the middle stages (512^3: 60 us off)
                 cplx<R> fv[L::B][L::RAD];
                 if constexpr (KIND == XOP_FILTER) {
 #pragma unroll
@@ -185,7 +214,7 @@ __global__ __launch_bounds__(T) void k_cols_op(XArgs<R> A) {
                     s, tw, [&](int k, cplx<R> v, int b, int m) { return op(k, v, KIND == XOP_FILTER ? fv[b][m] : none); },
                     tid);
             }
-            first_load<R, N, NL, T>(cur, [&](int j, int) { return s[j * NL + l]; }, tid);
+            first_load<R, N, NL, T>(cur, [&](int j, int) { return settle(s[j * NL + l]); }, tid);
             __syncthreads();
         } else {
 #pragma unroll
