@@ -259,6 +259,16 @@ int pyl_graph_destroy(void* graph);
 int pyl_pk_adjoint(const float* pos, int64_t n, int dims, double BoxSize, int scheme, const double* w, int nb,
                    float* grad, double* out, void* stream);
 
+/* The same in two halves, for callers that need P0 before the weights are known (automatic
+ * differentiation): pyl_pk_forward_keep is pyl_pk_particles (float32, no weights, axis 0, no 1-D / 2-D
+ * / phase outputs; deposit and mode check as there) and also writes the window-corrected half spectrum
+ * to spec, device complex64 (dims, dims, dims/2+1) owned by the caller; pyl_pk_adjoint_keep forms the
+ * gradient from it.  spec is not modified. */
+int pyl_pk_forward_keep(const float* pos, int64_t n, int dims, double BoxSize, int scheme, void* spec, double* out,
+                        void* stream);
+int pyl_pk_adjoint_keep(const float* pos, int64_t n, int dims, double BoxSize, int scheme, const double* w, int nb,
+                        const void* spec, float* grad, void* stream);
+
 /* Replaces MAS_library.CIC_interp(density, BoxSize, pos, den) (MAS_library.pyx:558-599) for scheme 2,
  * and generalises it to NGP/TSC/PCS: out[p] = sum over the stencil cells of density * weight.
  * density: device float32 (dims^3); pos: device float32 (n, 3); out: device float32 (n). */

@@ -72,6 +72,8 @@ SIGNATURES = {
     "pyl_field_smoothing": [_vp, _vp, _vp, _i, _vp],
     "pyl_bk": [_vp, _i, _d, _d, _d, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp],
     "pyl_pk_adjoint": [_vp, _i64, _i, _d, _i, _vp, _i, _vp, _vp, _vp],
+    "pyl_pk_forward_keep": [_vp, _i64, _i, _d, _i, _vp, _vp, _vp],
+    "pyl_pk_adjoint_keep": [_vp, _i64, _i, _d, _i, _vp, _i, _vp, _vp, _vp],
     "pyl_interp": [_vp, _i, _d, _vp, _i64, _i, _vp, _vp],
     "pyl_pk_batch": [_vp, _i, _vp],
     "pyl_graph_create": [_vp, _i, _vp, _vp],

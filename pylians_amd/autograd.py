@@ -5,9 +5,11 @@ adjoint (pyl_pk_adjoint).  Builder-defined; the reference has no gradients.
     loss = (w * P0).sum(); loss.backward()                 # pos.grad: (n, 3) float32
 
 Forward: fused deposit -> delta = rho/rhobar - 1 -> r2c -> window deconvolution -> binning
-(float32 grid and FFT, float64 shell sums).  Backward: the same forward recomputed on the GPU, the
-gradient spectrum H_k = (dL/dP0_b) (L/N^2)^3 / Nmodes_b c_k^2 delta_k, an unnormalised c2r and the
-stencil-derivative gather at the particles.
+(float32 grid and FFT, float64 shell sums); when a gradient is asked for, the corrected half spectrum
+is saved for the backward pass (complex64, dims x dims x (dims/2 + 1); computing it again instead
+would cost the forward pass a second time).  Backward: the gradient spectrum
+H_k = (dL/dP0_b) (L/N^2)^3 / Nmodes_b c_k^2 delta_k, an unnormalised c2r and the stencil-derivative
+gather at the particles.
 """
 import torch
 
@@ -21,27 +23,30 @@ def _kmax(dims):
 
 class _P0(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, pos, BoxSize, dims, scheme, nbins):
+    def forward(ctx, pos, BoxSize, dims, scheme, nbins, needs_grad):
         p = pos.detach().to(torch.float32).contiguous()
         _, _, kmax, nout = pk_layout(dims)
         out = torch.empty(nout, dtype=torch.float64, device=p.device)
-        _lib.check(_lib.lib().pyl_pk_particles(_lib.ptr(p), None, int(p.shape[0]), int(dims), float(BoxSize),
-                                               int(scheme), 0, _lib.F32, 0, _lib.ptr(out), _lib.stream()))
-        ctx.save_for_backward(p)
+        if needs_grad:
+            spec = torch.empty((dims, dims, dims // 2 + 1), dtype=torch.complex64, device=p.device)
+            _lib.check(_lib.lib().pyl_pk_forward_keep(_lib.ptr(p), int(p.shape[0]), int(dims), float(BoxSize),
+                                                      int(scheme), _lib.ptr(spec), _lib.ptr(out), _lib.stream()))
+            ctx.save_for_backward(p, spec)
+        else:
+            _lib.check(_lib.lib().pyl_pk_particles(_lib.ptr(p), None, int(p.shape[0]), int(dims), float(BoxSize),
+                                                   int(scheme), 0, _lib.F32, 0, _lib.ptr(out), _lib.stream()))
         ctx.cfg = (float(BoxSize), int(dims), int(scheme), int(nbins))
         return out[kmax:kmax + nbins].clone()
 
     @staticmethod
     def backward(ctx, gP0):
-        (p,) = ctx.saved_tensors
+        p, spec = ctx.saved_tensors
         BoxSize, dims, scheme, nbins = ctx.cfg
         w = gP0.detach().to(torch.float64).contiguous()
         grad = torch.empty_like(p)
-        _, _, _, nout = pk_layout(dims)
-        out = torch.empty(nout, dtype=torch.float64, device=p.device)
-        _lib.check(_lib.lib().pyl_pk_adjoint(_lib.ptr(p), int(p.shape[0]), dims, BoxSize, scheme, _lib.ptr(w),
-                                             nbins, _lib.ptr(grad), _lib.ptr(out), _lib.stream()))
-        return grad, None, None, None, None
+        _lib.check(_lib.lib().pyl_pk_adjoint_keep(_lib.ptr(p), int(p.shape[0]), dims, BoxSize, scheme, _lib.ptr(w),
+                                                  nbins, _lib.ptr(spec), _lib.ptr(grad), _lib.stream()))
+        return grad, None, None, None, None, None
 
 
 def pk0(pos, BoxSize, dims, MAS="CIC", nbins=None):
@@ -55,7 +60,8 @@ def pk0(pos, BoxSize, dims, MAS="CIC", nbins=None):
         raise ValueError("nbins must be in [1, %d]" % kmax)
     if not (isinstance(pos, torch.Tensor) and pos.is_cuda and pos.ndim == 2 and pos.shape[1] == 3):
         raise ValueError("pos must be a (n, 3) tensor on the GPU")
-    return _P0.apply(pos, BoxSize, dims, _lib.SCHEMES[MAS], nbins)
+    needs_grad = torch.is_grad_enabled() and pos.requires_grad
+    return _P0.apply(pos, BoxSize, int(dims), _lib.SCHEMES[MAS], nbins, needs_grad)
 
 
 def grad_loss(pos, BoxSize, dims, w, MAS="CIC"):

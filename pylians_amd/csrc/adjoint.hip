@@ -3,6 +3,7 @@
 // loss = sum_b w_b P0_b with P0_b = (L/N^2)^3 / Nmodes_b * sum_{independent k in bin b} |c_k delta_k|^2
 // (Pk_library.pyx:314-381, 410-417), delta = rho/rhobar - 1.  Then
 //   dL/d delta(x) = sum_{all k} H_k e^{i k x},  H_k = w_b (L/N^2)^3 / Nmodes_b c_k^2 delta_k
+// (the factor of delta_k is applied inside the inverse transform's pass along x, XOP_GRAD of fft_op.hip)
 // over the Hermitian-extended half spectrum, doubled on the self-conjugate modes (counted once in
 // the full-space sum but twice in d|delta_k|^2); dL/d rho = dL/d delta / rhobar; and
 //   dL/d pos_{p,a} = (N/L) sum_cells G(cell) W'_a prod_{b != a} W_b
@@ -11,31 +12,32 @@
 #include <math.h>
 
 #include "adjoint.hpp"
+#include "stencil.hpp"
 
 namespace pyl {
 
 // 1-D kernel and derivative (d/d dist) of the schemes, float64, same stencil cells as deposit.hip
 template <int S> struct AxisD;
 template <> struct AxisD<1> {
-    static __device__ __forceinline__ long long eval(double d, double* w, double* dw) {
+    static __device__ __forceinline__ double eval(double d, double* w, double* dw) {
         w[0] = 1.0;
         dw[0] = 0.0;
-        return (long long)floor(d + 0.5);
+        return floor(d + 0.5);
     }
 };
 template <> struct AxisD<2> {
-    static __device__ __forceinline__ long long eval(double d, double* w, double* dw) {
+    static __device__ __forceinline__ double eval(double d, double* w, double* dw) {
         const double b = floor(d);
         const double u = d - b;
         w[0] = 1.0 - u;
         w[1] = u;
         dw[0] = -1.0;
         dw[1] = 1.0;
-        return (long long)b;
+        return b;
     }
 };
 template <> struct AxisD<3> {
-    static __device__ __forceinline__ long long eval(double d, double* w, double* dw) {
+    static __device__ __forceinline__ double eval(double d, double* w, double* dw) {
         const double mn = floor(d - 1.5);
 #pragma unroll
         for (int j = 0; j < 3; ++j) {
@@ -52,11 +54,11 @@ template <> struct AxisD<3> {
                 dw[j] = 0.0;
             }
         }
-        return (long long)mn + 1;
+        return mn + 1.0;
     }
 };
 template <> struct AxisD<4> {
-    static __device__ __forceinline__ long long eval(double d, double* w, double* dw) {
+    static __device__ __forceinline__ double eval(double d, double* w, double* dw) {
         const double mn = floor(d - 2.0);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -73,14 +75,9 @@ template <> struct AxisD<4> {
                 dw[j] = 0.0;
             }
         }
-        return (long long)mn + 1;
+        return mn + 1.0;
     }
 };
-
-__device__ __forceinline__ int wrap_i(long long b, int N) {
-    long long r = b % N;
-    return (int)(r < 0 ? r + N : r);
-}
 
 // GRAD: out[3p..3p+2] = scale * dL/dpos;  else out[p] = sum_cells G * W (interpolation)
 template <int S, bool GRAD>
@@ -92,7 +89,7 @@ __global__ __launch_bounds__(256) void k_gather(const float* __restrict__ G, int
         int ix[3][S];
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            const int b = wrap_i(AxisD<S>::eval((double)pos[3 * p + a] * inv, w[a], dw[a]), N);
+            const int b = wrapN(AxisD<S>::eval((double)pos[3 * p + a] * inv, w[a], dw[a]), N);
 #pragma unroll
             for (int j = 0; j < S; ++j) ix[a][j] = b + j >= N ? b + j - N : b + j;
         }
@@ -153,55 +150,5 @@ int interp(const float* G, int N, double BoxSize, const float* pos, int64_t n, i
     if (n <= 0) return OK;
     return launch_gather<false>(G, N, pos, n, N / BoxSize, 1.0, scheme, out, st);
 }
-
-// H = g(bin) * fac * keep, keep = window-corrected spectrum on independent modes, raw elsewhere
-template <typename R>
-__global__ __launch_bounds__(256) void k_grad_spec(cplx<R>* __restrict__ spec, int N, long long P,
-                                                   const double* __restrict__ w, int nb,
-                                                   const unsigned long long* __restrict__ n3, double unit,
-                                                   const double* __restrict__ win, double post) {
-    const long long total = (long long)N * N * P;
-    const int middle = N / 2;
-    const bool even = (N % 2) == 0;
-    for (long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x; id < total;
-         id += (long long)gridDim.x * blockDim.x) {
-        const int kzz = (int)(id % P);
-        const long long t = id / P;
-        const int yy = (int)(t % N), xx = (int)(t / N);
-        if (kzz > middle) continue;
-        const int kx = kfreq(xx, N), ky = kfreq(yy, N), kz = kzz;
-        const int k2 = kx * kx + ky * ky + kz * kz;   // <= 3 (N/2)^2 < 2^24
-        const int bin = isqrt24(k2);
-        double g = 0.0;
-        if (bin >= 1 && bin <= nb) g = w[bin - 1] * unit / (double)n3[bin];
-        const double c = win[xx] * win[yy] * win[kzz];
-        bool ind = true;
-        if (kz == 0 || (kz == middle && even)) {
-            if (kx < 0) ind = false;
-            else if ((kx == 0 || (kx == middle && even)) && ky < 0) ind = false;
-        }
-        double f = g * (ind ? c : c * c) * post;
-        if (even && (kx == 0 || kx == middle) && (ky == 0 || ky == middle) && (kz == 0 || kz == middle)) f *= 2.0;
-        spec[id] = scale(spec[id], (R)f);
-    }
-}
-
-template <typename R>
-int grad_spectrum(cplx<R>* spec, int N, int64_t P, const double* w, int nb, const unsigned long long* n3,
-                  double BoxSize, const double* win, double post, hipStream_t st) {
-    const double u1 = BoxSize / ((double)N * N);
-    const double unit = u1 * u1 * u1;
-    const long long total = (long long)N * N * P;
-    long long blocks = (total + 255) / 256;
-    if (blocks > 65536) blocks = 65536;
-    hipLaunchKernelGGL((k_grad_spec<R>), dim3((unsigned)blocks), dim3(256), 0, st, spec, N, (long long)P, w, nb, n3,
-                       unit, win, post);
-    PYL_HIP(hipGetLastError());
-    return OK;
-}
-template int grad_spectrum<float>(cplx<float>*, int, int64_t, const double*, int, const unsigned long long*, double,
-                                  const double*, double, hipStream_t);
-template int grad_spectrum<double>(cplx<double>*, int, int64_t, const double*, int, const unsigned long long*,
-                                   double, const double*, double, hipStream_t);
 
 }  // namespace pyl

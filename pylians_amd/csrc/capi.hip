@@ -374,7 +374,7 @@ int deposit_kind(const float* pos, const float* W, int64_t n, int dims, double B
 }
 
 int pk_particles(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, int axis,
-                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd) {
+                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd, cplx<float>* keep) {
     int rc = check_fft(dims, prec);
     if (rc) return rc;
     PYL_CHECK(axis >= 0 && axis <= 2, E_ARG, "axis must be 0, 1 or 2");
@@ -402,7 +402,7 @@ int pk_particles(const float* pos, const float* W, int64_t n, int dims, double B
     if (f64)
         return pk_from_delta<double>((const double*)grid, dims, BoxSize, axis, scheme, pkflags, out, nullptr,
                                      kind == DK_ATOMIC, dmass, (double)n, st);
-    return pk_from_delta<float>((const float*)grid, dims, BoxSize, axis, scheme, pkflags, out, nullptr, false,
+    return pk_from_delta<float>((const float*)grid, dims, BoxSize, axis, scheme, pkflags, out, keep, false,
                                 dmass, (double)n, st);
 }
 }  // namespace pyl
@@ -463,20 +463,57 @@ extern "C" int pyl_pos_redshift_space(float* pos, const float* vel, int64_t n, i
 }
 
 // ------------------------------------------------------------------ adjoint and interpolation
-extern "C" int pyl_pk_adjoint(const float* pos, int64_t n, int dims, double BoxSize, int scheme, const double* w,
-                              int nb, float* grad, double* out, void* stream) {
+// dL/dpos from the kept spectrum of the forward pass (row pitch N / 2 + 1, not modified): gradient spectrum and inverse
+// transform along x in one pass, then y, rows, and the gather at the particles
+static int adjoint_from(const float* pos, int64_t n, int dims, double BoxSize, int scheme, const double* w, int nb,
+                        const cplx<float>* keep, float* grad, hipStream_t st) {
+    int rc = OK;
+    const int64_t P = padded_pitch<float>(dims);
+    const PkGeometry* g = pk_geometry(dims, 0, &rc);
+    if (rc) return rc;
+    XOp<float> op{XOP_GRAD};
+    op.win = pk_window_table(dims, scheme);
+    PYL_CHECK(op.win, E_ALLOC, "window table allocation failed");
+    op.w = w;
+    op.nb = nb;
+    op.n3 = g->n3;
+    const double u1 = BoxSize / ((double)dims * dims);
+    op.unit = u1 * u1 * u1;
+    op.post = 1.0 / ((double)n / ((double)dims * dims * dims));
+    float* grid = (float*)workspace(WS_GRID, sizeof(float) * (size_t)dims * dims * dims, &rc);
+    if (rc) return rc;
+    cplx<float>* ws = (cplx<float>*)workspace(WS_SPEC, sizeof(cplx<float>) * (size_t)dims * dims * P, &rc);
+    if (rc) return rc;
+    {
+        StageTimer t("adj_c2r", st);
+        if ((rc = fft_pass_x_op<float>(keep, half_len(dims), ws, dims, P, op, st))) return rc;
+        if ((rc = fft_pass_cols<float>(ws, ws, dims, P, 1, true, 1.0f, st))) return rc;
+        if ((rc = fft_pass_z_c2r<float>(ws, grid, dims, P, 1.0f, 1, nullptr, nullptr, st))) return rc;
+    }
+    StageTimer t("adj_gather", st);
+    return gather_grad(grid, dims, BoxSize, pos, n, scheme, 1.0, grad, st);
+}
+
+static int check_adjoint(int64_t n, int dims, int scheme, int nb) {
     int rc = check_fft(dims, PYL_F32);
     if (rc) return rc;
     PYL_CHECK(scheme >= 1 && scheme <= 4, E_ARG, "unknown mass-assignment scheme %d", scheme);
-    PYL_CHECK(n > 0 && pos && w && grad && out, E_ARG, "bad arguments");
+    PYL_CHECK(n > 0, E_ARG, "bad arguments");
     const PkDims d = pk_dims(dims, half_len(dims));
     PYL_CHECK(nb >= 0 && nb <= d.kmax, E_ARG, "nb must be in [0, kmax = %d]", d.kmax);
+    return OK;
+}
+
+extern "C" int pyl_pk_adjoint(const float* pos, int64_t n, int dims, double BoxSize, int scheme, const double* w,
+                              int nb, float* grad, double* out, void* stream) {
+    int rc = check_adjoint(n, dims, scheme, nb);
+    if (rc) return rc;
+    PYL_CHECK(pos && w && grad && out, E_ARG, "bad arguments");
     hipStream_t st = (hipStream_t)stream;
-    const int64_t P = half_len(dims);
     const size_t cells = (size_t)dims * dims * dims;
     float* grid = (float*)workspace(WS_GRID, cells * 4, &rc);
     if (rc) return rc;
-    cplx<float>* keep = (cplx<float>*)workspace(WS_SPEC2, sizeof(cplx<float>) * (size_t)dims * dims * P, &rc);
+    cplx<float>* keep = (cplx<float>*)workspace(WS_SPEC2, sizeof(cplx<float>) * (size_t)dims * dims * half_len(dims), &rc);
     if (rc) return rc;
     // forward: delta, spectrum (kept, window-corrected) and the binned outputs (out = P0 etc.)
     const int kind = binned_supported(3, dims) ? DK_BINNED : DK_ATOMIC;
@@ -487,25 +524,22 @@ extern "C" int pyl_pk_adjoint(const float* pos, int64_t n, int dims, double BoxS
     }
     rc = pk_from_delta<float>(grid, dims, BoxSize, 0, scheme, PK_ASYNC, out, keep, false, nullptr, (double)n, st);
     if (rc) return rc;
-    const PkGeometry* g = pk_geometry(dims, 0, &rc);
+    return adjoint_from(pos, n, dims, BoxSize, scheme, w, nb, keep, grad, st);
+}
+
+extern "C" int pyl_pk_forward_keep(const float* pos, int64_t n, int dims, double BoxSize, int scheme, void* spec,
+                                   double* out, void* stream) {
+    PYL_CHECK(spec, E_ARG, "null spectrum");
+    return pk_particles(pos, nullptr, n, dims, BoxSize, scheme, 0, PYL_F32, 0, out, (hipStream_t)stream, Rsd(),
+                        (cplx<float>*)spec);
+}
+
+extern "C" int pyl_pk_adjoint_keep(const float* pos, int64_t n, int dims, double BoxSize, int scheme, const double* w,
+                                   int nb, const void* spec, float* grad, void* stream) {
+    int rc = check_adjoint(n, dims, scheme, nb);
     if (rc) return rc;
-    const double* win = pk_window_table(dims, scheme);
-    PYL_CHECK(win, E_ALLOC, "window table allocation failed");
-    const double rhobar = (double)n / ((double)dims * dims * dims);
-    {
-        StageTimer t("adj_grad_spectrum", st);
-        rc = grad_spectrum<float>(keep, dims, P, w, nb, g->n3, BoxSize, win, 1.0 / rhobar, st);
-        if (rc) return rc;
-    }
-    {
-        StageTimer t("adj_c2r", st);
-        cplx<float>* ws = (cplx<float>*)workspace(WS_SPEC, sizeof(cplx<float>) * (size_t)dims * dims * P, &rc);
-        if (rc) return rc;
-        rc = fft3d_c2r<float>(keep, grid, ws, dims, P, 1.0f, st);
-        if (rc) return rc;
-    }
-    StageTimer t("adj_gather", st);
-    return gather_grad(grid, dims, BoxSize, pos, n, scheme, 1.0, grad, st);
+    PYL_CHECK(pos && w && spec && grad, E_ARG, "bad arguments");
+    return adjoint_from(pos, n, dims, BoxSize, scheme, w, nb, (const cplx<float>*)spec, grad, (hipStream_t)stream);
 }
 
 extern "C" int pyl_interp(const float* density, int dims, double BoxSize, const float* pos, int64_t n, int scheme,

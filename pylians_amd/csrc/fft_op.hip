@@ -20,9 +20,10 @@ template <typename R> struct XArgs {
     XOp<R> op;
 };
 
-// the operation on the mode (x, y, kz); b: its filter value (XOP_FILTER)
+// the operation on the mode (x, y, kz); b: its filter value (XOP_FILTER); gbin: w_b unit / Nmodes_b per 3-D bin, 0 for
+// the bins without weight (XOP_GRAD)
 template <typename R, int N, int KIND>
-__device__ __forceinline__ cplx<R> mode_op(const XOp<R>& op, cplx<R> a, cplx<R> b, int x, int y, int kz) {
+__device__ __forceinline__ cplx<R> mode_op(const XOp<R>& op, cplx<R> a, cplx<R> b, const double* gbin, int x, int y, int kz) {
 #pragma clang fp contract(off)
     constexpr int middle = N / 2;
     constexpr bool even = (N % 2) == 0;
@@ -47,8 +48,8 @@ __device__ __forceinline__ cplx<R> mode_op(const XOp<R>& op, cplx<R> a, cplx<R> 
         const int kx = kfreq(x, N), ky = kfreq(y, N);
         const int k2 = kx * kx + ky * ky + kz * kz;   // <= 3 (N/2)^2 < 2^24
         const int bin = isqrt24(k2);
-        double g = 0.0;
-        if (bin >= 1 && bin <= op.nb) g = op.w[bin - 1] * op.unit / (double)op.n3[bin];
+        // the stored spectrum is window-corrected on the independent modes and raw elsewhere
+        const double g = gbin[bin];
         const double c = op.win[x] * op.win[y] * op.win[kz];
         bool ind = true;
         if (kz == 0 || (kz == middle && even)) {
@@ -141,8 +142,13 @@ __global__ __launch_bounds__(T) void k_cols_op(XArgs<R> A) {
     constexpr int W = N / 2 + 1;
     __shared__ cplx<R> s[N * NL];
     __shared__ cplx<R> tw[N];
+    // 3-D bins floor(|k|): at most sqrt(3) N / 2, so N of them do
+    __shared__ double gbin[KIND == XOP_GRAD ? N : 1];
     const int tid = threadIdx.x;
     for (int i = tid; i < N; i += T) tw[i] = A.tw[i];
+    if (KIND == XOP_GRAD)
+        for (int i = tid; i < N; i += T)
+            gbin[i] = i >= 1 && i <= A.op.nb ? A.op.w[i - 1] * A.op.unit / (double)A.op.n3[i] : 0.0;
     const int l = tid % NL;
     const long long P = A.P, SP = A.SP, ncols = (long long)N * P, nblk = (ncols + NL - 1) / NL;
     const long long SEST = (long long)N * SP, EST = (long long)N * P;
@@ -176,7 +182,7 @@ __global__ __launch_bounds__(T) void k_cols_op(XArgs<R> A) {
         int y, kz;
         const bool ok = column(cb, y, kz);
         const cplx<R> none = mk<R>(0, 0);
-        auto op = [&](int k, cplx<R> v, cplx<R> f) { return ok ? mode_op<R, N, KIND>(A.op, v, f, k, y, kz) : v; };
+        auto op = [&](int k, cplx<R> v, cplx<R> f) { return ok ? mode_op<R, N, KIND>(A.op, v, f, gbin, k, y, kz) : v; };
         const cplx<R>* fp = KIND == XOP_FILTER ? A.op.filt + (ok ? (long long)y * A.op.FP + kz : 0) : nullptr;
         const long long FEST = (long long)N * A.op.FP;
         __syncthreads();   // LDS of the previous block consumed (and twiddles loaded)
@@ -254,7 +260,7 @@ template <typename R, int N, int KIND>
 static int launch_op(const XArgs<R>& a, hipStream_t st) {
     using SH = ColShape<R, N>;
     const long long nblk = ((long long)N * a.P + SH::NL - 1) / SH::NL;
-    int per_cu = (160 * 1024) / (SH::LDS + 1024);
+    int per_cu = (160 * 1024) / (SH::LDS + (KIND == XOP_GRAD ? 8 * N : 0) + 1024);
     per_cu = per_cu < 1 ? 1 : (per_cu > 8 ? 8 : per_cu);
     const long long nb = std::min<long long>((long long)cu_count() * per_cu, nblk);
     hipLaunchKernelGGL((k_cols_op<R, N, SH::NL, SH::T, KIND>), dim3((unsigned)nb), dim3(SH::T), 0, st, a);

@@ -114,13 +114,14 @@ int finalize_batch(int N, const FinArgs* tab, int nj, hipStream_t st);
 // Deposit algorithm of the fused particles -> P(k) path: cell-binned, direct atomic, or cell-binned
 // after a presort by supertile.  deposit_kind: the one `flags` forces (DEP_ATOMIC / DEP_BINNED /
 // DEP_SORTED), else the autotuner's (timing trials the first time a size class is seen, which
-// overwrite `grid`).  pk_particles: the whole fused path of one job (pyl_pk_particles).
+// overwrite `grid`).  pk_particles: the whole fused path of one job (pyl_pk_particles);
+// keep (float32 only, nullable) receives the corrected spectrum.
 enum DepositKind { DK_BINNED = 0, DK_ATOMIC = 1, DK_SORTED = 2 };
 struct Rsd;
 int deposit_kind(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, bool f64,
                  int flags, void* grid, const double* dmass, hipStream_t st, int* kind, const Rsd& rsd);
 int pk_particles(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, int axis,
-                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd);
+                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd, cplx<float>* keep = nullptr);
 
 // The whole estimator from a real (N,N,N) field: pass Z r2c (affine: delta = rho * N^3 / mass - 1
 // applied on the load, mass = dmass[0] when dmass is non-null), the column pass, the fused last pass
