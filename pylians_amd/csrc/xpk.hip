@@ -25,6 +25,7 @@ const double* pk_window_table(int N, int p);
 
 constexpr int XMAXF = 8;   // fields per call
 constexpr int XMAXC = 4;   // pairs per binning launch
+constexpr int XROUNDS = 4, XCOLS = 16;   // line of sight z: rounds of workgroups at most, columns each at least
 
 struct XBinArgs {
     const void* spec[XMAXF];
@@ -33,8 +34,9 @@ struct XBinArgs {
     int nc;
     int nf, fl[XMAXF];       // distinct fields of the launch's pairs
     int pa[XMAXC], pb[XMAXC];  // pair c = (fl[pa[c]], fl[pb[c]])
-    long long P;
-    int N, axis, last, fixk, nchunk, kmax_par, kmax_per, n1, n3, n2;
+    long long P;   // row pitch of the spectra
+    int W;         // kz < W hold data
+    int N, axis, last, fixk, nchunk, kfast, kmax_par, kmax_per, n1, n3, n2;
     double* s3;  // [nc][n3][3]
     double* s1;  // [nc][n1]
     double* s2;  // [nc][n2]
@@ -75,20 +77,26 @@ __global__ __launch_bounds__(T) void k_xbin(XBinArgs a) {
     unsigned* q2 = q1 + a.n1;
     const bool cnt = a.gc3 != nullptr;
     const int tid = threadIdx.x;
+    const int nkzb = (a.W + NL - 1) / NL;
     for (int i = tid; i < nsum; i += T) hs[i] = 0.0;
     for (int i = tid; i < a.n3 + a.n1 + wlen; i += T) q3[i] = 0u;
     __syncthreads();
     const int middle = N / 2;
     const bool even = (N % 2) == 0;
     const long long P = a.P;
-    const int nkzb = (int)((P + NL - 1) / NL);
     const long long EST = a.last == 0 ? (long long)N * P : P;
     const long long UST = a.last == 0 ? P : (long long)N * P;
     const int l = tid % NL, jrow = tid / NL;
-    const int E = (N + TPC - 1) / TPC;
+    // A thread takes consecutive pairs of rows k_j = j, -j of its column (j = 0 and N/2 alone): the two modes share
+    // |k|, k_perp, mu and the window, so one pass through the bins does for both.  The last UR threads of a column
+    // take one pair more.
+    const int EU = (N / 2 + 1) / TPC, UR = (N / 2 + 1) % TPC;
+    const int extra = jrow - (TPC - UR);
+    const int j0 = jrow * EU + (extra > 0 ? extra : 0), ne = EU + (extra >= 0 ? 1 : 0);
     int u0, u1, kzb0, kzb1;
     if (a.fixk) {
-        const int kzb = blockIdx.x / a.nchunk, ch = blockIdx.x % a.nchunk;
+        const int kzb = a.kfast ? blockIdx.x % nkzb : blockIdx.x / a.nchunk;
+        const int ch = a.kfast ? blockIdx.x / nkzb : blockIdx.x % a.nchunk;
         const int U = (N + a.nchunk - 1) / a.nchunk;
         u0 = ch * U;
         u1 = min(N, u0 + U);
@@ -111,147 +119,180 @@ __global__ __launch_bounds__(T) void k_xbin(XBinArgs a) {
         sp[f] = (const cplx<R>*)a.spec[ff];
         wp[f] = a.win[ff];
     }
-    for (int u = u0; u < u1; ++u)
-        for (int kzb = kzb0; kzb < kzb1; ++kzb) {
-            const int kz = kzb * NL + l;
-            if (kz >= P) continue;
-            const long long base = (long long)u * UST + kz;
-            const int ku = kfreq(u, N);
-            const bool zplane = (kz == 0) || (kz == middle && even);
-            // product of the window factors of the two fixed coordinates (u and kz), per field; a mode's
-            // window is this times the factor of its k_j (Pk_library.pyx:688-697, in float64, rounded
-            // once to the working precision)
-            double wuz[NF];
+    // Steps: batches of QB pairs of a column, nbat of them to a column, the columns (u, kz block) in order.  The field
+    // values and window entries of the next step load while the present one is binned: the histograms leave room for few
+    // waves a CU, which cannot hide the loads' latency (three fields of 384^3, line of sight z, 4 pairs: one row at a
+    // time, not prefetched 786 us, so 625).
+    constexpr int QB = NF <= 3 ? 4 : 2;
+    constexpr bool PRE = NF <= 4;
+    const int ncol = (u1 - u0) * (kzb1 - kzb0), nbat = (EU + 1 + QB - 1) / QB;
+    struct Step {
+        cplx<R> v[QB][2][NF];
+        double wj[QB][NF];
+    };
+    auto column = [&](int s, int& u, int& kz) {
+        const int c = s / nbat;
+        u = u0 + c / (kzb1 - kzb0);
+        kz = (kzb0 + c % (kzb1 - kzb0)) * NL + l;
+    };
+    auto load = [&](int s, Step& x) {
+        int u, kz;
+        column(s, u, kz);
+        const int q0 = (s % nbat) * QB;
+        if (q0 >= ne) return;
+        // without further conditions: padding columns and rows past the run read entries that are not used
+        const long long base = kz < a.W ? (long long)u * UST + kz : 0;
+#pragma unroll
+        for (int b = 0; b < QB; ++b) {
+            const int j = min(j0 + q0 + b, N / 2), jb = j == 0 ? 0 : N - j;
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+                if (f < nf) {
+                    x.v[b][0][f] = sp[f][base + j * EST];
+                    x.v[b][1][f] = sp[f][base + jb * EST];
+                    x.wj[b][f] = wp[f][j];
+                }
+        }
+    };
+    double wuz[NF], acc[NC][3], b1[NC], b2[NC];
+    int cur3 = -1, cur2 = -1, bin = 0, wb = 0;
+    unsigned m3 = 0u, m1 = 0u, m2 = 0u;   // modes of the current runs
+    Step nxt, now;
+    const int nstep = ncol * nbat;
+    if (PRE && nstep > 0) load(0, nxt);
+    for (int s = 0; s < nstep; ++s) {
+        if (PRE) {
+            now = nxt;
+            if (s + 1 < nstep) load(s + 1, nxt);
+        } else {
+            load(s, now);
+        }
+        int u, kz;
+        column(s, u, kz);
+        const int q0 = (s % nbat) * QB;
+        if (kz >= a.W || q0 >= ne) continue;   // no such column, or this thread's pairs of it are done
+        const int ku = kfreq(u, N);
+        const bool zplane = (kz == 0) || (kz == middle && even);
+        // |k|^2 = c0 + j^2 and k_perp^2 = cper + j^2 of a pair; their bins floor(sqrt) grow by at most one as j does
+        const int c0 = ku * ku + kz * kz;
+        const int kps = a.axis == 2 ? kz : ku;   // k_par is constant on the column
+        const int cper = c0 - kps * kps;
+        const R kps2 = (R)(kps * kps);
+        if (q0 == 0) {
+            // product of the window factors of the two fixed coordinates (u and kz), per field; a mode's window is
+            // this times the factor of its k_j (Pk_library.pyx:688-697, in float64, rounded once to the working
+            // precision)
 #pragma unroll
             for (int f = 0; f < NF; ++f)
                 if (f < nf) wuz[f] = wp[f][u] * wp[f][kz];
-            // |k|^2, k_perp^2 of the thread's first mode in the column and their bins floor(sqrt); along
-            // the run |k_j| changes by one per step (across j = N/2 too), so each bin moves by at most one
-            int bin = 0, wb = 0;
-            {
-                const int j0 = jrow * E;
-                if (j0 < N) {
-                    const int kj = kfreq(j0, N);
-                    const int kx = a.last == 0 ? kj : ku, ky = a.last == 0 ? ku : kj;
-                    bin = isqrt24(kx * kx + ky * ky + kz * kz);
-                    wb = isqrt24(a.axis == 0 ? ky * ky + kz * kz : (a.axis == 1 ? kx * kx + kz * kz : kx * kx + ky * ky));
-                }
-            }
-            int cur3 = -1, cur2 = -1;
-            unsigned m3 = 0u, m1 = 0u, m2 = 0u;   // modes of the current runs
-            double acc[NC][3], b1[NC], b2[NC];
+            bin = isqrt24(c0 + j0 * j0);
+            wb = isqrt24(cper + j0 * j0);
+            cur3 = cur2 = -1;
+            m3 = m1 = m2 = 0u;
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
                 acc[c][0] = acc[c][1] = acc[c][2] = 0.0;
                 b1[c] = b2[c] = 0.0;
             }
-            // QB modes per batch: every field value and window entry of the batch is loaded before
-            // any of them is used
-            constexpr int QB = 4;
-            for (int q0 = 0; q0 < E; q0 += QB) {
-                cplx<R> v[QB][NF];
-                double wj[QB][NF];
+        }
 #pragma unroll
-                for (int b = 0; b < QB; ++b) {
-                    const int j = jrow * E + q0 + b;
-                    const bool in = q0 + b < E && j < N;
+        for (int b = 0; b < QB; ++b) {
+            const int j = j0 + q0 + b;
+            if (q0 + b >= ne) break;
+            const int k2 = c0 + j * j, kp2 = cper + j * j;
+            bin += __mul24(bin + 1, bin + 1) <= k2 ? 1 : 0;
+            wb += __mul24(wb + 1, wb + 1) <= kp2 ? 1 : 0;
+            // the partner row N - j exists unless j = 0 or N/2 (k_j = N/2 is +N/2)
+            bool ia = true, ib = j != 0 && 2 * j != N;
+            if (zplane) {
+                const int xa = a.last == 0 ? j : ku, ya = a.last == 0 ? ku : j;
+                const int xb = a.last == 0 ? -j : ku, yb = a.last == 0 ? ku : -j;
+                ia = !(xa < 0 || ((xa == 0 || (xa == middle && even)) && ya < 0));
+                ib = ib && !(xb < 0 || ((xb == 0 || (xb == middle && even)) && yb < 0));
+                if (!ia && !ib) continue;
+            }
+            const R mu2 = k2 == 0 ? (R)0 : kps2 * recip((R)k2);
+            const R L2 = ((R)3 * mu2 - (R)1) * (R)0.5;
+            const R L4 = (((R)35 * mu2 - (R)30) * mu2 + (R)3) * (R)0.125;
+            // each field's value times its window W(x) W(y) W(z)
+            R val[2][NC];
 #pragma unroll
-                    for (int f = 0; f < NF; ++f)
-                        if (f < nf) {
-                            v[b][f] = in ? sp[f][base + j * EST] : mk<R>(0, 0);
-                            wj[b][f] = in ? wp[f][j] : 0.0;
-                        }
-                }
+            for (int h = 0; h < 2; ++h) {
+                cplx<R> w[NF];
 #pragma unroll
-                for (int b = 0; b < QB; ++b) {
-                    const int j = jrow * E + q0 + b;
-                    if (q0 + b >= E || j >= N) break;
-                    const int kj = kfreq(j, N);
-                    const int kx = a.last == 0 ? kj : ku;
-                    const int ky = a.last == 0 ? ku : kj;
-                    const int k2 = kx * kx + ky * ky + kz * kz;
-                    const int kp2 = a.axis == 0 ? ky * ky + kz * kz : (a.axis == 1 ? kx * kx + kz * kz : kx * kx + ky * ky);
-                    bin += __mul24(bin + 1, bin + 1) <= k2 ? 1 : 0;
-                    bin -= __mul24(bin, bin) > k2 ? 1 : 0;
-                    wb += __mul24(wb + 1, wb + 1) <= kp2 ? 1 : 0;
-                    wb -= __mul24(wb, wb) > kp2 ? 1 : 0;
-                    if (zplane && (kx < 0 || ((kx == 0 || (kx == middle && even)) && ky < 0))) continue;
-                    const int kps = a.axis == 0 ? kx : (a.axis == 1 ? ky : kz);
-                    const R mu2 = k2 == 0 ? (R)0 : (R)(kps * kps) * recip((R)k2);
-                    const R L2 = ((R)3 * mu2 - (R)1) * (R)0.5;
-                    const R L4 = (((R)35 * mu2 - (R)30) * mu2 + (R)3) * (R)0.125;
-                    // each field's value times its window W(x) W(y) W(z)
-                    cplx<R> w[NF];
+                for (int f = 0; f < NF; ++f)
+                    if (f < nf) w[f] = scale(now.v[b][h][f], (R)(now.wj[b][f] * wuz[f]));
 #pragma unroll
-                    for (int f = 0; f < NF; ++f)
-                        if (f < nf) w[f] = scale(v[b][f], (R)(wj[b][f] * wuz[f]));
-                    R val[NC];
+                for (int c = 0; c < NC; ++c) {
+                    cplx<R> va = w[0], vb = w[0];
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        cplx<R> va = w[0], vb = w[0];
-#pragma unroll
-                        for (int f = 1; f < NF; ++f) {
-                            if (a.pa[c] == f) va = w[f];
-                            if (a.pb[c] == f) vb = w[f];
-                        }
-                        val[c] = va.x * vb.x + va.y * vb.y;
+                    for (int f = 1; f < NF; ++f) {
+                        if (a.pa[c] == f) va = w[f];
+                        if (a.pb[c] == f) vb = w[f];
                     }
-                    if (bin != cur3) {
-                        if (cur3 >= 0) {
-#pragma unroll
-                            for (int c = 0; c < NC; ++c)
-                                for (int m = 0; m < 3; ++m) atomicAdd(&h3[(cur3 * nc + c) * 3 + m], acc[c][m]);
-                            if (cnt) atomicAdd(&q3[cur3], m3);
-                        }
-                        cur3 = bin;
-                        m3 = 0u;
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) acc[c][0] = acc[c][1] = acc[c][2] = 0.0;
-                    }
-                    ++m3;
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        acc[c][0] += (double)val[c];
-                        acc[c][1] += (double)(val[c] * L2);
-                        acc[c][2] += (double)(val[c] * L4);
-                    }
-                    if (k2 <= middle * middle) {
-                        ++m1;
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) b1[c] += (double)val[c];
-                    }
-                    const int kper = wb;
-                    const int w2 = (a.fixk ? l * nper : 0) + kper;
-                    if (w2 != cur2) {
-                        if (cur2 >= 0) {
-#pragma unroll
-                            for (int c = 0; c < NC; ++c) atomicAdd(&h2[c * wlen + cur2], b2[c]);
-                            if (cnt) atomicAdd(&q2[cur2], m2);
-                        }
-                        cur2 = w2;
-                        m2 = 0u;
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) b2[c] = 0.0;
-                    }
-                    ++m2;
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) b2[c] += (double)val[c];
+                    val[h][c] = (h == 0 ? ia : ib) ? va.x * vb.x + va.y * vb.y : (R)0;
                 }
             }
-            const int kpc = a.fixk ? kz : kpar_u;
+            const unsigned nm = (ia ? 1u : 0u) + (ib ? 1u : 0u);
+            if (bin != cur3) {
+                if (cur3 >= 0) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        for (int m = 0; m < 3; ++m) atomicAdd(&h3[(cur3 * nc + c) * 3 + m], acc[c][m]);
+                    if (cnt) atomicAdd(&q3[cur3], m3);
+                }
+                cur3 = bin;
+                m3 = 0u;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) acc[c][0] = acc[c][1] = acc[c][2] = 0.0;
+            }
+            m3 += nm;
+            // each mode's float32 products enter the float64 sums on their own
+            double both[NC];
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
-                if (cur3 >= 0)
-                    for (int m = 0; m < 3; ++m) atomicAdd(&h3[(cur3 * nc + c) * 3 + m], acc[c][m]);
-                if (cur2 >= 0) atomicAdd(&h2[c * wlen + cur2], b2[c]);
-                if (m1 != 0u) atomicAdd(&h1[c * a.n1 + kpc], b1[c]);
+                both[c] = (double)val[0][c] + (double)val[1][c];
+                acc[c][0] += both[c];
+                acc[c][1] += (double)(val[0][c] * L2) + (double)(val[1][c] * L2);
+                acc[c][2] += (double)(val[0][c] * L4) + (double)(val[1][c] * L4);
             }
-            if (cnt) {
-                if (cur3 >= 0) atomicAdd(&q3[cur3], m3);
-                if (cur2 >= 0) atomicAdd(&q2[cur2], m2);
-                if (m1 != 0u) atomicAdd(&q1[kpc], m1);
+            if (k2 <= middle * middle) {
+                m1 += nm;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) b1[c] += both[c];
             }
+            const int kper = wb;
+            const int w2 = (a.fixk ? l * nper : 0) + kper;
+            if (w2 != cur2) {
+                if (cur2 >= 0) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c) atomicAdd(&h2[c * wlen + cur2], b2[c]);
+                    if (cnt) atomicAdd(&q2[cur2], m2);
+                }
+                cur2 = w2;
+                m2 = 0u;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) b2[c] = 0.0;
+            }
+            m2 += nm;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) b2[c] += both[c];
         }
+        if (q0 + QB < ne) continue;   // the column goes on
+        const int kpc = a.fixk ? kz : kpar_u;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            if (cur3 >= 0)
+                for (int m = 0; m < 3; ++m) atomicAdd(&h3[(cur3 * nc + c) * 3 + m], acc[c][m]);
+            if (cur2 >= 0) atomicAdd(&h2[c * wlen + cur2], b2[c]);
+            if (m1 != 0u) atomicAdd(&h1[c * a.n1 + kpc], b1[c]);
+        }
+        if (cnt) {
+            if (cur3 >= 0) atomicAdd(&q3[cur3], m3);
+            if (cur2 >= 0) atomicAdd(&q2[cur2], m2);
+            if (m1 != 0u) atomicAdd(&q1[kpc], m1);
+        }
+    }
     __syncthreads();
     if (cnt) {
         for (int i = tid; i < a.n3; i += T)
@@ -299,7 +340,9 @@ static int launch_xbin(const XBinArgs& a, int grid, size_t shm, hipStream_t st) 
     constexpr int TW = NL == 8 ? 2 * T : T;
     if (a.nf <= 2)
         launch_xbin_nc<R, NL, TW, 2>(a, grid, shm, st);
-    else if (a.nf <= 4)
+    else if (a.nf == 3)
+        launch_xbin_nc<R, NL, TW, 3>(a, grid, shm, st);
+    else if (a.nf == 4)
         launch_xbin_nc<R, NL, TW, 4>(a, grid, shm, st);
     else
         launch_xbin_nc<R, NL, T, 8>(a, grid, shm, st);
@@ -319,7 +362,7 @@ template <typename R, int NL, int T>
 static int xpk_run_k(const void* const* deltas, int F, int N, double BoxSize, int axis, const int* mas_p, double* out,
                      hipStream_t st) {
     int rc = OK;
-    const int64_t P = half_len(N);
+    const int64_t P = padded_pitch<R>(N);   // (384^3, three fields: column passes 113 -> 103 us each)
     const PkGeometry* g = pk_geometry(N, axis, &rc);
     if (rc) return rc;
     const PkDims& d = g->d;
@@ -356,6 +399,7 @@ static int xpk_run_k(const void* const* deltas, int F, int N, double BoxSize, in
         PYL_CHECK(a.win[f], E_ALLOC, "window table allocation failed");
     }
     a.P = P;
+    a.W = (int)half_len(N);
     a.N = N;
     a.axis = axis;
     a.last = pk_last_axis(axis);
@@ -372,14 +416,9 @@ static int xpk_run_k(const void* const* deltas, int F, int N, double BoxSize, in
     while (cmax > 1 && (size_t)cmax * (3 * d.n3() + d.n1() + wlen) * 8 + (size_t)(d.n3() + d.n1() + wlen) * 4 >
                            120 * 1024)
         --cmax;
-    const int nkzb = (int)((P + NL - 1) / NL);
+    const int nkzb = (a.W + NL - 1) / NL;
     a.nchunk = 1;
     int grid = N;
-    if (a.fixk) {
-        a.nchunk = (num_cus_x() * 4 + nkzb - 1) / nkzb;
-        if (a.nchunk > N) a.nchunk = N;
-        grid = nkzb * a.nchunk;
-    }
     for (int c0 = 0; c0 < C; c0 += cmax) {
         a.nc = C - c0 < cmax ? C - c0 : cmax;
         for (int c = 0; c < a.nc; ++c) {
@@ -393,6 +432,21 @@ static int xpk_run_k(const void* const* deltas, int F, int N, double BoxSize, in
         a.s2 = a.s1 + (size_t)d.n1() * a.nc;
         const size_t shm = sizeof(double) * (size_t)a.nc * (3 * d.n3() + d.n1() + wlen) +
                            sizeof(unsigned) * (size_t)(d.n3() + d.n1() + wlen);
+        if (a.fixk) {
+            // Each workgroup adds its histograms (tens of kilobytes) to the sums with global atomics when it ends, so
+            // there are as few as fill the chip: one round of those that are resident beside their histograms, or up
+            // to XROUNDS where each still has XCOLS planes u, which evens out their ends.  In one round the kz blocks
+            // of a chunk run at the same time, next to each other, and share the lines of the spectra; in several
+            // they follow one another.  Three fields of 384^3, 4 pairs: 1 round 631 us, 2 rounds 599; 2 pairs, 1 round: kz
+            // blocks adjacent 378 us, one after another 418 (at about 4 CUs' worth of workgroups 436); four fields
+            // of 256^3: 135 and 154 (228); two fields of 512^3: 1 round 1055, 4 rounds 877 and 765 (809).
+            const int res = (int)std::min<size_t>(4, std::max<size_t>(1, 160 * 1024 / (shm + 1024)));
+            const int round = std::max(1, num_cus_x() * res / nkzb);
+            a.nchunk = std::min(N, round);
+            for (int r = 2; r <= XROUNDS && N >= XCOLS * r * round; ++r) a.nchunk = r * round;
+            a.kfast = a.nchunk <= round;
+            grid = nkzb * a.nchunk;
+        }
         a.gc3 = c0 == 0 ? gcount : nullptr;
         a.gc1 = c0 == 0 ? gcount + d.n3() : nullptr;
         a.gc2 = c0 == 0 ? gcount + d.n3() + d.n1() : nullptr;
