@@ -43,11 +43,10 @@ struct JobPlan {
     int64_t P = 0;
     void* grid = nullptr;
     void* spec = nullptr;
-    double* sums_base = nullptr;
     double* part = nullptr;
     double* dmass = nullptr;
     char* dep = nullptr;
-    PkSums sums{};
+    PkCheck chk{};
     const PkGeometry* geom = nullptr;
     BinnedJob bj{};
 };
@@ -97,12 +96,6 @@ template <typename R> struct FftClass {
 template <typename R> struct BinClass {
     int N, axis;
     Table<LastBinArgs<R>> last;
-    Table<ReduceArgs> red;
-};
-
-struct FinClass {
-    int N;
-    Table<FinArgs> fin;
 };
 
 }  // namespace
@@ -116,7 +109,7 @@ struct BatchPlan {
     std::map<int, FftClass<double>> fft64;
     std::map<std::pair<int, int>, BinClass<float>> bin32;
     std::map<std::pair<int, int>, BinClass<double>> bin64;
-    std::map<int, FinClass> fin;
+    Table<ReduceArgs> red;
     Table<ZeroArgs> zero;
 };
 
@@ -136,12 +129,10 @@ static int plan_spectrum(BatchPlan* B, JobPlan& J, char*& p) {
     int rc = OK;
     J.geom = pk_geometry(N, j.axis, &rc);
     if (rc) return rc;
-    J.sums_base = (double*)p;
-    p += al256(sizeof(double) * pk_sums_doubles(J.geom->d));
-    pk_sums_carve(J.geom->d, J.sums_base, &J.sums);
+    pk_check_carve(J.geom->d, (double*)p, &J.chk);
+    p += al256(sizeof(double) * pk_check_doubles(J.geom->d));
     J.part = (double*)p;
     p += al256(sizeof(double) * last_bin_part_doubles(N, j.axis, j.prec));
-    B->zero.add(ZeroArgs{J.sums_base, sizeof(double) * pk_sums_doubles(J.geom->d)}, 0);
     const int flags = (j.flags & PYL_PK_ALL) | PK_ASYNC;
     R2cArgs<R> ra;
     ColArgs<R> ca;
@@ -152,7 +143,7 @@ static int plan_spectrum(BatchPlan* B, JobPlan& J, char*& p) {
     if (rc) return rc;
     rc = cols_job<R>((const cplx<R>*)J.spec, (cplx<R>*)J.spec, N, J.P, pk_last_axis(j.axis) == 0 ? 1 : 0, &ca, &b2);
     if (rc) return rc;
-    rc = last_bin_job<R>((const cplx<R>*)J.spec, N, J.P, j.axis, j.scheme, flags, J.sums, J.part, &la, &rd, &b3);
+    rc = last_bin_job<R>((const cplx<R>*)J.spec, J.geom, J.P, j.BoxSize, j.scheme, flags, J.chk, j.out, J.part, &la, &rd, &b3);
     if (rc) return rc;
     FftClass<R>& F = fft_map(B, (R*)nullptr)[N];
     F.N = N;
@@ -163,10 +154,7 @@ static int plan_spectrum(BatchPlan* B, JobPlan& J, char*& p) {
     C.N = N;
     C.axis = j.axis;
     C.last.add(la, b3);
-    C.red.add(rd, 0);
-    auto& Fi = B->fin[N];
-    Fi.N = N;
-    Fi.fin.add(finalize_args(J.geom, J.sums, j.BoxSize, flags, j.out), 0);
+    B->red.add(rd, pk_reduce_blocks(N));
     return OK;
 }
 
@@ -189,8 +177,7 @@ static void plan_spectrum_steps(BatchPlan* B, std::map<int, FftClass<R>>& fft,
         BinClass<R>* C = &kv.second;
         B->steps.push_back([C](hipStream_t st) {
             StageTimer t("fft_last_bin", st);
-            return last_bin_batch<R>(C->N, C->axis, C->last.dev, C->last.dstart, C->last.nj(), C->last.total(),
-                                     C->red.dev, st);
+            return last_bin_batch<R>(C->N, C->axis, C->last.dev, C->last.dstart, C->last.nj(), C->last.total(), st);
         });
     }
 }
@@ -241,7 +228,7 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
         int r = OK;
         const PkGeometry* g = pk_geometry(j.dims, j.axis, &r);
         if (r) return r;
-        bytes += al256(sizeof(double) * pk_sums_doubles(g->d)) + al256(sizeof(double) * last_bin_part_doubles(j.dims, j.axis, j.prec));
+        bytes += al256(sizeof(double) * pk_check_doubles(g->d)) + al256(sizeof(double) * last_bin_part_doubles(j.dims, j.axis, j.prec));
         bytes += j.W ? 256 : 0;
         bytes += al256(binned_job_bytes(j.n, j.dims, j.scheme, j.W != nullptr, J.kind == DK_SORTED));
     }
@@ -290,9 +277,9 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
                                   kv.second.ov.bytes() + kv.second.tile.bytes();
     for (auto& kv : B->fft32) tb += kv.second.r2c.bytes() + kv.second.cols.bytes();
     for (auto& kv : B->fft64) tb += kv.second.r2c.bytes() + kv.second.cols.bytes();
-    for (auto& kv : B->bin32) tb += kv.second.last.bytes() + kv.second.red.bytes();
-    for (auto& kv : B->bin64) tb += kv.second.last.bytes() + kv.second.red.bytes();
-    for (auto& kv : B->fin) tb += kv.second.fin.bytes();
+    for (auto& kv : B->bin32) tb += kv.second.last.bytes();
+    for (auto& kv : B->bin64) tb += kv.second.last.bytes();
+    tb += B->red.bytes();
     // the previous contents of the workspaces may still be in use by queued work
     PYL_HIP(hipStreamSynchronize(st));
     if (tb) {
@@ -325,9 +312,7 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
     auto place_bin = [&](auto& m) {
         for (auto& kv : m) {
             p = kv.second.last.place(p);
-            p = kv.second.red.place(p);
             int r = kv.second.last.upload();
-            if (!r) r = kv.second.red.upload();
             if (r) return r;
         }
         return (int)OK;
@@ -335,10 +320,8 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
     if ((rc = place_fft(B->fft32)) || (rc = place_fft(B->fft64)) || (rc = place_bin(B->bin32)) ||
         (rc = place_bin(B->bin64)))
         return rc;
-    for (auto& kv : B->fin) {
-        p = kv.second.fin.place(p);
-        if ((rc = kv.second.fin.upload())) return rc;
-    }
+    p = B->red.place(p);
+    if ((rc = B->red.upload())) return rc;
     // 5. the launch sequence
     if (B->zero.nj() > 0) {
         Table<ZeroArgs>* Z = &B->zero;
@@ -365,11 +348,11 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
     }
     plan_spectrum_steps<float>(B, B->fft32, B->bin32);
     plan_spectrum_steps<double>(B, B->fft64, B->bin64);
-    for (auto& kv : B->fin) {
-        FinClass* F = &kv.second;
-        B->steps.push_back([F](hipStream_t st) {
+    if (B->red.nj() > 0) {
+        Table<ReduceArgs>* T = &B->red;
+        B->steps.push_back([T](hipStream_t st) {
             StageTimer t("finalize", st);
-            return finalize_batch(F->N, F->fin.dev, F->fin.nj(), st);
+            return pk_reduce_batch(T->dev, T->dstart, T->nj(), T->total(), st);
         });
     }
     // jobs outside the classes: the single-job path, in order

@@ -132,34 +132,22 @@ extern "C" int pyl_pk_layout(int dims, int* kmax_par, int* kmax_per, int* kmax, 
     return OK;
 }
 
-// float64 sums and mode counts live in one zeroed workspace (pk_sums_carve)
-static int pk_sums_ws(const PkDims& d, PkSums* s, hipStream_t st) {
-    int rc = OK;
-    const size_t n = pk_sums_doubles(d);
-    double* b = (double*)workspace(WS_SUMS, sizeof(double) * n, &rc);
-    if (rc) return rc;
-    rc = zero_fill(b, sizeof(double) * n, st);
-    if (rc) return rc;
-    pk_sums_carve(d, b, s);
-    return OK;
-}
-
-// check_number_modes (Pk_library.pyx:90-102) on the counts of the binning kernel: pk_finalize
-// counted the bins whose count differs from the independent-mode geometry into sums.status.
+// check_number_modes (Pk_library.pyx:90-102) on the counts of the binning kernel: pk_reduce
+// counted the bins whose count differs from the independent-mode geometry into chk.status.
 // Synchronises the stream unless PK_ASYNC is set or the stream is being captured (then the
 // counts are only in the output's Nmodes, for the caller to check).
-static int check_modes(const PkGeometry* g, const PkSums& sums, int flags, hipStream_t st) {
+static int check_modes(const PkGeometry* g, const PkCheck& chk, int flags, hipStream_t st) {
     if (flags & PK_ASYNC) return OK;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     PYL_HIP(hipStreamIsCapturing(st, &cs));
     if (cs != hipStreamCaptureStatusNone) return OK;
     unsigned bad = 0u;
-    PYL_HIP(hipMemcpyAsync(&bad, sums.status, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    PYL_HIP(hipMemcpyAsync(&bad, chk.status, sizeof(unsigned), hipMemcpyDeviceToHost, st));
     PYL_HIP(hipStreamSynchronize(st));
     if (bad == 0u) return OK;
     const PkDims& d = g->d;
     std::vector<double> c3(d.n3());
-    PYL_HIP(hipMemcpy(c3.data(), sums.c3, sizeof(double) * d.n3(), hipMemcpyDeviceToHost));
+    PYL_HIP(hipMemcpy(c3.data(), chk.c3, sizeof(double) * d.n3(), hipMemcpyDeviceToHost));
     double tot = 0.0;
     for (double v : c3) tot += v;
     const long long N = d.N;
@@ -183,9 +171,11 @@ int pk_from_delta(const R* delta, int dims, double BoxSize, int axis, int mas_p,
     if (rc) return rc;
     cplx<R>* spec = (cplx<R>*)workspace(WS_SPEC, sizeof(cplx<R>) * (size_t)dims * dims * P, &rc);
     if (rc) return rc;
-    PkSums sums;
-    rc = pk_sums_ws(g->d, &sums, st);
+    double* cb = (double*)workspace(WS_SUMS, sizeof(double) * pk_check_doubles(g->d), &rc);
     if (rc) return rc;
+    PkCheck chk;
+    pk_check_carve(g->d, cb, &chk);
+    ReduceArgs ra;
     {
         StageTimer t("fft_z_r2c", st);
         rc = fft_pass_z_r2c<R>(delta, spec, dims, P, affine, dmass, mass, st);
@@ -199,15 +189,15 @@ int pk_from_delta(const R* delta, int dims, double BoxSize, int axis, int mas_p,
     }
     {
         StageTimer t("fft_last_bin", st);
-        rc = pk_last_pass_bin<R>(spec, keep, dims, P, axis, mas_p, flags, sums, st);
+        rc = pk_last_pass_bin<R>(spec, keep, g, P, BoxSize, mas_p, flags, chk, out, &ra, st);
         if (rc) return rc;
     }
     {
         StageTimer t("finalize", st);
-        rc = pk_finalize(g, sums, BoxSize, flags, out, st);
+        rc = pk_reduce(ra, st);
         if (rc) return rc;
     }
-    return check_modes(g, sums, flags, st);
+    return check_modes(g, chk, flags, st);
 }
 template int pk_from_delta<float>(const float*, int, double, int, int, int, double*, cplx<float>*, bool, const double*,
                                   double, hipStream_t);

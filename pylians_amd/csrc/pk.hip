@@ -431,6 +431,7 @@ __device__ __forceinline__ void last_bin_body(const LastBinArgs<R>& A, Blk B) {
     }
     for (int i = tid; i < nsum; i += T) hs[i] = 0.0;
     for (int i = tid; i < n3 + n1 + n2w; i += T) c3[i] = 0u;
+    if (B.x == 0 && tid == 0) *A.status = 0u;   // counted by k_pk_reduce
     const bool drop0 = flags & PK_DROP_KZ0;
 
     const int middle = N / 2;
@@ -632,7 +633,7 @@ __device__ __forceinline__ void last_bin_body(const LastBinArgs<R>& A, Blk B) {
             atomicAdd(&c2[cur2], m2);
         }
     }
-    // this block's histograms -> its row of the partials (summed by k_bin_reduce31 / k_bin_reduce2)
+    // this block's histograms -> its row of the partials (summed by k_pk_reduce)
     __syncthreads();
     double* row = part + (long long)B.x * RS;
     const int n31 = 5 * n3 + 2 * n1;
@@ -654,87 +655,182 @@ __global__ __launch_bounds__(T) void k_last_bin_b(const LastBinArgs<R>* __restri
     last_bin_body<R, N, NL, T>(tab[bj_], blk_);
 }
 
-// Sum the per-block histogram rows of k_last_bin into the pass sums.
-// 3-D and 1-D entries (k_bin_reduce31): 64 entries per workgroup, the blocks split over the 4 waves
-// and over gridDim.y slices; each slice adds its total with one atomic.  Entries: 3-D sums, 1-D
-// sums, 3-D counts, 1-D counts.
+// Sum the per-block histogram rows of k_last_bin and normalise (Pk_library.pyx:387-421): every workgroup sums its bins
+// over all rows and writes their results, so no sums are cleared, added to or read back in memory, and one launch does
+// what took four (a clear, the 3-D and 1-D rows, the 2-D rows, the normalisation): 320^3, line of sight z (1008 rows,
+// 43 MB) 56 -> 19 us; 32^3 15 -> 4.3 us.  Bound by the latency of its few loads (with 32 threads instead of 64 a sum:
+// 27 us) and, at the first size, by reading the rows.
+// Workgroups of RT threads, in this order:
+//  * RE / 4 3-D bins (RE sums and their counts) each, then RE 1-D bins, the rows split over RT / RE threads a sum: the
+//    longest chains, so they start first;
+//  * 16 x 16 tiles of 2-D entries, (k_per, k_par) from the blocks whose window holds k_par (fixk = 0: the blocks of
+//    u = k_par and u = N - k_par, k_par = |k_u|; fixk = 1: those of kz block k_par / NL, row k_par % NL; the 2-D counts
+//    sit n2w entries after the 2-D sums of a row): four threads share an entry's rows, read with k_per fastest and
+//    written with k_par fastest, as the row and the output have them.
+// Nmodes of every histogram enabled in `flags` come from the binning kernel's counts and are
+// compared, bin by bin, with the geometry (the 3-D comparison includes the DC bin, so it contains
+// the total test of check_number_modes, Pk_library.pyx:90-102); histograms that were not binned
+// report the geometry.
+constexpr int RT = 1024;   // threads
+constexpr int RE = 16;     // sums of 3-D bins (4 a bin) or 1-D bins of a workgroup
+constexpr int R2 = 16;     // edge of a 2-D tile
 
-__device__ __forceinline__ void reduce31_body(const ReduceArgs& A) {
-    const double* __restrict__ part = A.part;
-    const int RS = A.RS, nblocks = A.nblocks, n3 = A.n3, n1 = A.n1;
-    double* __restrict__ g3 = A.g3;
-    double* __restrict__ g1 = A.g1;
-    double* __restrict__ gc3 = A.gc3;
-    double* __restrict__ gc1 = A.gc1;
-    __shared__ double red[4][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int i = blockIdx.x * 64 + lane;
-    const int n31 = 5 * n3 + 2 * n1;
-    const int step = 4 * gridDim.y;
-    double a[4] = {0.0, 0.0, 0.0, 0.0};
-    if (i < n31) {
-        int b = blockIdx.y * 4 + w, q = 0;
-        for (; b < nblocks; b += step, q = (q + 1) & 3) a[q] += part[(long long)b * RS + i];
-    }
-    red[w][lane] = (a[0] + a[1]) + (a[2] + a[3]);
-    __syncthreads();
-    if (w == 0 && i < n31) {
-        const double t = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
-        double* dst = i < 4 * n3 ? &g3[i]
-                      : i < 4 * n3 + n1 ? &g1[i - 4 * n3]
-                      : i < 5 * n3 + n1 ? &gc3[i - 4 * n3 - n1]
-                                        : &gc1[i - 5 * n3 - n1];
-        if (t != 0.0) atomicAdd(dst, t);
-    }
-}
-__global__ __launch_bounds__(256) void k_bin_reduce31(ReduceArgs a) { reduce31_body(a); }
-// batched: job blockIdx.z
-__global__ __launch_bounds__(256) void k_bin_reduce31_b(const ReduceArgs* __restrict__ tab) {
-    const ReduceArgs& a = tab[blockIdx.z];
-    reduce31_body(a);
+static unsigned reduce_blocks(const PkDims& d) {
+    const unsigned tiles = (unsigned)((d.kmax_par + R2) / R2) * (unsigned)((d.kmax_per + R2) / R2);
+    return tiles + (unsigned)((4 * d.n3() + RE - 1) / RE + (d.n1() + RE - 1) / RE);
 }
 
-// 2-D entries (k_bin_reduce2): (k_per, k_par) comes from the blocks whose window holds k_par:
-// fixk = 0, the blocks of u = k_par and u = N - k_par (k_par = |k_u|); fixk = 1, the blocks of kz
-// block k_par / NL, row k_par % NL.
-// The 2-D counts sit n2w entries after the 2-D sums of a row.
-__device__ __forceinline__ void reduce2_body(const ReduceArgs& A) {
+__device__ __forceinline__ double pk_unit(int N, double BoxSize) {
+#pragma clang fp contract(off)
+    return (BoxSize / ((double)N * N)) * (BoxSize / ((double)N * N)) * (BoxSize / ((double)N * N));
+}
+
+// The three normalisations evaluate as written (no fused multiply-add), as the reference's Python arithmetic does:
+// the last 1-D bin needs kN^2 - k^2 == 0 exactly.  Each returns 1 where the count is not the geometry's.
+__device__ __forceinline__ unsigned finish_3d(const ReduceArgs& A, int i, const double* s, double n) {
+#pragma clang fp contract(off)
+    const unsigned bad = n != (double)A.n3c[i] ? 1u : 0u;
+    A.c3[i] = n;
+    if (i == 0) return bad;   // DC: counted and checked, not reported (Pk_library.pyx:412)
+    const double kF = 2.0 * M_PI / A.BoxSize, unit = pk_unit(A.N, A.BoxSize);
+    double* o = A.out + (i - 1);
+    const int kmax = A.n3 - 1;
+    o[0] = (A.k3s[i] / n) * kF;
+    o[kmax] = (s[0] / n) * unit;
+    o[2 * kmax] = (s[1] * 5.0 / n) * unit;
+    o[3 * kmax] = (s[2] * 9.0 / n) * unit;
+    o[4 * kmax] = (s[3] / n) * unit;
+    o[5 * kmax] = n;
+    return bad;
+}
+
+__device__ __forceinline__ unsigned finish_1d(const ReduceArgs& A, int i, double s, double n) {
+#pragma clang fp contract(off)
+    const bool do1 = A.flags & PK_1D;
+    if (!do1) n = (double)A.n1c[i];
+    const unsigned bad = n != (double)A.n1c[i] ? 1u : 0u;
+    if (i == 0) return bad;
+    const double kF = 2.0 * M_PI / A.BoxSize, unit = pk_unit(A.N, A.BoxSize);
+    const double kN = (A.N / 2) * kF;
+    const double k = ((double)i * n / n) * kF;
+    const double kmaxper = sqrt(kN * kN - k * k);
+    double* o = A.out + 6 * (A.n3 - 1) + (i - 1);
+    o[0] = k;
+    o[A.kmax_par] = s * unit * (M_PI * kmaxper * kmaxper / n) / ((2.0 * M_PI) * (2.0 * M_PI));
+    o[2 * A.kmax_par] = n;
+    return bad;
+}
+
+__device__ __forceinline__ unsigned finish_2d(const ReduceArgs& A, int kp, int kq, double s, double n) {
+#pragma clang fp contract(off)
+    const int n2 = (A.kmax_par + 1) * A.nper, i = (A.kmax_par + 1) * kq + kp;
+    if (!(A.flags & PK_2D)) n = (double)A.n2c[i];
+    const unsigned bad = n != (double)A.n2c[i] ? 1u : 0u;
+    const double kF = 2.0 * M_PI / A.BoxSize, unit = pk_unit(A.N, A.BoxSize);
+    double* o = A.out + 6 * (A.n3 - 1) + 3 * A.kmax_par + i;
+    o[0] = 0.5 * (kp + kp + 1) * kF;
+    o[n2] = 0.5 * (kq + kq + 1) * kF;
+    o[2 * (long long)n2] = s * unit / n;
+    o[3 * (long long)n2] = n;
+    return bad;
+}
+
+__device__ __forceinline__ void reduce_body(const ReduceArgs& A, Blk B) {
+    __shared__ double sa[4][R2 * (R2 + 1)], sm[4][R2 * (R2 + 1)];
     const double* __restrict__ part = A.part;
-    const int RS = A.RS, nblocks = A.nblocks, n31 = 5 * A.n3 + 2 * A.n1, n2w = A.n2w, nper = A.nper;
-    const int kmax_par = A.kmax_par, fixk = A.fixk, nchunk = A.nchunk, NL = A.NL, N = A.N;
-    double* __restrict__ g2 = A.g2;
-    double* __restrict__ gc2 = A.gc2;
-    const long long i2 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i2 >= (long long)(kmax_par + 1) * nper) return;
-    const int kpar = (int)(i2 % (kmax_par + 1)), kper = (int)(i2 / (kmax_par + 1));
-    double a = 0.0, m = 0.0;
-    if (fixk) {
-        const int kzb = kpar / NL, r = kpar % NL;
-        for (int c = 0; c < nchunk; ++c) {
-            const long long b = (long long)kzb * nchunk + c;
-            if (b < nblocks) {
-                a += part[b * RS + n31 + r * nper + kper];
-                m += part[b * RS + n31 + n2w + r * nper + kper];
+    const int tid = threadIdx.x, n31 = 5 * A.n3 + 2 * A.n1, nchunk = A.nchunk;
+    const int nb3 = (4 * A.n3 + RE - 1) / RE, nb1 = (A.n1 + RE - 1) / RE;
+    unsigned bad = 0u;
+    if ((int)B.x >= nb3 + nb1) {
+        const int tp = (A.kmax_par + R2) / R2, tile = (int)B.x - nb3 - nb1;
+        const int kp0 = (tile % tp) * R2, kq0 = (tile / tp) * R2;
+        const int t = tid & 255, g = tid >> 8;
+        const int kq = kq0 + (t & 15), kp = kp0 + (t >> 4);
+        double a = 0.0, m = 0.0;
+        if ((A.flags & PK_2D) && kp <= A.kmax_par && kq < A.nper) {
+            const bool two = !A.fixk && kp > 0 && A.N - kp > A.N / 2;   // rows of -k_u too
+            const int E = two ? 2 * nchunk : nchunk;
+            const long long b0 = (long long)(A.fixk ? kp / A.NL : kp) * nchunk;
+            const long long b1 = (long long)(A.N - kp) * nchunk - nchunk;
+            const double* p = part + n31 + (A.fixk ? (kp % A.NL) * A.nper : 0) + kq;
+#pragma unroll 4
+            for (int e = g; e < E; e += 4) {
+                const double* q = p + ((e < nchunk ? b0 : b1) + e) * A.RS;
+                a += q[0];
+                m += q[A.n2w];
             }
         }
+        const int w = (t >> 4) * (R2 + 1) + (t & 15);
+        sa[g][w] = a;
+        sm[g][w] = m;
+        __syncthreads();
+        if (tid < 256) {
+            const int kpl = tid & 15, kql = tid >> 4, r = kpl * (R2 + 1) + kql;
+            if (kp0 + kpl <= A.kmax_par && kq0 + kql < A.nper)
+                bad = finish_2d(A, kp0 + kpl, kq0 + kql, (sa[0][r] + sa[1][r]) + (sa[2][r] + sa[3][r]),
+                                (sm[0][r] + sm[1][r]) + (sm[2][r] + sm[3][r]));
+        }
     } else {
-        const int us[2] = {kpar, N - kpar};
-        const int nu = (kpar > 0 && N - kpar != kpar && N - kpar > N / 2) ? 2 : 1;
-        for (int q = 0; q < nu; ++q)
-            for (int c = 0; c < nchunk; ++c) {
-                const long long b = (long long)us[q] * nchunk + c;
-                a += part[b * RS + n31 + kper];
-                m += part[b * RS + n31 + n2w + kper];
+        const int b3 = (int)B.x, b1 = b3 - nb3;
+        const bool is3 = b3 < nb3;
+        const int e = tid % RE;
+        constexpr int ROWS = RT / RE;
+        // row entries: 3-D sums (4 n3) | 1-D sums (n1) | 3-D counts (n3) | 1-D counts (n1)
+        const int s = is3 ? RE * b3 + e : 4 * A.n3 + RE * b1 + e;
+        const bool ins = s < (is3 ? 4 * A.n3 : 4 * A.n3 + A.n1);
+        const int c = is3 ? 4 * A.n3 + A.n1 + RE / 4 * b3 + e : 5 * A.n3 + A.n1 + RE * b1 + e;
+        const bool inc = is3 ? e < RE / 4 && c < 5 * A.n3 + A.n1 : c < n31;
+        double a[4] = {0.0, 0.0, 0.0, 0.0}, m[4] = {0.0, 0.0, 0.0, 0.0};
+        if (is3 || (A.flags & PK_1D)) {
+            int b = tid / RE;
+            for (; b + 3 * ROWS < A.nblocks; b += 4 * ROWS)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const double* row = part + (long long)(b + ROWS * q) * A.RS;
+                    if (ins) a[q] += row[s];
+                    if (inc) m[q] += row[c];
+                }
+            for (; b < A.nblocks; b += ROWS) {
+                const double* row = part + (long long)b * A.RS;
+                if (ins) a[0] += row[s];
+                if (inc) m[0] += row[c];
             }
+        }
+        double ta = (a[0] + a[1]) + (a[2] + a[3]), tm = (m[0] + m[1]) + (m[2] + m[3]);
+#pragma unroll
+        for (int d = RE; d < 64; d *= 2) {
+            ta += __shfl_xor(ta, d);
+            tm += __shfl_xor(tm, d);
+        }
+        double* const pa = &sa[0][0];   // [16 waves][RE + 1]
+        double* const pm = &sm[0][0];
+        if ((tid & 63) < RE) {
+            pa[(tid >> 6) * (RE + 1) + e] = ta;
+            pm[(tid >> 6) * (RE + 1) + e] = tm;
+        }
+        __syncthreads();
+        if (tid < 2 * RE) {
+            double* const q = tid < RE ? pa : pm;
+            double t = 0.0;
+            for (int w = 0; w < RT / 64; ++w) t += q[w * (RE + 1) + e];
+            q[e] = t;
+        }
+        __syncthreads();
+        if (is3) {
+            const int i = RE / 4 * b3 + tid;
+            if (tid < RE / 4 && i < A.n3) bad = finish_3d(A, i, &pa[4 * tid], pm[tid]);
+        } else {
+            const int i = RE * b1 + tid;
+            if (tid < RE && i < A.n1) bad = finish_1d(A, i, pa[tid], pm[tid]);
+        }
     }
-    if (a != 0.0) g2[i2] += a;
-    if (m != 0.0) gc2[i2] += m;
+    if (bad) atomicAdd(A.status, bad);
 }
-__global__ void k_bin_reduce2(ReduceArgs a) { reduce2_body(a); }
-// batched: job blockIdx.y
-__global__ void k_bin_reduce2_b(const ReduceArgs* __restrict__ tab) {
-    const ReduceArgs& a = tab[blockIdx.y];
-    reduce2_body(a);
+__global__ __launch_bounds__(RT) void k_pk_reduce(ReduceArgs a) { reduce_body(a, own_blk()); }
+__global__ __launch_bounds__(RT) void k_pk_reduce_b(const ReduceArgs* __restrict__ tab,
+                                                    const unsigned* __restrict__ start, int nj) {
+    PYL_BATCH_BLK(start, nj);
+    reduce_body(tab[bj_], blk_);
 }
 
 static int num_cus() {
@@ -757,8 +853,7 @@ template <typename R, int N, bool FIXK> struct BinShape {
     static constexpr int NL = nl_bin<R, N, FIXK>();
     static constexpr int T = threads_bin<R, N, FIXK>();
     static constexpr int W = N / 2 + 1;   // kz = 0 .. N/2; rows of the spectrum may be padded to P >= W
-    int nchunk, grid, n2w, RS, n31;
-    long long n2;
+    int nchunk, grid, n2w, RS;
     size_t shm;
     PkDims d;
     BinShape() {
@@ -775,73 +870,61 @@ template <typename R, int N, bool FIXK> struct BinShape {
         const int nper = d.kmax_per + 1;
         n2w = (FIXK ? NL : 1) * nper;
         RS = 5 * d.n3() + 2 * d.n1() + 2 * n2w;
-        n31 = 5 * d.n3() + 2 * d.n1();
-        n2 = (long long)(d.kmax_par + 1) * nper;
         // LDS: float64 sums (4 n3 + n1 + n2w), then 32-bit counts (n3 + n1 + n2w)
         shm = sizeof(double) * (size_t)(4 * d.n3() + d.n1() + n2w) + sizeof(unsigned) * (size_t)(d.n3() + d.n1() + n2w);
     }
-    int slices() const { return std::max(1, std::min(16, grid / 32)); }
 };
 
 template <typename R, int N, bool FIXK>
-static int last_bin_job_k(const cplx<R>* spec, cplx<R>* keep, int64_t P, int axis, int p, int flags,
-                          const PkSums& sums, double* part, LastBinArgs<R>* la, ReduceArgs* ra, unsigned* blocks) {
+static int last_bin_job_k(const cplx<R>* spec, cplx<R>* keep, int64_t P, const PkGeometry* g, double BoxSize, int p,
+                          int flags, const PkCheck& chk, double* out, double* part, LastBinArgs<R>* la, ReduceArgs* ra,
+                          unsigned* blocks) {
     const BinShape<R, N, FIXK> sh;
     const cplx<R>* tw = twiddles<R>(N);
     const double* win = window_table(N, p);
     PYL_CHECK(tw && win, E_ALLOC, "table allocation failed");
     const PkDims& d = sh.d;
     const int fixk = FIXK ? 1 : 0;
-    *la = LastBinArgs<R>{spec, keep, (long long)P, sh.W, pk_last_axis(axis), axis, fixk, sh.nchunk, flags,
-                         d.kmax_par, d.kmax_per, d.n1(), d.n3(), win, tw, part, sh.RS};
+    *la = LastBinArgs<R>{spec, keep, (long long)P, sh.W, pk_last_axis(g->axis), g->axis, fixk, sh.nchunk, flags,
+                         d.kmax_par, d.kmax_per, d.n1(), d.n3(), win, tw, part, sh.RS, chk.status};
     *ra = ReduceArgs{part, sh.RS, sh.grid, d.n3(), d.n1(), sh.n2w, d.kmax_per + 1, d.kmax_par, fixk, sh.nchunk,
-                     sh.NL, N, sums.s3, sums.s1, sums.c3, sums.c1, sums.s2, sums.c2};
+                     sh.NL, N, flags, BoxSize, g->n1, g->n2, g->n3, g->k3sum, chk.c3, chk.status, out};
     *blocks = (unsigned)sh.grid;
     return OK;
 }
 
 template <typename R, int N, bool FIXK>
-static int launch_last_bin_k(const cplx<R>* spec, cplx<R>* keep, int64_t P, int axis, int p, int flags,
-                             const PkSums& sums, hipStream_t st) {
+static int launch_last_bin_k(const cplx<R>* spec, cplx<R>* keep, int64_t P, const PkGeometry* g, double BoxSize, int p,
+                             int flags, const PkCheck& chk, double* out, ReduceArgs* ra, hipStream_t st) {
     const BinShape<R, N, FIXK> sh;
     int rc = OK;
     double* part = (double*)workspace(WS_PART, sizeof(double) * (size_t)sh.grid * sh.RS, &rc);
     if (rc) return rc;
     LastBinArgs<R> la;
-    ReduceArgs ra;
     unsigned grid = 0;
-    rc = last_bin_job_k<R, N, FIXK>(spec, keep, P, axis, p, flags, sums, part, &la, &ra, &grid);
+    rc = last_bin_job_k<R, N, FIXK>(spec, keep, P, g, BoxSize, p, flags, chk, out, part, &la, ra, &grid);
     if (rc) return rc;
     hipLaunchKernelGGL((k_last_bin<R, N, sh.NL, sh.T>), dim3(grid), dim3(sh.T), sh.shm, st, la);
-    PYL_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_bin_reduce31, dim3((unsigned)((sh.n31 + 63) / 64), (unsigned)sh.slices()), dim3(256), 0, st,
-                       ra);
-    PYL_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_bin_reduce2, dim3((unsigned)((sh.n2 + 255) / 256)), dim3(256), 0, st, ra);
     PYL_HIP(hipGetLastError());
     return OK;
 }
 
 template <typename R, int N, bool FIXK>
 static int launch_last_bin_batch_k(const LastBinArgs<R>* tab, const unsigned* start, int nj, unsigned total,
-                                   const ReduceArgs* rtab, hipStream_t st) {
+                                   hipStream_t st) {
     const BinShape<R, N, FIXK> sh;
     hipLaunchKernelGGL((k_last_bin_b<R, N, sh.NL, sh.T>), dim3(total), dim3(sh.T), sh.shm, st, tab, start, nj);
-    PYL_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_bin_reduce31_b, dim3((unsigned)((sh.n31 + 63) / 64), (unsigned)sh.slices(), (unsigned)nj),
-                       dim3(256), 0, st, rtab);
-    PYL_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_bin_reduce2_b, dim3((unsigned)((sh.n2 + 255) / 256), (unsigned)nj), dim3(256), 0, st, rtab);
     PYL_HIP(hipGetLastError());
     return OK;
 }
 
 // blocks own one kz block (fixk) when the line of sight is z, else one u: separate LDS budgets
 template <typename R, int N>
-static int launch_last_bin(const cplx<R>* spec, cplx<R>* keep, int64_t P, int axis, int p, int flags,
-                           const PkSums& sums, hipStream_t st) {
-    return axis == 2 ? launch_last_bin_k<R, N, true>(spec, keep, P, axis, p, flags, sums, st)
-                     : launch_last_bin_k<R, N, false>(spec, keep, P, axis, p, flags, sums, st);
+static int launch_last_bin(const cplx<R>* spec, cplx<R>* keep, int64_t P, const PkGeometry* g, double BoxSize, int p,
+                           int flags, const PkCheck& chk, double* out, ReduceArgs* ra, hipStream_t st) {
+    return g->axis == 2
+               ? launch_last_bin_k<R, N, true>(spec, keep, P, g, BoxSize, p, flags, chk, out, ra, st)
+               : launch_last_bin_k<R, N, false>(spec, keep, P, g, BoxSize, p, flags, chk, out, ra, st);
 }
 
 #define PYL_PK_SIZES(X) \
@@ -849,23 +932,23 @@ static int launch_last_bin(const cplx<R>* spec, cplx<R>* keep, int64_t P, int ax
     X(320) X(384) X(512) X(640) X(768) X(1024)
 
 template <typename R>
-int pk_last_pass_bin(const cplx<R>* spec, cplx<R>* keep, int N, int64_t P, int axis, int mas_p, int flags,
-                     const PkSums& sums, hipStream_t st) {
-    switch (N) {
+int pk_last_pass_bin(const cplx<R>* spec, cplx<R>* keep, const PkGeometry* g, int64_t P, double BoxSize, int mas_p,
+                     int flags, const PkCheck& chk, double* out, ReduceArgs* ra, hipStream_t st) {
+    switch (g->d.N) {
 #define PYL_CASE(n) \
     case n:         \
-        return launch_last_bin<R, n>(spec, keep, P, axis, mas_p, flags, sums, st);
+        return launch_last_bin<R, n>(spec, keep, P, g, BoxSize, mas_p, flags, chk, out, ra, st);
         PYL_PK_SIZES(PYL_CASE)
 #undef PYL_CASE
         default:
-            set_error("grid size %d not supported", N);
+            set_error("grid size %d not supported", g->d.N);
             return E_UNSUPPORTED;
     }
 }
-template int pk_last_pass_bin<float>(const cplx<float>*, cplx<float>*, int, int64_t, int, int, int, const PkSums&,
-                                     hipStream_t);
-template int pk_last_pass_bin<double>(const cplx<double>*, cplx<double>*, int, int64_t, int, int, int, const PkSums&,
-                                      hipStream_t);
+template int pk_last_pass_bin<float>(const cplx<float>*, cplx<float>*, const PkGeometry*, int64_t, double, int, int,
+                                     const PkCheck&, double*, ReduceArgs*, hipStream_t);
+template int pk_last_pass_bin<double>(const cplx<double>*, cplx<double>*, const PkGeometry*, int64_t, double, int, int,
+                                      const PkCheck&, double*, ReduceArgs*, hipStream_t);
 
 size_t last_bin_part_doubles(int N, int axis, int prec) {
     switch (N) {
@@ -884,29 +967,32 @@ size_t last_bin_part_doubles(int N, int axis, int prec) {
 }
 
 template <typename R>
-int last_bin_job(const cplx<R>* spec, int N, int64_t P, int axis, int mas_p, int flags, const PkSums& sums,
-                 double* part, LastBinArgs<R>* a, ReduceArgs* r, unsigned* blocks) {
-    switch (N) {
-#define PYL_CASE(n)                                                                                      \
-    case n:                                                                                              \
-        return axis == 2 ? last_bin_job_k<R, n, true>(spec, nullptr, P, axis, mas_p, flags, sums, part, a, r, blocks) \
-                         : last_bin_job_k<R, n, false>(spec, nullptr, P, axis, mas_p, flags, sums, part, a, r, blocks);
+int last_bin_job(const cplx<R>* spec, const PkGeometry* g, int64_t P, double BoxSize, int mas_p, int flags,
+                 const PkCheck& chk, double* out, double* part, LastBinArgs<R>* a, ReduceArgs* r, unsigned* blocks) {
+    switch (g->d.N) {
+#define PYL_CASE(n)                                                                                                   \
+    case n:                                                                                                           \
+        return g->axis == 2                                                                                           \
+                   ? last_bin_job_k<R, n, true>(spec, nullptr, P, g, BoxSize, mas_p, flags, chk, out, part, a, r,     \
+                                                blocks)                                                               \
+                   : last_bin_job_k<R, n, false>(spec, nullptr, P, g, BoxSize, mas_p, flags, chk, out, part, a, r,    \
+                                                 blocks);
         PYL_PK_SIZES(PYL_CASE)
 #undef PYL_CASE
         default:
-            set_error("grid size %d not supported", N);
+            set_error("grid size %d not supported", g->d.N);
             return E_UNSUPPORTED;
     }
 }
 
 template <typename R>
 int last_bin_batch(int N, int axis, const LastBinArgs<R>* tab, const unsigned* start, int nj, unsigned total,
-                   const ReduceArgs* rtab, hipStream_t st) {
+                   hipStream_t st) {
     switch (N) {
 #define PYL_CASE(n)                                                                                      \
     case n:                                                                                              \
-        return axis == 2 ? launch_last_bin_batch_k<R, n, true>(tab, start, nj, total, rtab, st)         \
-                         : launch_last_bin_batch_k<R, n, false>(tab, start, nj, total, rtab, st);
+        return axis == 2 ? launch_last_bin_batch_k<R, n, true>(tab, start, nj, total, st)               \
+                         : launch_last_bin_batch_k<R, n, false>(tab, start, nj, total, st);
         PYL_PK_SIZES(PYL_CASE)
 #undef PYL_CASE
         default:
@@ -914,132 +1000,30 @@ int last_bin_batch(int N, int axis, const LastBinArgs<R>* tab, const unsigned* s
             return E_UNSUPPORTED;
     }
 }
-template int last_bin_job<float>(const cplx<float>*, int, int64_t, int, int, int, const PkSums&, double*,
-                                 LastBinArgs<float>*, ReduceArgs*, unsigned*);
-template int last_bin_job<double>(const cplx<double>*, int, int64_t, int, int, int, const PkSums&, double*,
-                                  LastBinArgs<double>*, ReduceArgs*, unsigned*);
-template int last_bin_batch<float>(int, int, const LastBinArgs<float>*, const unsigned*, int, unsigned,
-                                   const ReduceArgs*, hipStream_t);
-template int last_bin_batch<double>(int, int, const LastBinArgs<double>*, const unsigned*, int, unsigned,
-                                    const ReduceArgs*, hipStream_t);
+template int last_bin_job<float>(const cplx<float>*, const PkGeometry*, int64_t, double, int, int, const PkCheck&,
+                                 double*, double*, LastBinArgs<float>*, ReduceArgs*, unsigned*);
+template int last_bin_job<double>(const cplx<double>*, const PkGeometry*, int64_t, double, int, int, const PkCheck&,
+                                  double*, double*, LastBinArgs<double>*, ReduceArgs*, unsigned*);
+template int last_bin_batch<float>(int, int, const LastBinArgs<float>*, const unsigned*, int, unsigned, hipStream_t);
+template int last_bin_batch<double>(int, int, const LastBinArgs<double>*, const unsigned*, int, unsigned, hipStream_t);
 
-// ------------------------------------------------------------------ finalize
-size_t pk_sums_doubles(const PkDims& d) { return 5 * (size_t)d.n3() + 2 * (size_t)d.n1() + 2 * (size_t)d.n2() + 1; }
+size_t pk_check_doubles(const PkDims& d) { return (size_t)d.n3() + 1; }
 
-void pk_sums_carve(const PkDims& d, double* b, PkSums* s) {
-    s->s3 = b;
-    s->s1 = s->s3 + 4 * d.n3();
-    s->s2 = s->s1 + d.n1();
-    s->c3 = s->s2 + d.n2();
-    s->c1 = s->c3 + d.n3();
-    s->c2 = s->c1 + d.n1();
-    s->status = (unsigned*)(s->c2 + d.n2());
+void pk_check_carve(const PkDims& d, double* b, PkCheck* c) {
+    c->c3 = b;
+    c->status = (unsigned*)(b + d.n3());
 }
 
-// Nmodes of every histogram enabled in `flags` come from the binning kernel's counts and are
-// compared, bin by bin, with the geometry (the 3-D comparison includes the DC bin, so it contains
-// the total test of check_number_modes, Pk_library.pyx:90-102); histograms that were not binned
-// report the geometry.
+unsigned pk_reduce_blocks(int N) { return reduce_blocks(pk_dims(N, half_len(N))); }
 
-__device__ __forceinline__ void finalize_body(const FinArgs& A, Blk B) {
-    // evaluate as written (no fused multiply-add), as the reference's Python arithmetic does:
-    // the last 1-D bin needs kN^2 - k^2 == 0 exactly
-#pragma clang fp contract(off)
-    const int N = A.N, kmax = A.kmax, kmax_par = A.kmax_par, n2 = A.n2, flags = A.flags;
-    const double BoxSize = A.BoxSize;
-    const unsigned long long* __restrict__ n1c = A.n1c;
-    const unsigned long long* __restrict__ n2c = A.n2c;
-    const unsigned long long* __restrict__ n3c = A.n3c;
-    const double* __restrict__ k3s = A.k3s;
-    const double* __restrict__ s3 = A.s3;
-    const double* __restrict__ s1 = A.s1;
-    const double* __restrict__ s2 = A.s2;
-    const double* __restrict__ c3 = A.c3;
-    const double* __restrict__ c1 = A.c1;
-    const double* __restrict__ c2 = A.c2;
-    unsigned* __restrict__ status = A.status;
-    double* __restrict__ out = A.out;
-    const double kF = 2.0 * M_PI / BoxSize;
-    const int middle = N / 2;
-    const double kN = middle * kF;
-    const double unit = (BoxSize / ((double)N * N)) * (BoxSize / ((double)N * N)) * (BoxSize / ((double)N * N));
-    double* k3D = out;
-    double* P0 = k3D + kmax;
-    double* P2 = P0 + kmax;
-    double* P4 = P2 + kmax;
-    double* ph = P4 + kmax;
-    double* N3 = ph + kmax;
-    double* k1D = N3 + kmax;
-    double* P1 = k1D + kmax_par;
-    double* N1 = P1 + kmax_par;
-    double* kpar = N1 + kmax_par;
-    double* kper = kpar + n2;
-    double* P2D = kper + n2;
-    double* N2 = P2D + n2;
-    const bool do1 = flags & PK_1D, do2 = flags & PK_2D;
-    const int gi = B.x * blockDim.x + threadIdx.x, gs = B.gx * blockDim.x;
-    unsigned bad = 0u;
-    for (int i = gi; i <= kmax; i += gs) {
-        const double n = c3[i];
-        bad += n != (double)n3c[i] ? 1u : 0u;
-        if (i == 0) continue;   // DC: counted and checked, not reported (Pk_library.pyx:412)
-        const int o = i - 1;
-        k3D[o] = (k3s[i] / n) * kF;
-        P0[o] = (s3[4 * i + 0] / n) * unit;
-        P2[o] = (s3[4 * i + 1] * 5.0 / n) * unit;
-        P4[o] = (s3[4 * i + 2] * 9.0 / n) * unit;
-        ph[o] = (s3[4 * i + 3] / n) * unit;
-        N3[o] = n;
-    }
-    for (int i = gi; i <= kmax_par; i += gs) {
-        const double n = do1 ? c1[i] : (double)n1c[i];
-        if (do1) bad += n != (double)n1c[i] ? 1u : 0u;
-        if (i == 0) continue;
-        const int o = i - 1;
-        const double k = ((double)i * n / n) * kF;
-        const double kmaxper = sqrt(kN * kN - k * k);
-        k1D[o] = k;
-        P1[o] = s1[i] * unit * (M_PI * kmaxper * kmaxper / n) / ((2.0 * M_PI) * (2.0 * M_PI));
-        N1[o] = n;
-    }
-    for (int i = gi; i < n2; i += gs) {
-        const int kp = i % (kmax_par + 1), kq = i / (kmax_par + 1);
-        const double n = do2 ? c2[i] : (double)n2c[i];
-        if (do2) bad += n != (double)n2c[i] ? 1u : 0u;
-        kpar[i] = 0.5 * (kp + kp + 1) * kF;
-        kper[i] = 0.5 * (kq + kq + 1) * kF;
-        P2D[i] = s2[i] * unit / n;
-        N2[i] = n;
-    }
-    if (bad) atomicAdd(status, bad);
-}
-__global__ void k_pk_finalize(FinArgs a) { finalize_body(a, own_blk()); }
-// batched: job blockIdx.y
-__global__ void k_pk_finalize_b(const FinArgs* __restrict__ tab) {
-    const FinArgs& a = tab[blockIdx.y];
-    finalize_body(a, own_blk());
-}
-
-FinArgs finalize_args(const PkGeometry* g, const PkSums& sums, double BoxSize, int flags, double* out) {
-    const PkDims& d = g->d;
-    return FinArgs{d.N, d.kmax, d.kmax_par, d.n2(), BoxSize, flags, g->n1, g->n2, g->n3, g->k3sum, sums.s3, sums.s1,
-                   sums.s2, sums.c3, sums.c1, sums.c2, sums.status, out};
-}
-
-static unsigned finalize_blocks(int N) {
-    const PkDims d = pk_dims(N, half_len(N));
-    return (unsigned)((std::max(d.kmax + 1, d.n2()) + 255) / 256);
-}
-
-int finalize_batch(int N, const FinArgs* tab, int nj, hipStream_t st) {
-    hipLaunchKernelGGL(k_pk_finalize_b, dim3(finalize_blocks(N), (unsigned)nj), dim3(256), 0, st, tab);
+int pk_reduce_batch(const ReduceArgs* tab, const unsigned* start, int nj, unsigned total, hipStream_t st) {
+    hipLaunchKernelGGL(k_pk_reduce_b, dim3(total), dim3(RT), 0, st, tab, start, nj);
     PYL_HIP(hipGetLastError());
     return OK;
 }
 
-int pk_finalize(const PkGeometry* g, const PkSums& sums, double BoxSize, int flags, double* out, hipStream_t st) {
-    const FinArgs fa = finalize_args(g, sums, BoxSize, flags, out);
-    hipLaunchKernelGGL(k_pk_finalize, dim3(finalize_blocks(g->d.N)), dim3(256), 0, st, fa);
+int pk_reduce(const ReduceArgs& ra, hipStream_t st) {
+    hipLaunchKernelGGL(k_pk_reduce, dim3(pk_reduce_blocks(ra.N)), dim3(RT), 0, st, ra);
     PYL_HIP(hipGetLastError());
     return OK;
 }

@@ -30,45 +30,21 @@ struct PkGeometry {
 };
 const PkGeometry* pk_geometry(int N, int axis, int* rc);
 
-// float64 per-bin sums of the data-dependent quantities and the mode counts of the binning
-// kernel (integers held in float64, exact below 2^53), device arrays owned by caller
-struct PkSums {
-    double* s3;   // n3 * 4: sum d2, sum d2 L2(mu), sum d2 L4(mu), sum phase^2
-    double* s1;   // n1: sum d2 over modes with |k| <= N/2, binned by |k_par|
-    double* s2;   // n2: sum d2 over 2-D bins (kmax_par+1)*k_per + k_par
-    double* c3;   // n3: modes binned per 3-D bin
-    double* c1;   // n1: modes binned per 1-D bin
-    double* c2;   // n2: modes binned per 2-D bin
-    unsigned* status;   // [1]: bins whose count differs from the mode geometry (set by pk_finalize)
+// The mode check's part of a call's results, device arrays owned by the caller (pk_check_doubles doubles)
+struct PkCheck {
+    double* c3;         // n3: modes binned per 3-D bin
+    unsigned* status;   // [1]: bins whose count differs from the mode geometry
 };
-size_t pk_sums_doubles(const PkDims& d);   // doubles of one PkSums block (status word included)
-void pk_sums_carve(const PkDims& d, double* base, PkSums* s);
+size_t pk_check_doubles(const PkDims& d);
+void pk_check_carve(const PkDims& d, double* base, PkCheck* c);
 
 // PK_ASYNC: no host synchronisation for the mode check (the counts are still in the output).
 // PK_DROP_KZ0: the binning kernel leaves out the kz = 0 plane -- fault injection for the tests of
 // the mode check, never set by the library itself.
 enum PkFlags { PK_1D = 1, PK_2D = 2, PK_PHASE = 4, PK_ASYNC = 256, PK_DROP_KZ0 = 512 };
 
-// Axis of the last forward FFT pass for a line of sight `axis`: 1 (y) for axis 0, else 0 (x).
-// The half spectrum must have gone through pass Z and the column pass along the other axis.
-int pk_last_axis(int axis);
-// That last pass fused with the window deconvolution and the binning of the independent modes.
-// keep (nullable) receives the window-corrected spectrum (Pk_library.pyx:354-355, 423).
-template <typename R>
-int pk_last_pass_bin(const cplx<R>* spec, cplx<R>* keep, int N, int64_t P, int axis, int mas_p, int flags,
-                     const PkSums& sums, hipStream_t st);
-
-// Normalisation of Pk_library.pyx:387-421 on the device, with Nmodes from the binning kernel's
-// counts; every bin whose count differs from the geometry is counted into sums.status (the
-// check_number_modes test, Pk_library.pyx:90-102, made per bin).  out layout (float64):
-//   [k3D (kmax) | P0 (kmax) | P2 (kmax) | P4 (kmax) | Pkphase (kmax) | Nmodes3D (kmax) |
-//    k1D (kmax_par) | Pk1D (kmax_par) | Nmodes1D (kmax_par) |
-//    kpar (n2) | kper (n2) | Pk2D (n2) | Nmodes2D (n2)]
-size_t pk_out_len(const PkDims& d);
-int pk_finalize(const PkGeometry* g, const PkSums& sums, double BoxSize, int flags, double* out, hipStream_t st);
-
-// Argument blocks of the fused last pass + binning, of the two reductions of its per-block
-// histograms and of the normalisation (shared with the batch planner)
+// Argument blocks of the fused last pass + binning and of the reduction of its per-block histograms with the
+// normalisation (shared with the batch planner)
 template <typename R> struct LastBinArgs {
     const cplx<R>* src;
     cplx<R>* keep;
@@ -78,38 +54,52 @@ template <typename R> struct LastBinArgs {
     const cplx<R>* tw;
     double* part;
     int RS;
+    unsigned* status;   // cleared here, counted by the reduction
 };
 
 struct ReduceArgs {
     const double* part;
-    int RS, nblocks, n3, n1, n2w, nper, kmax_par, fixk, nchunk, NL, N;
-    double *g3, *g1, *gc3, *gc1, *g2, *gc2;
-};
-
-struct FinArgs {
-    int N, kmax, kmax_par, n2;
+    int RS, nblocks, n3, n1, n2w, nper, kmax_par, fixk, nchunk, NL, N, flags;
     double BoxSize;
-    int flags;
-    const unsigned long long *n1c, *n2c, *n3c;
+    const unsigned long long *n1c, *n2c, *n3c;   // the geometry
     const double* k3s;
-    const double *s3, *s1, *s2, *c3, *c1, *c2;
+    double* c3;
     unsigned* status;
     double* out;
 };
 
-// Batched last pass + binning + reductions + normalisation over jobs of one grid size N and line
-// of sight class (z or not): *_job builds a job's arguments (part: its per-block histogram rows,
-// last_bin_part_doubles(N, axis, prec) of them) and block count; last_bin_batch launches the
-// tables (block ranges start[0..nj]).
+// Axis of the last forward FFT pass for a line of sight `axis`: 1 (y) for axis 0, else 0 (x).
+// The half spectrum must have gone through pass Z and the column pass along the other axis.
+int pk_last_axis(int axis);
+// That last pass fused with the window deconvolution and the binning of the independent modes, into per-block histogram
+// rows; `ra` receives the arguments of pk_reduce, which makes the results of them.
+// keep (nullable) receives the window-corrected spectrum (Pk_library.pyx:354-355, 423).
+template <typename R>
+int pk_last_pass_bin(const cplx<R>* spec, cplx<R>* keep, const PkGeometry* g, int64_t P, double BoxSize, int mas_p,
+                     int flags, const PkCheck& chk, double* out, ReduceArgs* ra, hipStream_t st);
+
+// Sum of the rows and normalisation of Pk_library.pyx:387-421 on the device, with Nmodes from the binning kernel's
+// counts; every bin whose count differs from the geometry is counted into chk.status (the
+// check_number_modes test, Pk_library.pyx:90-102, made per bin).  out layout (float64):
+//   [k3D (kmax) | P0 (kmax) | P2 (kmax) | P4 (kmax) | Pkphase (kmax) | Nmodes3D (kmax) |
+//    k1D (kmax_par) | Pk1D (kmax_par) | Nmodes1D (kmax_par) |
+//    kpar (n2) | kper (n2) | Pk2D (n2) | Nmodes2D (n2)]
+size_t pk_out_len(const PkDims& d);
+int pk_reduce(const ReduceArgs& ra, hipStream_t st);
+
+// Batched last pass + binning over jobs of one grid size N and line of sight class (z or not), and the reduction of
+// jobs of any size: last_bin_job builds a job's arguments (part: its per-block histogram rows,
+// last_bin_part_doubles(N, axis, prec) of them) and block count, pk_reduce_blocks the blocks of its reduction; the
+// launches take tables (block ranges start[0..nj]).
 size_t last_bin_part_doubles(int N, int axis, int prec);
 template <typename R>
-int last_bin_job(const cplx<R>* spec, int N, int64_t P, int axis, int mas_p, int flags, const PkSums& sums,
-                 double* part, LastBinArgs<R>* a, ReduceArgs* r, unsigned* blocks);
+int last_bin_job(const cplx<R>* spec, const PkGeometry* g, int64_t P, double BoxSize, int mas_p, int flags,
+                 const PkCheck& chk, double* out, double* part, LastBinArgs<R>* a, ReduceArgs* r, unsigned* blocks);
 template <typename R>
 int last_bin_batch(int N, int axis, const LastBinArgs<R>* tab, const unsigned* start, int nj, unsigned total,
-                   const ReduceArgs* rtab, hipStream_t st);
-FinArgs finalize_args(const PkGeometry* g, const PkSums& sums, double BoxSize, int flags, double* out);
-int finalize_batch(int N, const FinArgs* tab, int nj, hipStream_t st);
+                   hipStream_t st);
+unsigned pk_reduce_blocks(int N);
+int pk_reduce_batch(const ReduceArgs* tab, const unsigned* start, int nj, unsigned total, hipStream_t st);
 
 // Deposit algorithm of the fused particles -> P(k) path: cell-binned, direct atomic, or cell-binned
 // after a presort by supertile.  deposit_kind: the one `flags` forces (DEP_ATOMIC / DEP_BINNED /
