@@ -8,8 +8,8 @@
 //             step are already loading), reserves room with one global atomic per distinct key and
 //             writes the records (position, and weight).  Records beyond
 //             a segment's capacity go to an overflow list.
-// 2. k_ov_*   the overflow list is grouped by tile with an exact count + scan (empty in the common
-//             case: the kernels then only read a zero counter).
+// 2. k_ov     the overflow list is grouped by tile with an exact count + scan (empty in the common
+//             case: the kernel then only reads a zero counter).
 // 3. k_tile   one workgroup per tile accumulates into TILE^3 float64 LDS cells (ds_add_f64: the per-
 //             cell sum is exact to float64, the "compensated" accumulator) the stencil weights that
 //             fall inside the tile, from its own particles and from those of its 7 lower neighbours
@@ -34,6 +34,8 @@ constexpr int BT = 512;    // k_bin: threads per workgroup
 constexpr int KP = 4;      // k_bin: particles per thread per step
 constexpr int HT = 4096;   // k_bin: LDS hash slots (> BT * KP, so an insertion always finds a slot)
 constexpr int TT = 512;    // k_tile: threads per workgroup
+constexpr int OT = 1024;   // k_ov: threads per workgroup
+constexpr int OB = 256;    // k_ov: workgroups (per job)
 // particles per cell from which CIC tiles accumulate in register runs (measured at 512^3 particles: 8 per
 // cell 0.94 -> 0.78 ms, 4.1: 0.82 -> 0.75, 2.4: equal, 1.5: 0.75 -> 0.81; NGP gains nothing)
 constexpr double RUN_PPC = 3.0;
@@ -228,33 +230,30 @@ __global__ __launch_bounds__(BT) void k_bin_b(const BinArgs* __restrict__ tab,
     bin_body<S, HASW, 2, false>(tab[bj_], blk_);
 }
 
-// overflow grouping: count per tile, exclusive scan, scatter (records copied from the inputs)
-
-__device__ __forceinline__ void ov_count_body(const OvArgs& a, Blk B) {
-    const long long n = *a.ov_count;
-    for (long long i = (long long)B.x * blockDim.x + threadIdx.x; i < n; i += (long long)B.gx * blockDim.x)
-        atomicAdd(&a.ocnt[a.ov_key[i] >> 3], 1u);
-}
-__global__ __launch_bounds__(256) void k_ov_count(OvArgs a) { ov_count_body(a, own_blk()); }
-// batched: job blockIdx.y
-__global__ __launch_bounds__(256) void k_ov_count_b(const OvArgs* __restrict__ tab) {
-    const OvArgs& a = tab[blockIdx.y];
-    ov_count_body(a, own_blk());
-}
-
-// (nothing overflowed: every group is empty and k_tile never reads an offset, so skip the scan)
-__device__ __forceinline__ void scan_body(const unsigned* __restrict__ ov_count, const unsigned* __restrict__ cnt,
-                                          unsigned* __restrict__ off, int n) {
-    __shared__ unsigned part[1024];
-    if (*ov_count == 0u) return;
-    const int tid = threadIdx.x;
-    const int per = (n + 1023) / 1024;
+// Overflow grouping in one launch: the first workgroup to arrive counts and scans, then all copy the records.  A tile's
+// records are what its class fills exceed their capacities by, so the list itself is not counted.  The others wait for
+// a workgroup that is running by then (it took its ticket) and waits for none, so the wait ends whatever else the card
+// runs.  Nothing overflowed (every group is empty and k_tile reads no offset): one read and out, 4.7 us where three
+// launches took 14.
+__device__ __forceinline__ void ov_scan(const OvArgs& a) {
+    __shared__ unsigned part[OT];
+    const int tid = threadIdx.x, n = a.ntiles;
+    const int per = (n + OT - 1) / OT;
     const int lo = tid * per, hi = min(n, lo + per);
     unsigned s = 0;
-    for (int i = lo; i < hi; ++i) s += cnt[i];
+#pragma unroll 4
+    for (int i = lo; i < hi; ++i) {
+        unsigned f[8], k = 0u;
+        const uint4 fa = ((const uint4*)a.fill)[2 * (long long)i], fb = ((const uint4*)a.fill)[2 * (long long)i + 1];
+        f[0] = fa.x, f[1] = fa.y, f[2] = fa.z, f[3] = fa.w, f[4] = fb.x, f[5] = fb.y, f[6] = fb.z, f[7] = fb.w;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) k += f[c] - min(f[c], (unsigned)a.cap[c]);
+        a.ocnt[i] = k;
+        s += k;
+    }
     part[tid] = s;
     __syncthreads();
-    for (int d = 1; d < 1024; d <<= 1) {
+    for (int d = 1; d < OT; d <<= 1) {
         unsigned v = tid >= d ? part[tid - d] : 0u;
         __syncthreads();
         part[tid] += v;
@@ -262,27 +261,36 @@ __device__ __forceinline__ void scan_body(const unsigned* __restrict__ ov_count,
     }
     unsigned run = tid ? part[tid - 1] : 0u;
     for (int i = lo; i < hi; ++i) {
-        off[i] = run;
-        run += cnt[i];
+        a.ooff[i] = run;
+        run += a.ocnt[i];
     }
-    if (tid == 1023) off[n] = part[1023];
-}
-__global__ __launch_bounds__(1024) void k_scan(OvArgs a) { scan_body(a.ov_count, a.ocnt, a.ooff, a.ntiles); }
-// batched: one workgroup per job
-__global__ __launch_bounds__(1024) void k_scan_b(const OvArgs* __restrict__ tab) {
-    const OvArgs& a = tab[blockIdx.x];
-    scan_body(a.ov_count, a.ocnt, a.ooff, a.ntiles);
 }
 
 template <bool HASW>
-__device__ __forceinline__ void ov_scatter_body(const OvArgs& a, Blk B) {
+__device__ __forceinline__ void ov_body(const OvArgs& a, Blk B) {
     constexpr int R = HASW ? 4 : 3;
+    __shared__ unsigned ticket;
     const long long n = *a.ov_count;
     if (n == 0) return;
+    if (threadIdx.x == 0) ticket = atomicAdd(&a.turn[0], 1u);
+    __syncthreads();
+    if (ticket == 0u) {
+        ov_scan(a);
+        __threadfence();
+        __syncthreads();
+        if (threadIdx.x == 0) __hip_atomic_store(&a.turn[1], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        if (threadIdx.x == 0)
+            // (an acquire for every look would keep emptying the caches that the scan works in)
+            while (__hip_atomic_load(&a.turn[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
+                __builtin_amdgcn_s_sleep(32);
+        __syncthreads();
+        __threadfence();
+    }
     const bool sel = a.sel && *a.sel;
     const float* __restrict__ pos = sel ? a.spos : a.pos;
     const float* __restrict__ W = sel ? a.sw : a.W;
-    for (long long i = (long long)B.x * blockDim.x + threadIdx.x; i < n; i += (long long)B.gx * blockDim.x) {
+    for (long long i = (long long)B.x * OT + threadIdx.x; i < n; i += (long long)B.gx * OT) {
         const unsigned key = a.ov_key[i], t = key >> 3;
         const long long p = a.ov_idx[i];
         const unsigned s = a.ooff[t] + atomicAdd(&a.ocur[t], 1u);
@@ -297,11 +305,12 @@ __device__ __forceinline__ void ov_scatter_body(const OvArgs& a, Blk B) {
     }
 }
 template <bool HASW>
-__global__ __launch_bounds__(256) void k_ov_scatter(OvArgs a) { ov_scatter_body<HASW>(a, own_blk()); }
+__global__ __launch_bounds__(OT) void k_ov(OvArgs a) { ov_body<HASW>(a, own_blk()); }
+// batched: job blockIdx.y
 template <bool HASW>
-__global__ __launch_bounds__(256) void k_ov_scatter_b(const OvArgs* __restrict__ tab) {
+__global__ __launch_bounds__(OT) void k_ov_b(const OvArgs* __restrict__ tab) {
     const OvArgs& a = tab[blockIdx.y];
-    ov_scatter_body<HASW>(a, own_blk());
+    ov_body<HASW>(a, own_blk());
 }
 
 enum { OUT_ACC = 0, OUT_SET = 1, OUT_DELTA = 2 };
@@ -904,7 +913,7 @@ struct Presort {
 struct Layout {
     int nt, cap[8], cofs[8];
     long long ntiles, CT;
-    size_t ncnt;   // counters: fill (8 ntiles) | ocnt | ocur | ooff (ntiles + 1) | ov_count
+    size_t ncnt;   // counters: fill (8 ntiles) | ocnt | ocur | ooff (ntiles + 1) | ov_count | turn (2)
     size_t cnt_bytes, bucket_bytes, ov_bytes;
 };
 
@@ -923,7 +932,7 @@ static int layout_of(int64_t n, int dims, int S, bool hasw, Layout* L) {
         L->cofs[c] = (int)L->CT;
         L->CT += v;
     }
-    L->ncnt = 11 * (size_t)L->ntiles + 2;
+    L->ncnt = 11 * (size_t)L->ntiles + 4;
     L->cnt_bytes = sizeof(unsigned) * L->ncnt + 64;
     L->bucket_bytes = sizeof(float) * (size_t)L->ntiles * L->CT * R;
     // overflow: ov_idx (8n) | ov_key (4n) | gcls (4n) | grouped (4Rn)
@@ -982,11 +991,10 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
     }
     {
         StageTimer tm("deposit_overflow", st);
-        const OvArgs oa{ov_count, ov_idx, ov_key, ocnt, ooff, ocur, pos, W, grouped, gcls, rsd, (int)ntiles,
-                        ps.sel, ps.pos, ps.W};
-        hipLaunchKernelGGL(k_ov_count, dim3(256), dim3(256), 0, st, oa);
-        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, oa);
-        hipLaunchKernelGGL((k_ov_scatter<HASW>), dim3(256), dim3(256), 0, st, oa);
+        OvArgs oa{ov_count, ov_idx, ov_key, fill, {}, ocnt, ooff, ocur, ov_count + 1, pos, W, grouped, gcls, rsd,
+                  (int)ntiles, ps.sel, ps.pos, ps.W};
+        for (int c = 0; c < 8; ++c) oa.cap[c] = cap[c];
+        hipLaunchKernelGGL((k_ov<HASW>), dim3(OB), dim3(OT), 0, st, oa);
         PYL_HIP(hipGetLastError());
     }
     {
@@ -1210,7 +1218,9 @@ int binned_job_plan(const float* pos, const float* W, int64_t n, int dims, doubl
     long long bb = (n + (long long)BT * KP - 1) / ((long long)BT * KP);
     if (bb > 2048) bb = 2048;
     j->bin_blocks = (unsigned)((bb + XCDS - 1) / XCDS * XCDS);
-    j->ov = OvArgs{ov_count, ov_idx, ov_key, ocnt, ooff, ocur, bpos, bW, grouped, gcls, Rsd(), (int)ntiles};
+    j->ov = OvArgs{ov_count, ov_idx, ov_key, fill, {}, ocnt, ooff, ocur, ov_count + 1, bpos, bW, grouped, gcls, Rsd(),
+                   (int)ntiles};
+    for (int c = 0; c < 8; ++c) j->ov.cap[c] = L.cap[c];
     j->tile_blocks = (unsigned)((ntiles + XCDS - 1) / XCDS * XCDS);
     j->cnt = cnt;
     j->cnt_bytes = sizeof(unsigned) * L.ncnt;
@@ -1234,9 +1244,7 @@ static int batch_launch_s(bool sorted, const BinnedTables& t, hipStream_t st) {
     }
     {
         StageTimer tm("deposit_overflow", st);
-        hipLaunchKernelGGL(k_ov_count_b, dim3(256, nj), dim3(256), 0, st, t.ov);
-        hipLaunchKernelGGL(k_scan_b, dim3(nj), dim3(1024), 0, st, t.ov);
-        hipLaunchKernelGGL((k_ov_scatter_b<HASW>), dim3(256, nj), dim3(256), 0, st, t.ov);
+        hipLaunchKernelGGL((k_ov_b<HASW>), dim3(OB, nj), dim3(OT), 0, st, t.ov);
         PYL_HIP(hipGetLastError());
     }
     {

@@ -52,9 +52,12 @@ struct OvArgs {
     const unsigned* ov_count;   // [1] records in the overflow list
     const long long* ov_idx;    // particle index of each
     const unsigned* ov_key;     // (tile, class) key of each
+    const unsigned* fill;       // [8 ntiles] records per (tile, class), overflow included
+    int cap[8];                 // capacity of each class segment
     unsigned* ocnt;             // [ntiles] overflow records per tile
-    unsigned* ooff;             // [ntiles + 1] first grouped slot of each tile
+    unsigned* ooff;             // [ntiles] first grouped slot of each tile
     unsigned* ocur;             // [ntiles] slots handed out
+    unsigned* turn;             // [2] workgroups that arrived, 1 when the offsets are written
     const float* pos;
     const float* W;
     float* grouped;             // records grouped by tile
