@@ -100,9 +100,20 @@ template <typename R> struct BinClass {
 
 }  // namespace
 
+// One step of a plan's launch sequence: steps of one stage with different chains touch different jobs (or, in the last
+// chain, the shared workspaces of the single-job path), steps of one chain run in order
+enum { ST_PREPARE, ST_DEPOSIT, ST_SPECTRUM, ST_REDUCE, ST_SINGLE };
+struct BatchStep {
+    int stage, chain;
+    std::function<int(hipStream_t)> run;
+};
+
 struct BatchPlan {
     std::vector<JobPlan> jobs;
-    std::vector<std::function<int(hipStream_t)>> steps;
+    std::vector<BatchStep> steps;
+    void step(int stage, int chain, std::function<int(hipStream_t)> f) {
+        steps.push_back(BatchStep{stage, chain, std::move(f)});
+    }
     // classes (kept alive: the steps hold pointers to their device tables)
     std::map<std::tuple<int, int, int, int, int>, DepClass> dep;
     std::map<int, FftClass<float>> fft32;
@@ -160,10 +171,12 @@ static int plan_spectrum(BatchPlan* B, JobPlan& J, char*& p) {
 
 template <typename R>
 static void plan_spectrum_steps(BatchPlan* B, std::map<int, FftClass<R>>& fft,
-                                std::map<std::pair<int, int>, BinClass<R>>& bins) {
+                                std::map<std::pair<int, int>, BinClass<R>>& bins, int* chains) {
+    std::map<int, int> chain;   // of a size
     for (auto& kv : fft) {
         FftClass<R>* F = &kv.second;
-        B->steps.push_back([F](hipStream_t st) {
+        chain[F->N] = (*chains)++;
+        B->step(ST_SPECTRUM, chain[F->N], [F](hipStream_t st) {
             {
                 StageTimer t("fft_z_r2c", st);
                 int rc = r2c_batch<R>(F->N, F->r2c.dev, F->r2c.dstart, F->r2c.nj(), F->r2c.total(), st);
@@ -175,7 +188,7 @@ static void plan_spectrum_steps(BatchPlan* B, std::map<int, FftClass<R>>& fft,
     }
     for (auto& kv : bins) {
         BinClass<R>* C = &kv.second;
-        B->steps.push_back([C](hipStream_t st) {
+        B->step(ST_SPECTRUM, chain[C->N], [C](hipStream_t st) {
             StageTimer t("fft_last_bin", st);
             return last_bin_batch<R>(C->N, C->axis, C->last.dev, C->last.dstart, C->last.nj(), C->last.total(), st);
         });
@@ -325,7 +338,7 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
     // 5. the launch sequence
     if (B->zero.nj() > 0) {
         Table<ZeroArgs>* Z = &B->zero;
-        B->steps.push_back([Z](hipStream_t st) {
+        B->step(ST_PREPARE, 0, [Z](hipStream_t st) {
             hipLaunchKernelGGL(k_zero_b, dim3(64, (unsigned)Z->nj()), dim3(256), 0, st, Z->dev);
             PYL_HIP(hipGetLastError());
             return (int)OK;
@@ -336,21 +349,23 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
         const float* W = J.job.W;
         const int64_t n = J.job.n;
         double* dm = J.dmass;
-        B->steps.push_back([W, n, dm](hipStream_t st) { return weight_sum(W, n, dm, st); });
+        B->step(ST_PREPARE, 0, [W, n, dm](hipStream_t st) { return weight_sum(W, n, dm, st); });
     }
+    int chains = 0;
     for (auto& kv : B->dep) {
         DepClass* D = &kv.second;
-        B->steps.push_back([D](hipStream_t st) {
+        B->step(ST_DEPOSIT, chains++, [D](hipStream_t st) {
             BinnedTables t{D->bin.nj(), D->sup.dev, D->sup.dstart, D->sup.total(), D->bin.dev,
                            D->bin.dstart, D->bin.total(), D->ov.dev, D->tile.dev, D->tile.dstart, D->tile.total()};
             return binned_batch_launch(D->scheme, D->hasw, D->prec == PYL_F64, D->acc, D->sorted, t, st);
         });
     }
-    plan_spectrum_steps<float>(B, B->fft32, B->bin32);
-    plan_spectrum_steps<double>(B, B->fft64, B->bin64);
+    chains = 0;
+    plan_spectrum_steps<float>(B, B->fft32, B->bin32, &chains);
+    plan_spectrum_steps<double>(B, B->fft64, B->bin64, &chains);
     if (B->red.nj() > 0) {
         Table<ReduceArgs>* T = &B->red;
-        B->steps.push_back([T](hipStream_t st) {
+        B->step(ST_REDUCE, 0, [T](hipStream_t st) {
             StageTimer t("finalize", st);
             return pk_reduce_batch(T->dev, T->dstart, T->nj(), T->total(), st);
         });
@@ -359,7 +374,7 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
     for (auto& J : B->jobs) {
         if (J.batched) continue;
         const pyl_pk_job j = J.job;
-        B->steps.push_back([j](hipStream_t st) {
+        B->step(ST_SINGLE, 0, [j](hipStream_t st) {
             return pk_particles(j.pos, j.W, j.n, j.dims, j.BoxSize, j.scheme, j.axis, j.prec,
                                 j.flags | PYL_PK_ASYNC | (j.flags & DEP_ATOMIC ? 0 : DEP_ATOMIC), j.out, st, Rsd());
         });
@@ -369,11 +384,73 @@ static int batch_build(const pyl_pk_job* jobs, int njobs, hipStream_t st, BatchP
 }
 
 static int batch_run(const BatchPlan* B, hipStream_t st) {
-    for (auto& f : B->steps) {
-        int rc = f(st);
+    for (auto& s : B->steps) {
+        int rc = s.run(st);
         if (rc) return rc;
     }
     return OK;
+}
+
+// The same sequence, recorded into a capture on `st` with its independent chains side by side: the classes of the
+// deposit, then the sizes of the transforms, on LANES streams, and the jobs of the single-job path beside both on one of
+// their own.  Many of the kernels fill a part of the chip only, or take a launch's latency and no more (twelve mocks of
+// 32^3 to 256^3, 95 kernels: one after another 1783 us a replay with its results, side by side 1600).  Four streams: as many as the hardware has
+// queues.  The streams only serve the capture; a replay needs none of them.
+constexpr int LANES = 3;
+struct CaptureLanes {
+    hipStream_t side[LANES] = {};   // side[0] takes the single-job path; the lanes are the captured stream and the rest
+    hipEvent_t ev = nullptr;
+    int create() {
+        PYL_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        for (auto& s : side) PYL_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+        return OK;
+    }
+    ~CaptureLanes() {   // after the capture has ended
+        for (auto& s : side)
+            if (s) (void)hipStreamDestroy(s);
+        if (ev) (void)hipEventDestroy(ev);
+    }
+};
+
+static int batch_capture(const BatchPlan* B, const CaptureLanes& C, hipStream_t st) {
+    hipStream_t const* side = C.side;
+    hipEvent_t ev = C.ev;
+    hipStream_t lane[LANES] = {st, side[1], side[2]};
+    // a wait in a capture is on the recorded point, so one event serves them all
+    auto order = [&](hipStream_t before, hipStream_t after) -> int {
+        PYL_HIP(hipEventRecord(ev, before));
+        PYL_HIP(hipStreamWaitEvent(after, ev, 0));
+        return OK;
+    };
+    int rc = OK, stage = ST_PREPARE;
+    bool forked = false, single = false;
+    for (auto& s : B->steps) {
+        if (s.stage == ST_SINGLE) continue;
+        if (s.stage != stage) {   // stages follow one another
+            if (!single) {
+                // the single-job path starts with the first deposits
+                if ((rc = order(st, side[0]))) return rc;
+                for (auto& q : B->steps)
+                    if (q.stage == ST_SINGLE && (rc = q.run(side[0]))) return rc;
+                single = true;
+            }
+            for (int i = 1; i < LANES; ++i)
+                if (forked && (rc = order(lane[i], st))) return rc;
+            for (int i = 1; i < LANES; ++i)
+                if ((rc = order(st, lane[i]))) return rc;
+            forked = true;
+            stage = s.stage;
+        }
+        if ((rc = s.run(lane[s.chain % LANES]))) return rc;
+    }
+    if (!single) {   // no batched jobs
+        for (auto& q : B->steps)
+            if (q.stage == ST_SINGLE && (rc = q.run(st))) return rc;
+        return OK;
+    }
+    for (int i = 1; i < LANES; ++i)
+        if ((rc = order(lane[i], st))) return rc;
+    return order(side[0], st);
 }
 
 }  // namespace pyl
@@ -421,7 +498,7 @@ extern "C" int pyl_graph_create(const pyl_pk_job* jobs, int njobs, void* stream,
     {
         ArenaScope scope(h->arena);
         // plan in the graph's own workspaces (autotuner trials, tables, geometry), one eager run that
-        // sizes every remaining workspace, then the capture of the same launch sequence
+        // sizes every remaining workspace, then the capture of the same launches
         rc = batch_build(jobs, njobs, st, &h->plan);
         if (rc == OK) rc = batch_run(h->plan, st);
         hipError_t e = rc ? hipSuccess : hipStreamSynchronize(st);
@@ -429,6 +506,8 @@ extern "C" int pyl_graph_create(const pyl_pk_job* jobs, int njobs, void* stream,
             set_error("hipStreamSynchronize -> %s", hipGetErrorString(e));
             rc = (int)e + 1000;
         }
+        CaptureLanes lanes;
+        if (rc == OK) rc = lanes.create();
         if (rc == OK) {
             ws_arena_seal(h->arena);
             e = hipStreamBeginCapture(st, hipStreamCaptureModeRelaxed);
@@ -436,7 +515,7 @@ extern "C" int pyl_graph_create(const pyl_pk_job* jobs, int njobs, void* stream,
                 set_error("hipStreamBeginCapture -> %s", hipGetErrorString(e));
                 rc = (int)e + 1000;
             } else {
-                rc = batch_run(h->plan, st);
+                rc = batch_capture(h->plan, lanes, st);
                 e = hipStreamEndCapture(st, &h->graph);
                 if (rc == OK && e != hipSuccess) {
                     set_error("hipStreamEndCapture -> %s", hipGetErrorString(e));
