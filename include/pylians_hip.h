@@ -139,6 +139,10 @@ int pyl_pk_layout(int dims, int* kmax_par, int* kmax_per, int* kmax, int64_t* ou
  * stream capture) the call does not synchronise and the caller checks the returned Nmodes. */
 int pyl_pk(const void* delta, int dims, double BoxSize, int axis, int mas_p, int prec, int flags, double* out,
            void* deltak_out, void* stream);
+/* The same with the results in host memory (`host`, out_len values), there when the call returns; not with PYL_PK_ASYNC
+ * or inside a stream capture (PYL_E_ARG). */
+int pyl_pk_host(const void* delta, int dims, double BoxSize, int axis, int mas_p, int prec, int flags, double* host,
+                void* deltak_out, void* stream);
 
 /* No counterpart in the reference.  pyl_pk for callers that cannot allocate device memory (code
  * under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): the same arguments
@@ -158,6 +162,10 @@ int pyl_pk_noalloc(const void* delta, int dims, double BoxSize, int axis, int ma
  * and PYL_PK_ASYNC behave as in pyl_pk. */
 int pyl_pk_particles(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, int axis,
                      int prec, int flags, double* out, void* stream);
+/* The same, or with `vel` pyl_pk_particles_rsd, with the results in host memory as pyl_pk_host. */
+int pyl_pk_particles_host(const float* pos, const float* vel, const float* W, int64_t n, int dims, double BoxSize,
+                          float Hubble, float redshift, int rsd_axis, int scheme, int axis, int prec, int flags,
+                          double* host, void* stream);
 
 /* Replaces Pk_library.correct_MAS (Pk_library.pyx:1749-1806): r2c of the (dims^3) field, every
  * independent mode multiplied by the float window factor prod_i (x_i/sin x_i)^mas_p (the dependent

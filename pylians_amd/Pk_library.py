@@ -17,6 +17,7 @@ Inputs may be numpy arrays or torch tensors on the GPU.  A float32 field runs th
 path (float32 FFT, float64 shell sums, as the reference); a float64 field runs the float64
 path.  ``threads`` is accepted for signature parity and ignored.
 """
+import functools
 import sys
 import time
 
@@ -143,6 +144,7 @@ def IFFT3Dr_d(a, threads=1):
     return _fft_c2r(a, _lib.F64T, _lib.C128T, _lib.F64)
 
 
+@functools.lru_cache(maxsize=64)
 def pk_layout(dims):
     """(kmax_par, kmax_per, kmax, out_len) of the pyl_pk output vector."""
     import ctypes
@@ -188,15 +190,15 @@ class Pk:
         d = _grid3(delta, real_t, "delta")
         dims = int(d.shape[0])
         _, _, _, nout = pk_layout(dims)
-        out = _lib.empty((nout,), _lib.F64T)
+        out = np.empty(nout)
         dk = _lib.empty((dims, dims, dims // 2 + 1), cplx_t) if keep_deltak else None
-        rc = _lib.lib().pyl_pk(_lib.ptr(d), dims, float(BoxSize), int(axis), MAS_function(MAS),
-                               _lib.F64 if f64 else _lib.F32, _lib.PK_ALL | _EXTRA_FLAGS, _lib.ptr(out),
-                               _lib.ptr(dk), _lib.stream())
+        rc = _lib.lib().pyl_pk_host(_lib.ptr(d), dims, float(BoxSize), int(axis), MAS_function(MAS),
+                                    _lib.F64 if f64 else _lib.F32, _lib.PK_ALL | _EXTRA_FLAGS, out.ctypes.data,
+                                    _lib.ptr(dk), _lib.stream())
         if rc == _lib.E_MODES:
             _modes_exit(rc)
         _lib.check(rc)
-        unpack_pk(self, _lib.to_host(out), dims)
+        unpack_pk(self, out, dims)
         if keep_deltak:
             self.delta_k = _ret(delta, dk)
         if VERBOSE:

@@ -60,6 +60,8 @@ SIGNATURES = {
     "pyl_pk_layout": [_i, _vp, _vp, _vp, _vp],
     "pyl_pk": [_vp, _i, _d, _i, _i, _i, _i, _vp, _vp, _vp],
     "pyl_pk_noalloc": [_vp, _i, _d, _i, _i, _i, _i, _vp, _vp, _vp],
+    "pyl_pk_host": [_vp, _i, _d, _i, _i, _i, _i, _vp, _vp, _vp],
+    "pyl_pk_particles_host": [_vp, _vp, _vp, _i64, _i, _d, _f, _f, _i, _i, _i, _i, _i, _vp, _vp],
     "pyl_pk_particles": [_vp, _vp, _i64, _i, _d, _i, _i, _i, _i, _vp, _vp],
     "pyl_pk_particles_rsd": [_vp, _vp, _vp, _i64, _i, _d, _f, _f, _i, _i, _i, _i, _i, _vp, _vp],
     "pyl_pos_redshift_space": [_vp, _vp, _i64, _i, _f, _f, _f, _i, _vp],

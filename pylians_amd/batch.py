@@ -31,11 +31,14 @@ class PkBatch:
         self._keep = []
         self._outs = []
         arr = (_lib.PkJob * len(jobs))()
+        # the jobs' outputs side by side: one copy brings them all to the host
+        sizes = [pk_layout(int(j["dims"]))[3] for j in jobs]
+        self._out = torch.empty(sum(sizes), dtype=torch.float64, device="cuda")
         for i, j in enumerate(jobs):
             p = _lib.to_dev(j["pos"], torch.float32)
             w = None if j.get("W") is None else _lib.to_dev(j["W"], torch.float32)
             dims = int(j["dims"])
-            out = torch.empty(pk_layout(dims)[3], dtype=torch.float64, device="cuda")
+            out = self._out[sum(sizes[:i]):sum(sizes[:i + 1])]
             self._keep += [p, w]
             self._outs.append((out, dims))
             arr[i] = _lib.PkJob(p.data_ptr(), 0 if w is None else w.data_ptr(), int(p.shape[0]), dims,
@@ -66,9 +69,11 @@ class PkBatch:
     def results(self):
         self.stream.synchronize()
         res = []
+        host, at = _lib.to_host(self._out), 0
         for out, dims in self._outs:
             r = _Res()
-            unpack_pk(r, _lib.to_host(out), dims)
+            unpack_pk(r, host[at:at + out.shape[0]], dims)
+            at += out.shape[0]
             # the DC mode is counted by the kernel and dropped from the output (Pk_library.pyx:411-412)
             check_number_modes(np.concatenate([[1.0], r.Nmodes3D]), dims)
             res.append(r)

@@ -136,6 +136,7 @@ extern "C" int pyl_pk_layout(int dims, int* kmax_par, int* kmax_per, int* kmax, 
 // counted the bins whose count differs from the independent-mode geometry into chk.status.
 // Synchronises the stream unless PK_ASYNC is set or the stream is being captured (then the
 // counts are only in the output's Nmodes, for the caller to check).
+static int modes_error(const PkGeometry* g, const PkCheck& chk, unsigned bad);
 static int check_modes(const PkGeometry* g, const PkCheck& chk, int flags, hipStream_t st) {
     if (flags & PK_ASYNC) return OK;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -144,7 +145,10 @@ static int check_modes(const PkGeometry* g, const PkCheck& chk, int flags, hipSt
     unsigned bad = 0u;
     PYL_HIP(hipMemcpyAsync(&bad, chk.status, sizeof(unsigned), hipMemcpyDeviceToHost, st));
     PYL_HIP(hipStreamSynchronize(st));
-    if (bad == 0u) return OK;
+    return bad == 0u ? (int)OK : modes_error(g, chk, bad);
+}
+
+static int modes_error(const PkGeometry* g, const PkCheck& chk, unsigned bad) {
     const PkDims& d = g->d;
     std::vector<double> c3(d.n3());
     PYL_HIP(hipMemcpy(c3.data(), chk.c3, sizeof(double) * d.n3(), hipMemcpyDeviceToHost));
@@ -158,11 +162,45 @@ static int check_modes(const PkGeometry* g, const PkCheck& chk, int flags, hipSt
     return E_MODES;
 }
 
+// The results of one call in the caller's host array.  The reduction left [status | k3D .. Nmodes1D | Pk2D] behind each
+// other, a quarter of the output: the wave numbers of the 2-D bins and their Nmodes (which the status says are the
+// geometry's) are written here while the device still works.  One copy and one wait take the rest (a status
+// word, a wait, then 3.0 MB at 512^3 copied twice after the last kernel: a call of 2690 us, now 2493; 32^3 134 and 73).
+static int host_results(const PkGeometry* g, const PkCheck& chk, double BoxSize, double* host, hipStream_t st) {
+    const PkDims& d = g->d;
+    const size_t head = 6 * (size_t)d.kmax + 3 * (size_t)d.kmax_par, n2 = d.n2();
+    PinnedScope pin;
+    int rc = pin.take(sizeof(double) * (1 + head + n2));
+    if (rc) return rc;
+    PYL_HIP(hipMemcpyAsync(pin.p, chk.status, sizeof(double) * (1 + head + n2), hipMemcpyDeviceToHost, st));
+    const double kF = 2.0 * M_PI / BoxSize;
+    double *kpar = host + head, *kper = kpar + n2, *P2 = kper + n2, *N2 = P2 + n2;
+    for (int q = 0, i = 0; q <= d.kmax_per; ++q)
+        for (int p = 0; p <= d.kmax_par; ++p, ++i) {
+            kpar[i] = 0.5 * (p + p + 1) * kF;
+            kper[i] = 0.5 * (q + q + 1) * kF;
+            N2[i] = (double)g->h_n2[i];
+        }
+    PYL_HIP(hipStreamSynchronize(st));
+    const double* r = (const double*)pin.p;
+    unsigned bad;
+    memcpy(&bad, r, sizeof bad);
+    if (bad) return modes_error(g, chk, bad);
+    memcpy(host, r + 1, sizeof(double) * head);
+    memcpy(P2, r + 1 + head, sizeof(double) * n2);
+    return OK;
+}
+
 namespace pyl {
 template <typename R>
 int pk_from_delta(const R* delta, int dims, double BoxSize, int axis, int mas_p, int flags, double* out,
-                  cplx<R>* keep, bool affine, const double* dmass, double mass, hipStream_t st) {
+                  cplx<R>* keep, bool affine, const double* dmass, double mass, hipStream_t st, double* host) {
     int rc = OK;
+    if (host) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        PYL_HIP(hipStreamIsCapturing(st, &cs));
+        PYL_CHECK(cs == hipStreamCaptureStatusNone, E_ARG, "results in host memory cannot be captured");
+    }
     // rows of the internal spectrum padded to 128 bytes: the strided column passes then read whole
     // cache lines (kz = N/2+1 .. P-1 are never touched)
     constexpr int64_t ALIGN = 128 / (int64_t)sizeof(cplx<R>);
@@ -171,10 +209,12 @@ int pk_from_delta(const R* delta, int dims, double BoxSize, int axis, int mas_p,
     if (rc) return rc;
     cplx<R>* spec = (cplx<R>*)workspace(WS_SPEC, sizeof(cplx<R>) * (size_t)dims * dims * P, &rc);
     if (rc) return rc;
-    double* cb = (double*)workspace(WS_SUMS, sizeof(double) * pk_check_doubles(g->d), &rc);
+    const size_t nchk = pk_check_doubles(g->d);
+    double* cb = (double*)workspace(WS_SUMS, sizeof(double) * (nchk + (host ? pk_out_len(g->d) : 0)), &rc);
     if (rc) return rc;
     PkCheck chk;
     pk_check_carve(g->d, cb, &chk);
+    if (host) out = cb + nchk;
     ReduceArgs ra;
     {
         StageTimer t("fft_z_r2c", st);
@@ -194,31 +234,43 @@ int pk_from_delta(const R* delta, int dims, double BoxSize, int axis, int mas_p,
     }
     {
         StageTimer t("finalize", st);
+        ra.compact = host != nullptr;
         rc = pk_reduce(ra, st);
         if (rc) return rc;
     }
-    return check_modes(g, chk, flags, st);
+    return host ? host_results(g, chk, BoxSize, host, st) : check_modes(g, chk, flags, st);
 }
 template int pk_from_delta<float>(const float*, int, double, int, int, int, double*, cplx<float>*, bool, const double*,
-                                  double, hipStream_t);
+                                  double, hipStream_t, double*);
 template int pk_from_delta<double>(const double*, int, double, int, int, int, double*, cplx<double>*, bool,
-                                   const double*, double, hipStream_t);
+                                   const double*, double, hipStream_t, double*);
 }  // namespace pyl
 
-extern "C" int pyl_pk(const void* delta, int dims, double BoxSize, int axis, int mas_p, int prec, int flags,
-                      double* out, void* deltak_out, void* stream) {
+static int pk_field(const void* delta, int dims, double BoxSize, int axis, int mas_p, int prec, int flags, double* out,
+                    void* deltak_out, hipStream_t st, double* host) {
     int rc = check_fft(dims, prec);
     if (rc) return rc;
     PYL_CHECK(axis >= 0 && axis <= 2, E_ARG, "axis must be 0, 1 or 2");
     PYL_CHECK(mas_p >= 0 && mas_p <= 4, E_ARG, "window exponent must be in [0, 4]");
     PYL_CHECK(BoxSize > 0, E_ARG, "BoxSize must be positive");
-    PYL_CHECK(delta && out, E_ARG, "null pointer");
-    hipStream_t st = (hipStream_t)stream;
+    PYL_CHECK(delta && (out || host), E_ARG, "null pointer");
     if (prec == PYL_F32)
         return pk_from_delta<float>((const float*)delta, dims, BoxSize, axis, mas_p, flags, out,
-                                    (cplx<float>*)deltak_out, false, nullptr, 1.0, st);
+                                    (cplx<float>*)deltak_out, false, nullptr, 1.0, st, host);
     return pk_from_delta<double>((const double*)delta, dims, BoxSize, axis, mas_p, flags, out,
-                                 (cplx<double>*)deltak_out, false, nullptr, 1.0, st);
+                                 (cplx<double>*)deltak_out, false, nullptr, 1.0, st, host);
+}
+
+extern "C" int pyl_pk(const void* delta, int dims, double BoxSize, int axis, int mas_p, int prec, int flags,
+                      double* out, void* deltak_out, void* stream) {
+    return pk_field(delta, dims, BoxSize, axis, mas_p, prec, flags, out, deltak_out, (hipStream_t)stream, nullptr);
+}
+
+extern "C" int pyl_pk_host(const void* delta, int dims, double BoxSize, int axis, int mas_p, int prec, int flags,
+                           double* host, void* deltak_out, void* stream) {
+    PYL_CHECK(host, E_ARG, "null pointer");
+    PYL_CHECK(!(flags & PK_ASYNC), E_ARG, "results in host memory are not asynchronous");
+    return pk_field(delta, dims, BoxSize, axis, mas_p, prec, flags, nullptr, deltak_out, (hipStream_t)stream, host);
 }
 
 // ------------------------------------------------------------------ deposit autotuner
@@ -364,12 +416,12 @@ int deposit_kind(const float* pos, const float* W, int64_t n, int dims, double B
 }
 
 int pk_particles(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, int axis,
-                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd, cplx<float>* keep) {
+                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd, cplx<float>* keep, double* host) {
     int rc = check_fft(dims, prec);
     if (rc) return rc;
     PYL_CHECK(axis >= 0 && axis <= 2, E_ARG, "axis must be 0, 1 or 2");
     PYL_CHECK(scheme >= 1 && scheme <= 4, E_ARG, "unknown mass-assignment scheme %d", scheme);
-    PYL_CHECK(n > 0 && pos && out, E_ARG, "bad particle arguments");
+    PYL_CHECK(n > 0 && pos && (out || host), E_ARG, "bad particle arguments");
     const size_t cells = (size_t)dims * dims * dims;
     const bool f64 = prec == PYL_F64;
     void* grid = workspace(WS_GRID, cells * (f64 ? 8 : 4), &rc);
@@ -391,9 +443,9 @@ int pk_particles(const float* pos, const float* W, int64_t n, int dims, double B
     const int pkflags = flags & (PYL_PK_ALL | PYL_PK_ASYNC | PYL_PK_DROP_KZ0);
     if (f64)
         return pk_from_delta<double>((const double*)grid, dims, BoxSize, axis, scheme, pkflags, out, nullptr,
-                                     kind == DK_ATOMIC, dmass, (double)n, st);
+                                     kind == DK_ATOMIC, dmass, (double)n, st, host);
     return pk_from_delta<float>((const float*)grid, dims, BoxSize, axis, scheme, pkflags, out, keep, false,
-                                dmass, (double)n, st);
+                                dmass, (double)n, st, host);
 }
 }  // namespace pyl
 
@@ -428,18 +480,35 @@ extern "C" int pyl_pk_particles(const float* pos, const float* W, int64_t n, int
     return pk_particles(pos, W, n, dims, BoxSize, scheme, axis, prec, flags, out, (hipStream_t)stream, Rsd());
 }
 
-extern "C" int pyl_pk_particles_rsd(const float* pos, const float* vel, const float* W, int64_t n, int dims,
-                                    double BoxSize, float Hubble, float redshift, int rsd_axis, int scheme, int axis,
-                                    int prec, int flags, double* out, void* stream) {
+static int rsd_of(const float* vel, double BoxSize, float Hubble, float redshift, int rsd_axis, Rsd* r) {
     PYL_CHECK(vel, E_ARG, "null velocity array");
     PYL_CHECK(rsd_axis >= 0 && rsd_axis <= 2, E_ARG, "rsd_axis must be 0, 1 or 2");
     PYL_CHECK(Hubble != 0.0f, E_ARG, "Hubble must be non-zero");
+    r->vel = vel;
+    r->axis = rsd_axis;
+    r->fac = (float)((1.0 + (double)redshift) / (double)Hubble);   // redshift_space_library.pyx:36
+    r->box = (float)BoxSize;
+    return OK;
+}
+
+extern "C" int pyl_pk_particles_rsd(const float* pos, const float* vel, const float* W, int64_t n, int dims,
+                                    double BoxSize, float Hubble, float redshift, int rsd_axis, int scheme, int axis,
+                                    int prec, int flags, double* out, void* stream) {
     Rsd r;
-    r.vel = vel;
-    r.axis = rsd_axis;
-    r.fac = (float)((1.0 + (double)redshift) / (double)Hubble);   // redshift_space_library.pyx:36
-    r.box = (float)BoxSize;
-    return pk_particles(pos, W, n, dims, BoxSize, scheme, axis, prec, flags, out, (hipStream_t)stream, r);
+    const int rc = rsd_of(vel, BoxSize, Hubble, redshift, rsd_axis, &r);
+    return rc ? rc : pk_particles(pos, W, n, dims, BoxSize, scheme, axis, prec, flags, out, (hipStream_t)stream, r);
+}
+
+extern "C" int pyl_pk_particles_host(const float* pos, const float* vel, const float* W, int64_t n, int dims,
+                                     double BoxSize, float Hubble, float redshift, int rsd_axis, int scheme, int axis,
+                                     int prec, int flags, double* host, void* stream) {
+    PYL_CHECK(host, E_ARG, "null pointer");
+    PYL_CHECK(!(flags & PK_ASYNC), E_ARG, "results in host memory are not asynchronous");
+    Rsd r;
+    const int rc = vel ? rsd_of(vel, BoxSize, Hubble, redshift, rsd_axis, &r) : (int)OK;
+    return rc ? rc
+              : pk_particles(pos, W, n, dims, BoxSize, scheme, axis, prec, flags, nullptr, (hipStream_t)stream, r,
+                             nullptr, host);
 }
 
 extern "C" int pyl_pos_redshift_space(float* pos, const float* vel, int64_t n, int cols, float BoxSize, float Hubble,

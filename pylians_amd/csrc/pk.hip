@@ -728,6 +728,10 @@ __device__ __forceinline__ unsigned finish_2d(const ReduceArgs& A, int kp, int k
     const unsigned bad = n != (double)A.n2c[i] ? 1u : 0u;
     const double kF = 2.0 * M_PI / A.BoxSize, unit = pk_unit(A.N, A.BoxSize);
     double* o = A.out + 6 * (A.n3 - 1) + 3 * A.kmax_par + i;
+    if (A.compact) {
+        o[0] = s * unit / n;
+        return bad;
+    }
     o[0] = 0.5 * (kp + kp + 1) * kF;
     o[n2] = 0.5 * (kq + kq + 1) * kF;
     o[2 * (long long)n2] = s * unit / n;

@@ -66,6 +66,7 @@ struct ReduceArgs {
     double* c3;
     unsigned* status;
     double* out;
+    int compact = 0;   // out holds [k3D .. Nmodes1D | Pk2D] only: the rest of the layout the host knows by itself
 };
 
 // Axis of the last forward FFT pass for a line of sight `axis`: 1 (y) for axis 0, else 0 (x).
@@ -111,14 +112,17 @@ struct Rsd;
 int deposit_kind(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, bool f64,
                  int flags, void* grid, const double* dmass, hipStream_t st, int* kind, const Rsd& rsd);
 int pk_particles(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, int axis,
-                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd, cplx<float>* keep = nullptr);
+                 int prec, int flags, double* out, hipStream_t st, const Rsd& rsd, cplx<float>* keep = nullptr,
+                 double* host = nullptr);
 
 // The whole estimator from a real (N,N,N) field: pass Z r2c (affine: delta = rho * N^3 / mass - 1
 // applied on the load, mass = dmass[0] when dmass is non-null), the column pass, the fused last pass
 // + binning, the normalisation and the mode check (see pyl_pk).  keep (nullable) receives the
-// corrected spectrum.
+// corrected spectrum.  host (nullable): the results go to this host array instead of `out`, which is not used; the call
+// then returns when they are there.
 template <typename R>
 int pk_from_delta(const R* delta, int dims, double BoxSize, int axis, int mas_p, int flags, double* out,
-                  cplx<R>* keep, bool affine, const double* dmass, double mass, hipStream_t st);
+                  cplx<R>* keep, bool affine, const double* dmass, double mass, hipStream_t st,
+                  double* host = nullptr);
 
 }  // namespace pyl

@@ -301,4 +301,54 @@ StreamScope::~StreamScope() {
 ArenaScope::ArenaScope(WsArena* a) : prev(t_arena) { t_arena = a; }
 ArenaScope::~ArenaScope() { t_arena = prev; }
 
+constexpr size_t PINNED_KEPT = 4;
+static std::mutex g_pin_mu;
+static std::vector<std::pair<void*, size_t>>& pin_free() {
+    static auto* v = new std::vector<std::pair<void*, size_t>>();   // outlives every caller
+    return *v;
+}
+
+int PinnedScope::take(size_t want) {
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        auto& v = pin_free();
+        for (size_t i = 0; i < v.size(); ++i)
+            if (v[i].second >= want) {
+                p = v[i].first;
+                bytes = v[i].second;
+                v.erase(v.begin() + (long)i);
+                return OK;
+            }
+    }
+    size_t b = 1 << 16;
+    while (b < want) b *= 2;
+    if (hipHostMalloc(&p, b, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+        set_error("pinned host allocation of %zu bytes failed", b);
+        return E_ALLOC;
+    }
+    bytes = b;
+    return OK;
+}
+
+PinnedScope::~PinnedScope() {
+    if (!p) return;
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        auto& v = pin_free();
+        if (v.size() < PINNED_KEPT) {
+            v.emplace_back(p, bytes);
+            return;
+        }
+        for (auto& e : v)   // the larger one stays
+            if (e.second < bytes) {
+                std::swap(e.first, p);
+                std::swap(e.second, bytes);
+                break;
+            }
+    }
+    (void)hipHostFree(p);
+}
+
 }  // namespace pyl

@@ -67,4 +67,13 @@ struct StreamScope {
     std::shared_ptr<StreamWs> ws;
 };
 
+// A pinned host buffer for one call's results, from a pool of at most PINNED_KEPT free ones (any thread or stream); given
+// back by the destructor, so only after the copies into it are done.
+struct PinnedScope {
+    void* p = nullptr;
+    size_t bytes = 0;
+    int take(size_t want);
+    ~PinnedScope();
+};
+
 }  // namespace pyl

@@ -60,16 +60,25 @@ class PkParticles:
                 raise ValueError("vel must have the shape of pos")
             rsd = (v, Hubble, redshift, axis if rsd_axis is None else rsd_axis)
         _, _, _, nout = pk_layout(dims)
-        out = _lib.empty((nout,), _lib.F64T)
         f = flags | {None: 0, "atomic": _lib.ATOMIC, "binned": _lib.BINNED, "presorted": _lib.SORTED}[deposit]
         try:
-            run_device(p, w, out, BoxSize, dims, _lib.SCHEMES[MAS], axis, PRECISION[precision], f, rsd)
+            if f & _lib.PK_ASYNC:   # no mode check: the counts come with the results
+                dev = _lib.empty((nout,), _lib.F64T)
+                run_device(p, w, dev, BoxSize, dims, _lib.SCHEMES[MAS], axis, PRECISION[precision], f, rsd)
+                out = _lib.to_host(dev)
+            else:
+                out = np.empty(nout)
+                v, hubble, z, rsd_axis = rsd or (None, 0.0, 0.0, 0)
+                _lib.check(_lib.lib().pyl_pk_particles_host(
+                    _lib.ptr(p), _lib.ptr(v), _lib.ptr(w), int(p.shape[0]), int(dims), float(BoxSize), float(hubble),
+                    float(z), int(rsd_axis), _lib.SCHEMES[MAS], int(axis), PRECISION[precision], int(f),
+                    out.ctypes.data, _lib.stream()))
         except _lib.PylError as e:
             if e.code == _lib.E_MODES:
                 from .Pk_library import _modes_exit
                 _modes_exit(e.code)
             raise
-        unpack_pk(self, _lib.to_host(out), dims)
+        unpack_pk(self, out, dims)
 
 
 def overdensity(pos, BoxSize, dims, MAS="CIC", W=None, precision="fp32", deposit=None):

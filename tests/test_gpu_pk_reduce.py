@@ -71,3 +71,32 @@ def test_batched_sizes(gpu):
             assert np.array_equal(r.Nmodes2D, s.Nmodes2D)
             assert np.max(np.abs(r.Pk - s.Pk)) <= 1e-5 * np.max(np.abs(s.Pk))
     b.close()
+
+
+@pytest.mark.parametrize("axis", [0, 2])
+@pytest.mark.parametrize("N", [8, 40, 128])
+def test_results_in_host_memory(gpu, N, axis):
+    """pyl_pk_host and pyl_pk_particles_host fill the whole layout with what the device entry points leave in device
+    memory; an asynchronous call is refused, and so is a null array."""
+    from pylians_amd import _lib
+    from pylians_amd.Pk_library import pk_layout
+    L, n = _lib.lib(), pk_layout(N)[3]
+    f = torch.from_numpy(np.random.default_rng(N).standard_normal((N, N, N)).astype(np.float32)).cuda()
+    pos = torch.rand((500, 3), device="cuda", generator=torch.Generator("cuda").manual_seed(N)) * 70
+    dev, host = torch.zeros(n, dtype=torch.float64, device="cuda"), np.full(n, -1.0)
+    for flags in (_lib.PK_ALL, 0):
+        _lib.check(L.pyl_pk(_lib.ptr(f), N, 70.0, axis, 2, _lib.F32, flags, _lib.ptr(dev), None, _lib.stream()))
+        _lib.check(L.pyl_pk_host(_lib.ptr(f), N, 70.0, axis, 2, _lib.F32, flags, host.ctypes.data, None, _lib.stream()))
+        a = dev.cpu().numpy()
+        assert np.array_equal(np.isnan(a), np.isnan(host))
+        ok = ~np.isnan(a)
+        assert np.all(np.abs(a[ok] - host[ok]) <= 1e-12 * np.abs(a[ok]) + 1e-12)   # LDS sums in another order
+    args = (_lib.ptr(pos), None, None, 500, N, 70.0, 0.0, 0.0, 0, 2, axis, _lib.F32)
+    _lib.check(L.pyl_pk_particles_host(*args, _lib.PK_ALL | _lib.ATOMIC, host.ctypes.data, _lib.stream()))
+    _lib.check(L.pyl_pk_particles(_lib.ptr(pos), None, 500, N, 70.0, 2, axis, _lib.F32, _lib.PK_ALL | _lib.ATOMIC,
+                                  _lib.ptr(dev), _lib.stream()))
+    a = dev.cpu().numpy()
+    pw = np.nan_to_num(a - host)
+    assert np.max(np.abs(pw)) <= 1e-5 * np.nanmax(np.abs(a))   # float64 deposit, one rounding to float32
+    assert L.pyl_pk_particles_host(*args, _lib.PK_ASYNC, host.ctypes.data, _lib.stream()) != 0
+    assert L.pyl_pk_host(_lib.ptr(f), N, 70.0, axis, 2, _lib.F32, _lib.PK_ALL, None, None, _lib.stream()) != 0
