@@ -422,11 +422,23 @@ template <typename R> const cplx<R>* twiddles(int N) {
 template const cplx<float>* twiddles<float>(int);
 template const cplx<double>* twiddles<double>(int);
 
+// Rows of a workgroup in the passes along z (M = N/2 points a row).  Powers of two keep Geo's: 16 rows in float32, 8 in
+// float64 (8 rows, 256^3 float32: 32 -> 34 us).  Rows with a factor 3 or 5 have more stages, each with a barrier over the
+// workgroup, and odd thread counts: smaller workgroups wait less.  float32, 4 rows for 16 (8), r2c: 320^3 87 -> 59 us (74),
+// 384^3 151 -> 93 (116, a copy of the bytes takes 95), 640^3 556 -> 489; c2r: 320^3 77 -> 63, 384^3 124 -> 112, but
+// 640^3 624 -> 644.  float64, 4 rows for 8 where 8 leave LDS for two workgroups a CU: r2c 640^3 1237 -> 818, 768^3 1998 ->
+// 1553, c2r 640^3 1319 -> 860; below that 384^3 160 -> 165 and 181 -> 189.
+template <typename R> constexpr int rows_z(int M, bool inverse) {
+    if ((M & (M - 1)) == 0) return Geo<R>::NL;
+    if (sizeof(R) == 8) return M >= 320 ? 4 : Geo<R>::NL;
+    return inverse && M >= 320 ? Geo<R>::NL : 4;
+}
+
 // pass Z launch shape of one job: M = N/2-point complex rows, NL rows per block; persistent grid of
 // about as many blocks as fit on the chip at once (LDS bound)
 template <typename R, int N> struct R2cShape {
     static constexpr int M = N / 2;
-    static constexpr int NL = Geo<R>::NL;
+    static constexpr int NL = rows_z<R>(M, false);
     // 8 complex values per thread, whole wavefronts (16, with 80 or 160 threads for rows of 160 or 320 points: 320^3
     // float32 115 -> 86 us, float64 236 -> 114)
     static constexpr int T = (2 * threads_for(M, NL) + 63) / 64 * 64;
@@ -474,7 +486,7 @@ template <typename R, int N>
 static int launch_c2r_rows(const cplx<R>* in, R* out, long long nrows, int64_t P, R sc, int store,
                            const R* aux, double* acc, hipStream_t st, int K) {
     constexpr int M = N / 2;
-    constexpr int NL = Geo<R>::NL;
+    constexpr int NL = rows_z<R>(M, true);
     // 8 complex values per thread (16: 256^3 float32 43 -> 30 us with twice the threads), whole wavefronts
     constexpr int T = (2 * threads_for(M, NL) + 63) / 64 * 64;
     const cplx<R>* tw = twiddles<R>(N);
