@@ -13,7 +13,7 @@ using namespace pyl;
 
 // ------------------------------------------------------------------ no-allocation power spectrum
 // pyl_pk_noalloc: pyl_pk for callers that cannot allocate device memory.  Everything pyl_pk keeps
-// in library workspaces and cached tables -- the half spectrum, the float64 sums and mode counts,
+// in library workspaces and cached tables -- the half spectrum, the mode counts,
 // the per-workgroup partial histograms, the twiddles, the window table and the mode geometry --
 // is carved from `scratch`, a fixed per-GPU array, and the tables are uploaded into it on every
 // call.  Its address on a device comes from hipGetSymbolAddress on the first call made with that
