@@ -123,7 +123,9 @@ __global__ __launch_bounds__(T) void k_xbin(XBinArgs a) {
     // values and window entries of the next step load while the present one is binned: the histograms leave room for few
     // waves a CU, which cannot hide the loads' latency (three fields of 384^3, line of sight z, 4 pairs: one row at a
     // time, not prefetched 786 us, so 625).
-    constexpr int QB = NF <= 3 ? 4 : 2;
+    // float64 takes half as many pairs a batch: the registers of 4 spill (three fields of 256^3, line of sight x, 4 pairs
+    // 192 -> 180 us, 2 pairs 141 -> 123; 20^3, line of sight z 12.0 -> 6.1).
+    constexpr int QB = (NF <= 3 ? 4 : 2) * 4 / (int)sizeof(R);
     constexpr bool PRE = NF <= 4;
     const int ncol = (u1 - u0) * (kzb1 - kzb0), nbat = (EU + 1 + QB - 1) / QB;
     struct Step {
