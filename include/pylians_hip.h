@@ -89,7 +89,9 @@ int pyl_stream_sync(void* stream);
  * Replaces MAS_library.MA and the per-scheme Cython functions NGP/CIC/TSC/PCS, NGPW/CICW/TSCW/PCSW,
  * CICW_d/NGPW_d (MAS_library.pyx:57-545).  pos: (n, axes) float32 row-major; W: (n,) float32 or
  * NULL; grid: dims^axes float32 (float64 with PYL_GRID_F64), accumulated into (MA never zeroes,
- * MAS_library.pyx:159-166).  For the 2-D Cython semantics pass PYL_DUP2D [| PYL_RENORM2D]. */
+ * MAS_library.pyx:159-166).  For the 2-D Cython semantics pass PYL_DUP2D [| PYL_RENORM2D].  2-D grids and
+ * 3-D grids whose edge is no multiple of 16 may be filled on several streams and from several threads at once,
+ * hipStreamPerThread included (their workspaces belong to the stream). */
 int pyl_mas_deposit(const float* pos, const float* W, int64_t n, int axes, int dims, double BoxSize,
                     int scheme, int flags, void* grid, void* stream);
 

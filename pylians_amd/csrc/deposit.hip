@@ -225,15 +225,18 @@ int deposit(const float* pos, const float* W, int64_t n, int axes, int dims, dou
         if (map && !capturing) {
             const bool dup = flags & DEP_DUP2D;
             StreamScope scope(st);
-            const int rc = deposit_map(pos, W, n, dims, BoxSize, scheme, f64, (flags & DEP_ZERO) != 0,
-                                       dup ? (double)scheme : 1.0,
-                                       dup && (flags & DEP_RENORM2D) && scheme > 1 ? (double)scheme : 0.0, grid, st);
+            const int rc = !scope.ok ? (int)E_ALLOC
+                                     : deposit_map(pos, W, n, dims, BoxSize, scheme, f64, (flags & DEP_ZERO) != 0,
+                                                   dup ? (double)scheme : 1.0,
+                                                   dup && (flags & DEP_RENORM2D) && scheme > 1 ? (double)scheme : 0.0,
+                                                   grid, st);
             if (rc != E_ALLOC) return rc;   // no room for the records: the direct kernel
         }
         if (ragged && !capturing) {
             StreamScope scope(st);
-            const int rc = deposit_binned(pos, W, n, dims, BoxSize, scheme, f64, mode, 1.0, grid, nullptr, 0.0, st, rsd,
-                                          PRESORT_PROBE, acc_mode(flags));
+            const int rc = !scope.ok ? (int)E_ALLOC
+                                     : deposit_binned(pos, W, n, dims, BoxSize, scheme, f64, mode, 1.0, grid, nullptr,
+                                                      0.0, st, rsd, PRESORT_PROBE, acc_mode(flags));
             if (rc != E_ALLOC) return rc;   // no room for the buckets (nothing has touched the grid): the direct kernel
         }
     }

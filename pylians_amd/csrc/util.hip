@@ -4,6 +4,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "common.hpp"
@@ -252,16 +253,25 @@ size_t ws_arena_bytes(const WsArena* a) {
     return s;
 }
 
-// Workspaces of the deposits that may run on several streams at once (stream_ws).  At most STREAM_WS
-// sets are kept; a further stream takes the place of the one used longest ago.
+// Workspaces of the deposits that may run on several streams at once (StreamScope).  At most STREAM_WS
+// sets are kept; a further stream takes the place of the one used longest ago.  A stream's calls run in order, and its
+// handle comes back only after its work (hipStreamDestroy waits for it), so the handle names the set -- except
+// hipStreamPerThread, which is another queue in every thread: there the thread counts too, and as a thread's id may come
+// back as well, each call is ordered behind the last one by an event (which costs a call of 87 us 3, so not elsewhere).
 constexpr size_t STREAM_WS = 4;
 struct StreamWs {
     int dev;
     hipStream_t st;
-    std::mutex mu;   // held while a call queues its kernels
+    std::thread::id owner;       // hipStreamPerThread: the thread that passed it
+    std::mutex mu;               // held while a call queues its kernels
     WsArena* arena;
-    StreamWs(int d, hipStream_t s) : dev(d), st(s), arena(ws_arena_create()) {}
-    ~StreamWs() { ws_arena_destroy(arena); }
+    hipEvent_t done = nullptr;   // hipStreamPerThread: behind the last call's kernels
+    bool used = false;           // done is recorded
+    StreamWs(int d, hipStream_t s, std::thread::id o) : dev(d), st(s), owner(o), arena(ws_arena_create()) {}
+    ~StreamWs() {
+        ws_arena_destroy(arena);
+        if (done) (void)hipEventDestroy(done);
+    }
 };
 
 static std::shared_ptr<StreamWs> stream_ws(hipStream_t st) {
@@ -269,10 +279,11 @@ static std::shared_ptr<StreamWs> stream_ws(hipStream_t st) {
     static std::vector<std::shared_ptr<StreamWs>>* sets = new std::vector<std::shared_ptr<StreamWs>>();
     int dev = 0;
     (void)hipGetDevice(&dev);
+    const std::thread::id owner = st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
     std::shared_ptr<StreamWs> old;   // freed (and its work waited for) after the lock is given back
     std::lock_guard<std::mutex> lk(mu);
     for (size_t i = 0; i < sets->size(); ++i)
-        if ((*sets)[i]->dev == dev && (*sets)[i]->st == st) {
+        if ((*sets)[i]->dev == dev && (*sets)[i]->st == st && (*sets)[i]->owner == owner) {
             std::shared_ptr<StreamWs> w = (*sets)[i];
             sets->erase(sets->begin() + (long)i);
             sets->push_back(w);
@@ -282,19 +293,41 @@ static std::shared_ptr<StreamWs> stream_ws(hipStream_t st) {
         old = sets->front();
         sets->erase(sets->begin());
     }
-    sets->push_back(std::make_shared<StreamWs>(dev, st));
+    sets->push_back(std::make_shared<StreamWs>(dev, st, owner));
     return sets->back();
 }
 
-StreamScope::StreamScope(hipStream_t st) {
+// the set's last call is behind the event: later work on st waits for it
+static bool ws_order(StreamWs& w, hipStream_t st) {
+    hipError_t e = hipSuccess;
+    if (!w.done) e = hipEventCreateWithFlags(&w.done, hipEventDisableTiming | hipEventDisableSystemFence);
+    if (e == hipSuccess && w.used) e = hipStreamWaitEvent(st, w.done, 0);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
+StreamScope::StreamScope(hipStream_t s) : st(s) {
     if (t_arena) return;   // a graph's or a fixed arena: that one
     ws = stream_ws(st);
     ws->mu.lock();
+    if (st == hipStreamPerThread && !ws_order(*ws, st)) {
+        ws->mu.unlock();
+        ws.reset();
+        ok = false;
+        return;
+    }
     t_arena = ws->arena;
 }
 StreamScope::~StreamScope() {
     if (!ws) return;
     t_arena = nullptr;
+    if (st == hipStreamPerThread) {
+        ws->used = hipEventRecord(ws->done, st) == hipSuccess;
+        if (!ws->used) {   // nothing to order the next call behind: wait here
+            (void)hipGetLastError();
+            (void)hipStreamSynchronize(st);
+        }
+    }
     ws->mu.unlock();
 }
 

@@ -58,13 +58,19 @@ struct ArenaScope {
 };
 // While a StreamScope is alive on a thread, workspace() serves buffers that belong to the stream: for
 // calls that needed no workspace before (and so could run on several streams and threads at once).
-// Calls on one stream queue their kernels one after the other; the buffers of at most four streams are
-// kept, those of the stream used longest ago being freed for another one's.
+// Calls on one stream queue their kernels one after the other (hipStreamPerThread: one thread's calls); the buffers of
+// at most four streams are
+// kept, those of the stream used longest ago being freed for another one's.  ok: false when the runtime refused to order
+// the call behind the last one with its buffers; the caller then does without workspaces.
 struct StreamWs;
 struct StreamScope {
-    explicit StreamScope(hipStream_t st);
+    explicit StreamScope(hipStream_t s);
     ~StreamScope();
+    StreamScope(const StreamScope&) = delete;
+    StreamScope& operator=(const StreamScope&) = delete;
     std::shared_ptr<StreamWs> ws;
+    hipStream_t st;
+    bool ok = true;
 };
 
 // A pinned host buffer for one call's results, from a pool of at most PINNED_KEPT free ones (any thread or stream); given
