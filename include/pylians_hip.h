@@ -79,6 +79,11 @@ const char* pyl_last_error(void);
 int pyl_device_count(int* count);
 int pyl_dev_alloc(void** ptr, int64_t bytes);
 int pyl_dev_free(void* ptr);
+/* Frees what the library keeps for later calls of pyl_mas_deposit on 2-D grids (8 to 12 bytes a particle of the largest
+ * call) and on 3-D grids whose edge is no multiple of 16 (64 to 80 bytes a particle), up to four sets a device, and the
+ * host buffers of pyl_pk_host and pyl_pk_particles_host.  Waits for the device; later calls allocate again.  The
+ * library does the first part by itself before one of its own allocations fails. */
+int pyl_release_workspaces(void);
 int pyl_memcpy_h2d(void* dst, const void* src, int64_t bytes, void* stream);
 int pyl_memcpy_d2h(void* dst, const void* src, int64_t bytes, void* stream);
 int pyl_memcpy_d2d(void* dst, const void* src, int64_t bytes, void* stream);

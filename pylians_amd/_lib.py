@@ -44,6 +44,7 @@ SIGNATURES = {
     "pyl_device_count": [_vp],
     "pyl_dev_alloc": [_vp, _i64],
     "pyl_dev_free": [_vp],
+    "pyl_release_workspaces": [],
     "pyl_memcpy_h2d": [_vp, _vp, _i64, _vp],
     "pyl_memcpy_d2h": [_vp, _vp, _i64, _vp],
     "pyl_memcpy_d2d": [_vp, _vp, _i64, _vp],
@@ -237,13 +238,14 @@ def _pool_give(ptr_, nbytes):
 
 
 def release_pool():
-    """Free the device buffers kept for reuse."""
+    """Free the device buffers kept for reuse, the library's stream workspaces among them."""
     global _POOL_BYTES
     for nbytes, lst in _POOL.items():
         for p in lst:
             lib().pyl_dev_free(_c.c_void_p(p))
     _POOL.clear()
     _POOL_BYTES = 0
+    check(lib().pyl_release_workspaces())
 
 
 class DevArray:

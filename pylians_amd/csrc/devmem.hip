@@ -89,12 +89,17 @@ extern "C" int pyl_dev_alloc(void** ptr, int64_t bytes) {
     PYL_CHECK(ptr && bytes >= 0, E_ARG, "bad allocation request");
     *ptr = nullptr;
     if (bytes == 0) return OK;
-    if (hipMalloc(ptr, (size_t)bytes) != hipSuccess) {
-        (void)hipGetLastError();
+    if (device_alloc(ptr, (size_t)bytes) != hipSuccess) {
         *ptr = nullptr;
         set_error("device allocation of %lld bytes failed", (long long)bytes);
         return E_ALLOC;
     }
+    return OK;
+}
+
+extern "C" int pyl_release_workspaces(void) {
+    stream_ws_release(true);
+    pinned_release();
     return OK;
 }
 

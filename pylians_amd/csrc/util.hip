@@ -101,6 +101,17 @@ static void* carve(WsArena* a, size_t bytes, int* rc) {
     return a->base + at;
 }
 
+hipError_t device_alloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        stream_ws_release(false);
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc) {
     if (e.first) {
         hipDeviceSynchronize();
@@ -109,8 +120,7 @@ static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc) {
         e.second = 0;
     }
     size_t want = bytes < 256 ? 256 : bytes;
-    if (hipMalloc(&e.first, want) != hipSuccess) {
-        (void)hipGetLastError();
+    if (device_alloc(&e.first, want) != hipSuccess) {
         e.first = nullptr;
         set_error("workspace allocation of %zu bytes failed", want);
         *rc = E_ALLOC;
@@ -253,79 +263,120 @@ size_t ws_arena_bytes(const WsArena* a) {
     return s;
 }
 
-// Workspaces of the deposits that may run on several streams at once (StreamScope).  At most STREAM_WS
-// sets are kept; a further stream takes the place of the one used longest ago.  A stream's calls run in order, and its
-// handle comes back only after its work (hipStreamDestroy waits for it), so the handle names the set -- except
-// hipStreamPerThread, which is another queue in every thread: there the thread counts too, and as a thread's id may come
-// back as well, each call is ordered behind the last one by an event (which costs a call of 87 us 3, so not elsewhere).
+// Workspaces of the deposits that may run on several streams at once (StreamScope): at most STREAM_WS sets a device.  A
+// further stream takes over the set used longest ago: nothing is freed and the host does not wait, its kernels run
+// behind the event of that set's last call.  A stream's own calls run in order and need no event (it costs a call of
+// 87 us 3), and a handle comes back only after its work (hipStreamDestroy waits for it), so the handle names the queue --
+// except hipStreamPerThread, which is another queue in every thread: there the thread counts too, and as a
+// thread's id may come back as well, its calls always have the event.
 constexpr size_t STREAM_WS = 4;
+struct Queue {
+    hipStream_t st;
+    std::thread::id owner;   // hipStreamPerThread: the thread that passed it
+    explicit Queue(hipStream_t s) : st(s) {
+        if (s == hipStreamPerThread) owner = std::this_thread::get_id();
+    }
+    bool operator==(const Queue& o) const { return st == o.st && owner == o.owner; }
+};
 struct StreamWs {
     int dev;
-    hipStream_t st;
-    std::thread::id owner;       // hipStreamPerThread: the thread that passed it
-    std::mutex mu;               // held while a call queues its kernels
+    Queue q;                     // whose set it is (under the pool's mutex)
+    std::mutex mu;               // held while a call queues its kernels; guards what follows
     WsArena* arena;
-    hipEvent_t done = nullptr;   // hipStreamPerThread: behind the last call's kernels
-    bool used = false;           // done is recorded
-    StreamWs(int d, hipStream_t s, std::thread::id o) : dev(d), st(s), owner(o), arena(ws_arena_create()) {}
+    Queue last;                  // queue of the last call
+    enum { FREE, OPEN, MARKED } state = FREE;   // no call; a call without an event behind it; with
+    hipEvent_t done = nullptr;
+    StreamWs(int d, const Queue& k) : dev(d), q(k), arena(ws_arena_create()), last(k) {}
     ~StreamWs() {
         ws_arena_destroy(arena);
         if (done) (void)hipEventDestroy(done);
     }
 };
 
-static std::shared_ptr<StreamWs> stream_ws(hipStream_t st) {
-    static std::mutex mu;
-    static std::vector<std::shared_ptr<StreamWs>>* sets = new std::vector<std::shared_ptr<StreamWs>>();
+namespace {
+struct StreamPool {
+    std::mutex mu;
+    std::vector<std::shared_ptr<StreamWs>> sets;   // in the order of their last use
+};
+StreamPool& stream_pool() {
+    static StreamPool* p = new StreamPool();   // outlives every caller
+    return *p;
+}
+}  // namespace
+
+// the set of a queue; shared: whether another queue has one too (and may take this one over)
+static std::shared_ptr<StreamWs> stream_ws(hipStream_t st, bool* shared) {
+    StreamPool& P = stream_pool();
     int dev = 0;
     (void)hipGetDevice(&dev);
-    const std::thread::id owner = st == hipStreamPerThread ? std::this_thread::get_id() : std::thread::id();
-    std::shared_ptr<StreamWs> old;   // freed (and its work waited for) after the lock is given back
-    std::lock_guard<std::mutex> lk(mu);
-    for (size_t i = 0; i < sets->size(); ++i)
-        if ((*sets)[i]->dev == dev && (*sets)[i]->st == st && (*sets)[i]->owner == owner) {
-            std::shared_ptr<StreamWs> w = (*sets)[i];
-            sets->erase(sets->begin() + (long)i);
-            sets->push_back(w);
-            return w;
-        }
-    if (sets->size() >= STREAM_WS) {
-        old = sets->front();
-        sets->erase(sets->begin());
+    const Queue q(st);
+    std::lock_guard<std::mutex> lk(P.mu);
+    size_t n = 0, oldest = P.sets.size(), own = P.sets.size();
+    for (size_t i = P.sets.size(); i-- > 0;) {
+        if (P.sets[i]->dev != dev) continue;
+        ++n;
+        oldest = i;
+        if (P.sets[i]->q == q) own = i;
     }
-    sets->push_back(std::make_shared<StreamWs>(dev, st, owner));
-    return sets->back();
+    if (own == P.sets.size() && n >= STREAM_WS) {
+        own = oldest;
+        P.sets[own]->q = q;
+    }
+    std::shared_ptr<StreamWs> w;
+    if (own < P.sets.size()) {
+        w = P.sets[own];
+        P.sets.erase(P.sets.begin() + (long)own);
+    } else {
+        w = std::make_shared<StreamWs>(dev, q);
+        ++n;
+    }
+    P.sets.push_back(w);
+    *shared = n > 1;
+    return w;
 }
 
-// the set's last call is behind the event: later work on st waits for it
-static bool ws_order(StreamWs& w, hipStream_t st) {
-    hipError_t e = hipSuccess;
-    if (!w.done) e = hipEventCreateWithFlags(&w.done, hipEventDisableTiming | hipEventDisableSystemFence);
-    if (e == hipSuccess && w.used) e = hipStreamWaitEvent(st, w.done, 0);
-    if (e != hipSuccess) (void)hipGetLastError();
-    return e == hipSuccess;
+void stream_ws_release(bool all) {
+    std::vector<std::shared_ptr<StreamWs>> out;   // freed after the lock is given back; a set in use, by its last user
+    StreamPool& P = stream_pool();
+    std::lock_guard<std::mutex> lk(P.mu);
+    for (size_t i = P.sets.size(); i-- > 0;)
+        if (all || P.sets[i].use_count() == 1) {
+            out.push_back(P.sets[i]);
+            P.sets.erase(P.sets.begin() + (long)i);
+        }
 }
 
 StreamScope::StreamScope(hipStream_t s) : st(s) {
     if (t_arena) return;   // a graph's or a fixed arena: that one
-    ws = stream_ws(st);
+    ws = stream_ws(st, &mark);
+    mark = mark || st == hipStreamPerThread;
     ws->mu.lock();
-    if (st == hipStreamPerThread && !ws_order(*ws, st)) {
+    const Queue q(st);
+    hipError_t e = hipSuccess;
+    if (mark && !ws->done) e = hipEventCreateWithFlags(&ws->done, hipEventDisableTiming | hipEventDisableSystemFence);
+    if (e == hipSuccess && ws->state != StreamWs::FREE && (!(ws->last == q) || st == hipStreamPerThread))
+        // OPEN: the only set of its time when it was used last; the first to take it over waits
+        e = ws->state == StreamWs::MARKED ? hipStreamWaitEvent(st, ws->done, 0) : hipDeviceSynchronize();
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
         ws->mu.unlock();
         ws.reset();
         ok = false;
         return;
     }
+    ws->last = q;
     t_arena = ws->arena;
 }
 StreamScope::~StreamScope() {
     if (!ws) return;
     t_arena = nullptr;
-    if (st == hipStreamPerThread) {
-        ws->used = hipEventRecord(ws->done, st) == hipSuccess;
-        if (!ws->used) {   // nothing to order the next call behind: wait here
+    ws->state = StreamWs::OPEN;
+    if (mark) {
+        if (hipEventRecord(ws->done, st) == hipSuccess) {
+            ws->state = StreamWs::MARKED;
+        } else {   // nothing to order the next call behind: wait here
             (void)hipGetLastError();
-            (void)hipStreamSynchronize(st);
+            if (hipStreamSynchronize(st) == hipSuccess) ws->state = StreamWs::FREE;
         }
     }
     ws->mu.unlock();
@@ -363,6 +414,15 @@ int PinnedScope::take(size_t want) {
     }
     bytes = b;
     return OK;
+}
+
+void pinned_release() {
+    std::vector<std::pair<void*, size_t>> out;
+    {
+        std::lock_guard<std::mutex> lk(g_pin_mu);
+        out.swap(pin_free());
+    }
+    for (auto& e : out) (void)hipHostFree(e.first);
 }
 
 PinnedScope::~PinnedScope() {

@@ -58,10 +58,9 @@ struct ArenaScope {
 };
 // While a StreamScope is alive on a thread, workspace() serves buffers that belong to the stream: for
 // calls that needed no workspace before (and so could run on several streams and threads at once).
-// Calls on one stream queue their kernels one after the other (hipStreamPerThread: one thread's calls); the buffers of
-// at most four streams are
-// kept, those of the stream used longest ago being freed for another one's.  ok: false when the runtime refused to order
-// the call behind the last one with its buffers; the caller then does without workspaces.
+// Calls on one stream queue their kernels one after the other (hipStreamPerThread: one thread's calls).  Four sets of
+// buffers are kept; a further stream takes over the one used longest ago, and its kernels wait on the device
+// for that set's last call.  ok: false when the runtime refused that order; the caller then does without workspaces.
 struct StreamWs;
 struct StreamScope {
     explicit StreamScope(hipStream_t s);
@@ -70,8 +69,13 @@ struct StreamScope {
     StreamScope& operator=(const StreamScope&) = delete;
     std::shared_ptr<StreamWs> ws;
     hipStream_t st;
+    bool mark = false;   // an event goes behind the call
     bool ok = true;
 };
+// gives the sets back to the device: those that no call is using, or all (a set in use when its call has queued)
+void stream_ws_release(bool all);
+// hipMalloc that gives idle stream workspaces back before it fails
+hipError_t device_alloc(void** p, size_t bytes);
 
 // A pinned host buffer for one call's results, from a pool of at most PINNED_KEPT free ones (any thread or stream); given
 // back by the destructor, so only after the copies into it are done.
@@ -81,5 +85,6 @@ struct PinnedScope {
     int take(size_t want);
     ~PinnedScope();
 };
+void pinned_release();   // frees the pool's free buffers
 
 }  // namespace pyl

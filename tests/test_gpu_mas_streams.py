@@ -112,6 +112,42 @@ def test_a_stream_that_is_gone(gpu):
             _equal(g[j], c)
 
 
+def test_more_streams_than_kept_workspaces(gpu):
+    """Calls that go round more streams than there are sets of workspaces do not wait for the device, and what the sets
+    hold is given back on request."""
+    from pylians_amd import _lib
+    cases = [_case(2, 6), _case(3, 7)]
+    st = [torch.cuda.Stream() for _ in range(6)]
+    grids = _grids(cases)
+    for _ in range(2):   # sizes every set
+        for s in st:
+            for j, c in enumerate(cases):
+                assert _deposit(c, grids[j], s.cuda_stream) == 0
+    torch.cuda.synchronize()
+    a = torch.zeros(8192, 8192, device="cuda")
+    torch.mm(a, a)
+    turn = [_grids(cases) for _ in st]
+    busy, ev = torch.cuda.Stream(), torch.cuda.Event()
+    with torch.cuda.stream(busy):
+        for _ in range(40):
+            a = torch.mm(a, a)
+        ev.record()
+    for g, s in zip(turn, st):
+        for j, c in enumerate(cases):
+            assert _deposit(c, g[j], s.cuda_stream) == 0
+    assert not ev.query()
+    torch.cuda.synchronize()
+    for g in turn:
+        for j, c in enumerate(cases):
+            _equal(g[j], c)
+    held = torch.cuda.mem_get_info()[0]
+    _lib.release_pool()
+    assert torch.cuda.mem_get_info()[0] - held >= 4 * 60 * cases[1][0].shape[0]
+    assert _deposit(cases[1], grids[1], st[0].cuda_stream) == 0
+    torch.cuda.synchronize()
+    _equal(grids[1], cases[1])
+
+
 @pytest.mark.parametrize("axes", [2, 3])
 def test_captured(gpu, axes):
     """Inside a capture the same call takes the direct kernel (float32 atomics); its replays leave the oracle's grid."""
