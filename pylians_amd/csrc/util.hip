@@ -85,7 +85,8 @@ struct WsArena {
     // fixed arena: every slot and table is carved from [base, base + cap) in request order
     char* base = nullptr;
     size_t cap = 0, used = 0;
-    hipStream_t st = nullptr;
+    hipStream_t st = nullptr;   // fixed arena: of its uploads; a stream's set: the stream in a StreamScope
+    bool of_stream = false;     // a stream's set: all that used its buffers is on st or ordered before it
 };
 static thread_local WsArena* t_arena = nullptr;
 
@@ -112,10 +113,15 @@ hipError_t device_alloc(void** p, size_t bytes) {
     return e;
 }
 
-static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc) {
+static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc, const WsArena* a = nullptr) {
     if (e.first) {
-        hipDeviceSynchronize();
-        hipFree(e.first);
+        const hipError_t w = a && a->of_stream ? hipStreamSynchronize(a->st) : hipDeviceSynchronize();
+        if (w != hipSuccess || hipFree(e.first) != hipSuccess) {
+            (void)hipGetLastError();
+            set_error("a workspace in use could not be freed");
+            *rc = E_ALLOC;
+            return nullptr;
+        }
         e.first = nullptr;
         e.second = 0;
     }
@@ -159,7 +165,7 @@ void* workspace(int slot, size_t bytes, int* rc) {
             *rc = E_ALLOC;
             return nullptr;
         }
-        return grow(e, bytes, rc);
+        return grow(e, bytes, rc, a);
     }
     std::lock_guard<std::mutex> lk(mu);
     auto& e = ws[std::make_pair(dev, slot)];
@@ -286,7 +292,7 @@ struct StreamWs {
     Queue last;                  // queue of the last call
     enum { FREE, OPEN, MARKED } state = FREE;   // no call; a call without an event behind it; with
     hipEvent_t done = nullptr;
-    StreamWs(int d, const Queue& k) : dev(d), q(k), arena(ws_arena_create()), last(k) {}
+    StreamWs(int d, const Queue& k) : dev(d), q(k), arena(ws_arena_create()), last(k) { arena->of_stream = true; }
     ~StreamWs() {
         ws_arena_destroy(arena);
         if (done) (void)hipEventDestroy(done);
@@ -348,6 +354,8 @@ void stream_ws_release(bool all) {
 
 StreamScope::StreamScope(hipStream_t s) : st(s) {
     if (t_arena) return;   // a graph's or a fixed arena: that one
+    // another stream may be capturing: these calls touch nothing of its graph, and would end its capture otherwise
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
     ws = stream_ws(st, &mark);
     mark = mark || st == hipStreamPerThread;
     ws->mu.lock();
@@ -361,10 +369,12 @@ StreamScope::StreamScope(hipStream_t s) : st(s) {
         (void)hipGetLastError();
         ws->mu.unlock();
         ws.reset();
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
         ok = false;
         return;
     }
     ws->last = q;
+    ws->arena->st = st;
     t_arena = ws->arena;
 }
 StreamScope::~StreamScope() {
@@ -380,6 +390,8 @@ StreamScope::~StreamScope() {
         }
     }
     ws->mu.unlock();
+    ws.reset();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 
 ArenaScope::ArenaScope(WsArena* a) : prev(t_arena) { t_arena = a; }

@@ -69,6 +69,7 @@ struct StreamScope {
     StreamScope& operator=(const StreamScope&) = delete;
     std::shared_ptr<StreamWs> ws;
     hipStream_t st;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;   // the thread's own while the scope is alive
     bool mark = false;   // an event goes behind the call
     bool ok = true;
 };

@@ -164,3 +164,26 @@ def test_captured(gpu, axes):
         assert _deposit(c, e, torch.cuda.current_stream().cuda_stream) == 0
         _equal(e, c)
         assert torch.allclose(g, e, rtol=1e-4, atol=1e-4)
+
+
+@pytest.mark.parametrize("axes", [2, 3])
+def test_beside_a_capture(gpu, axes):
+    """A call on one stream leaves a capture on another as it is, also where its workspaces are made or grow."""
+    from pylians_amd import _lib
+    small, large = _case(axes, 1), _case(axes, 9)
+    grids = _grids([small, large])
+    _lib.release_pool()
+    x, side, graph = torch.zeros(4, device="cuda"), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x += 1
+        for c, g in zip((small, large), grids):
+            assert _deposit(c, g, side.cuda_stream) == 0
+        x += 1
+    side.synchronize()
+    for c, g in zip((small, large), grids):
+        o = c[2]
+        assert np.allclose(g.cpu().numpy(), o, rtol=1e-4, atol=1e-4)   # (either route)
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(x, torch.full_like(x, 2.0 * (i + 1)))
