@@ -1132,16 +1132,24 @@ int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double
             ps = Presort();
         }
     }
-    if (f64) {
-        const int a64 = dense_acc(ACC_F64, scheme, n, dims);
-        if (mode == OUT_ACC) return dispatch_s<double, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, ps);
-        if (mode == OUT_SET) return dispatch_s<double, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, ps);
-        return dispatch_s<double, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, ps);
-    }
-    acc = dense_acc(acc, scheme, n, dims);
-    if (mode == OUT_ACC) return dispatch_s<float, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc, ps);
-    if (mode == OUT_SET) return dispatch_s<float, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc, ps);
-    return dispatch_s<float, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, acc, ps);
+    auto run = [&](const Presort& q) -> int {
+        if (f64) {
+            const int a64 = dense_acc(ACC_F64, scheme, n, dims);
+            if (mode == OUT_ACC) return dispatch_s<double, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, q);
+            if (mode == OUT_SET) return dispatch_s<double, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, q);
+            return dispatch_s<double, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a64, q);
+        }
+        const int a32 = dense_acc(acc, scheme, n, dims);
+        if (mode == OUT_ACC) return dispatch_s<float, OUT_ACC>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a32, q);
+        if (mode == OUT_SET) return dispatch_s<float, OUT_SET>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a32, q);
+        return dispatch_s<float, OUT_DELTA>(pos, W, n, dims, BoxSize, scheme, mult, grid, dmass, mass, st, rsd, a32, q);
+    };
+    const int rc = run(ps);
+    if (rc != E_ALLOC || !ps.sel) return rc;
+    // the buckets do not fit beside the grouped copy: without it
+    workspace_drop(WS_STAGE);
+    workspace_drop(WS_SUP);
+    return run(Presort());
 }
 
 // ------------------------------------------------------------------ batched deposit

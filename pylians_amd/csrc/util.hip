@@ -113,18 +113,22 @@ hipError_t device_alloc(void** p, size_t bytes) {
     return e;
 }
 
-static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc, const WsArena* a = nullptr) {
-    if (e.first) {
-        const hipError_t w = a && a->of_stream ? hipStreamSynchronize(a->st) : hipDeviceSynchronize();
-        if (w != hipSuccess || hipFree(e.first) != hipSuccess) {
-            (void)hipGetLastError();
-            set_error("a workspace in use could not be freed");
-            *rc = E_ALLOC;
-            return nullptr;
-        }
-        e.first = nullptr;
-        e.second = 0;
+// frees a buffer once the work that may use it is done; a buffer that cannot be freed is kept
+static bool give_back(std::pair<void*, size_t>& e, int* rc, const WsArena* a) {
+    if (!e.first) return true;
+    const hipError_t w = a && a->of_stream ? hipStreamSynchronize(a->st) : hipDeviceSynchronize();
+    if (w != hipSuccess || hipFree(e.first) != hipSuccess) {
+        (void)hipGetLastError();
+        set_error("a workspace in use could not be freed");
+        *rc = E_ALLOC;
+        return false;
     }
+    e = std::make_pair(nullptr, (size_t)0);
+    return true;
+}
+
+static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc, const WsArena* a = nullptr) {
+    if (!give_back(e, rc, a)) return nullptr;
     size_t want = bytes < 256 ? 256 : bytes;
     if (device_alloc(&e.first, want) != hipSuccess) {
         e.first = nullptr;
@@ -136,9 +140,24 @@ static void* grow(std::pair<void*, size_t>& e, size_t bytes, int* rc, const WsAr
     return e.first;
 }
 
+static std::mutex g_ws_mu;
+static std::map<std::pair<int, int>, std::pair<void*, size_t>>& shared_ws() {
+    static auto* m = new std::map<std::pair<int, int>, std::pair<void*, size_t>>();   // outlives every caller
+    return *m;
+}
+
+void workspace_drop(int slot) {
+    int rc = OK, dev = 0;
+    if (WsArena* a = t_arena) {
+        if (!a->base && !a->sealed) give_back(a->slots[slot], &rc, a);
+        return;
+    }
+    if (hipGetDevice(&dev) != hipSuccess) return;
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    give_back(shared_ws()[std::make_pair(dev, slot)], &rc, nullptr);
+}
+
 void* workspace(int slot, size_t bytes, int* rc) {
-    static std::mutex mu;
-    static std::map<std::pair<int, int>, std::pair<void*, size_t>> ws;
     *rc = OK;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) {
@@ -167,8 +186,8 @@ void* workspace(int slot, size_t bytes, int* rc) {
         }
         return grow(e, bytes, rc, a);
     }
-    std::lock_guard<std::mutex> lk(mu);
-    auto& e = ws[std::make_pair(dev, slot)];
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    auto& e = shared_ws()[std::make_pair(dev, slot)];
     if (e.second >= bytes && e.first) return e.first;
     return grow(e, bytes, rc);
 }
