@@ -206,7 +206,7 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
                 if (HASW) r[3] = w[k];
             } else {
                 const unsigned o = atomicAdd(a.ov_count, 1u);
-                a.ov_idx[o] = p;
+                a.ov_idx[o] = (unsigned long long)(idx - (unsigned)scap[c]) << 32 | (unsigned long long)p;
                 a.ov_key[o] = (unsigned)key[k];
             }
         }
@@ -230,37 +230,33 @@ __global__ __launch_bounds__(BT) void k_bin_b(const BinArgs* __restrict__ tab,
     bin_body<S, HASW, 2, false>(tab[bj_], blk_);
 }
 
-// Overflow grouping in one launch: the first workgroup to arrive counts and scans, then all copy the records.  A tile's
-// records are what its class fills exceed their capacities by, so the list itself is not counted.  The others wait for
-// a workgroup that is running by then (it took its ticket) and waits for none, so the wait ends whatever else the card
-// runs.  Nothing overflowed (every group is empty and k_tile reads no offset): one read and out, 4.7 us where three
-// launches took 14.
-__device__ __forceinline__ void ov_scan(const OvArgs& a) {
-    __shared__ unsigned part[OT];
-    const int tid = threadIdx.x, n = a.ntiles;
-    const int per = (n + OT - 1) / OT;
-    const int lo = tid * per, hi = min(n, lo + per);
-    unsigned s = 0;
-#pragma unroll 4
-    for (int i = lo; i < hi; ++i) {
-        unsigned f[8], k = 0u;
-        const uint4 fa = ((const uint4*)a.fill)[2 * (long long)i], fb = ((const uint4*)a.fill)[2 * (long long)i + 1];
-        f[0] = fa.x, f[1] = fa.y, f[2] = fa.z, f[3] = fa.w, f[4] = fb.x, f[5] = fb.y, f[6] = fb.z, f[7] = fb.w;
+// Overflow grouping in one launch: the first workgroup to arrive counts and scans, then all that have records copy
+// them.  A tile's records are what its class fills exceed their capacities by, and a record's place among them is its
+// index in the segment beyond the capacity, so the list itself is not counted and nothing is added to.  The others wait
+// for a workgroup that is running by then (it took its ticket) and waits for none, so the wait ends whatever else the
+// card runs; workgroups past the end of the list leave at once.  Nothing overflowed (every group is empty and k_tile
+// reads no offset): one read and out, 4.7 us where three launches took 14.  One thread of a waiting workgroup makes its
+// fence (the barrier orders the others behind it).
+__device__ __forceinline__ unsigned ov_over(const OvArgs& a, long long tile, unsigned (&k)[8]) {
+    const uint4 fa = ((const uint4*)a.fill)[2 * tile], fb = ((const uint4*)a.fill)[2 * tile + 1];
+    k[0] = fa.x, k[1] = fa.y, k[2] = fa.z, k[3] = fa.w, k[4] = fb.x, k[5] = fb.y, k[6] = fb.z, k[7] = fb.w;
+    unsigned s = 0u;
 #pragma unroll
-        for (int c = 0; c < 8; ++c) k += f[c] - min(f[c], (unsigned)a.cap[c]);
-        a.ocnt[i] = k;
-        s += k;
+    for (int c = 0; c < 8; ++c) s += k[c] -= min(k[c], (unsigned)a.cap[c]);
+    return s;
+}
+// thread t takes the tiles t, t + OT, ...: their groups follow one another in that order
+__device__ __forceinline__ void ov_scan(const OvArgs& a) {
+    __shared__ unsigned wsum[OT / 64];
+    const int tid = threadIdx.x, n = a.ntiles;
+    unsigned k[8], s = 0u;
+    for (int i = tid; i < n; i += OT) {
+        const unsigned o = ov_over(a, i, k);
+        a.ocnt[i] = o;
+        s += o;
     }
-    part[tid] = s;
-    __syncthreads();
-    for (int d = 1; d < OT; d <<= 1) {
-        unsigned v = tid >= d ? part[tid - d] : 0u;
-        __syncthreads();
-        part[tid] += v;
-        __syncthreads();
-    }
-    unsigned run = tid ? part[tid - 1] : 0u;
-    for (int i = lo; i < hi; ++i) {
+    unsigned run = block_exscan(s, wsum);
+    for (int i = tid; i < n; i += OT) {
         a.ooff[i] = run;
         run += a.ocnt[i];
     }
@@ -271,7 +267,7 @@ __device__ __forceinline__ void ov_body(const OvArgs& a, Blk B) {
     constexpr int R = HASW ? 4 : 3;
     __shared__ unsigned ticket;
     const long long n = *a.ov_count;
-    if (n == 0) return;
+    if ((long long)B.x * OT >= n) return;
     if (threadIdx.x == 0) ticket = atomicAdd(&a.turn[0], 1u);
     __syncthreads();
     if (ticket == 0u) {
@@ -280,20 +276,25 @@ __device__ __forceinline__ void ov_body(const OvArgs& a, Blk B) {
         __syncthreads();
         if (threadIdx.x == 0) __hip_atomic_store(&a.turn[1], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     } else {
-        if (threadIdx.x == 0)
+        if (threadIdx.x == 0) {
             // (an acquire for every look would keep emptying the caches that the scan works in)
             while (__hip_atomic_load(&a.turn[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0u)
-                __builtin_amdgcn_s_sleep(32);
+                __builtin_amdgcn_s_sleep(8);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
         __syncthreads();
-        __threadfence();
     }
     const bool sel = a.sel && *a.sel;
     const float* __restrict__ pos = sel ? a.spos : a.pos;
     const float* __restrict__ W = sel ? a.sw : a.W;
     for (long long i = (long long)B.x * OT + threadIdx.x; i < n; i += (long long)B.gx * OT) {
-        const unsigned key = a.ov_key[i], t = key >> 3;
-        const long long p = a.ov_idx[i];
-        const unsigned s = a.ooff[t] + atomicAdd(&a.ocur[t], 1u);
+        const unsigned key = a.ov_key[i], t = key >> 3, cls = key & 7u;
+        const unsigned long long e = a.ov_idx[i];
+        const long long p = (long long)(e & 0xffffffffull);
+        unsigned k[8], s = a.ooff[t] + (unsigned)(e >> 32);
+        ov_over(a, t, k);
+#pragma unroll
+        for (unsigned c = 0; c < 8; ++c) s += c < cls ? k[c] : 0u;
         float* r = a.grouped + (long long)s * R;
         float c[3] = {pos[3 * p], pos[3 * p + 1], pos[3 * p + 2]};
         if (a.rsd.vel) c[a.rsd.axis] = rsd_shift(c[a.rsd.axis], a.rsd.vel[3 * p + a.rsd.axis], a.rsd.fac, a.rsd.box);
@@ -301,7 +302,7 @@ __device__ __forceinline__ void ov_body(const OvArgs& a, Blk B) {
         r[1] = c[1];
         r[2] = c[2];
         if (HASW) r[3] = W[p];
-        a.gcls[s] = key & 7u;
+        a.gcls[s] = cls;
     }
 }
 template <bool HASW>
@@ -913,7 +914,7 @@ struct Presort {
 struct Layout {
     int nt, cap[8], cofs[8];
     long long ntiles, CT;
-    size_t ncnt;   // counters: fill (8 ntiles) | ocnt | ocur | ooff (ntiles + 1) | ov_count | turn (2)
+    size_t ncnt;   // counters: fill (8 ntiles) | ocnt | ooff | ov_count | turn (2)
     size_t cnt_bytes, bucket_bytes, ov_bytes;
 };
 
@@ -932,10 +933,10 @@ static int layout_of(int64_t n, int dims, int S, bool hasw, Layout* L) {
         L->cofs[c] = (int)L->CT;
         L->CT += v;
     }
-    L->ncnt = 11 * (size_t)L->ntiles + 4;
+    L->ncnt = 10 * (size_t)L->ntiles + 4;
     L->cnt_bytes = sizeof(unsigned) * L->ncnt + 64;
     L->bucket_bytes = sizeof(float) * (size_t)L->ntiles * L->CT * R;
-    // overflow: ov_idx (8n) | ov_key (4n) | gcls (4n) | grouped (4Rn)
+    // overflow: ov_idx (8n: particle index, and the record's index beyond its segment in the upper half) | ov_key (4n) | gcls (4n) | grouped (4Rn)
     L->ov_bytes = (size_t)n * (16 + 4 * R) + 256;
     return OK;
 }
@@ -954,13 +955,12 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
     const size_t ncnt = L.ncnt;
     unsigned* cnt = (unsigned*)workspace(WS_BINS, L.cnt_bytes, &rc);
     if (rc) return rc;
-    unsigned *fill = cnt, *ocnt = cnt + 8 * ntiles, *ocur = cnt + 9 * ntiles, *ooff = cnt + 10 * ntiles,
-             *ov_count = cnt + 11 * ntiles + 1;
+    unsigned *fill = cnt, *ocnt = cnt + 8 * ntiles, *ooff = cnt + 9 * ntiles, *ov_count = cnt + 10 * ntiles;
     float* bucket = (float*)workspace(WS_AUX, L.bucket_bytes, &rc);
     if (rc) return rc;
     char* ov = (char*)workspace(WS_AUX2, L.ov_bytes, &rc);
     if (rc) return rc;
-    long long* ov_idx = (long long*)ov;
+    unsigned long long* ov_idx = (unsigned long long*)ov;
     unsigned* ov_key = (unsigned*)(ov + 8 * (size_t)n);
     unsigned* gcls = (unsigned*)(ov + 12 * (size_t)n);
     float* grouped = (float*)(ov + 16 * (size_t)n + 64);
@@ -991,7 +991,7 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
     }
     {
         StageTimer tm("deposit_overflow", st);
-        OvArgs oa{ov_count, ov_idx, ov_key, fill, {}, ocnt, ooff, ocur, ov_count + 1, pos, W, grouped, gcls, rsd,
+        OvArgs oa{ov_count, ov_idx, ov_key, fill, {}, ocnt, ooff, ov_count + 1, pos, W, grouped, gcls, rsd,
                   (int)ntiles, ps.sel, ps.pos, ps.W};
         for (int c = 0; c < 8; ++c) oa.cap[c] = cap[c];
         hipLaunchKernelGGL((k_ov<HASW>), dim3(OB), dim3(OT), 0, st, oa);
@@ -1187,9 +1187,8 @@ int binned_job_plan(const float* pos, const float* W, int64_t n, int dims, doubl
     char* ov = p;
     p += al256(L.ov_bytes);
     const long long ntiles = L.ntiles;
-    unsigned *fill = cnt, *ocnt = cnt + 8 * ntiles, *ocur = cnt + 9 * ntiles, *ooff = cnt + 10 * ntiles,
-             *ov_count = cnt + 11 * ntiles + 1;
-    long long* ov_idx = (long long*)ov;
+    unsigned *fill = cnt, *ocnt = cnt + 8 * ntiles, *ooff = cnt + 9 * ntiles, *ov_count = cnt + 10 * ntiles;
+    unsigned long long* ov_idx = (unsigned long long*)ov;
     unsigned* ov_key = (unsigned*)(ov + 8 * (size_t)n);
     unsigned* gcls = (unsigned*)(ov + 12 * (size_t)n);
     float* grouped = (float*)(ov + 16 * (size_t)n + 64);
@@ -1226,7 +1225,7 @@ int binned_job_plan(const float* pos, const float* W, int64_t n, int dims, doubl
     long long bb = (n + (long long)BT * KP - 1) / ((long long)BT * KP);
     if (bb > 2048) bb = 2048;
     j->bin_blocks = (unsigned)((bb + XCDS - 1) / XCDS * XCDS);
-    j->ov = OvArgs{ov_count, ov_idx, ov_key, fill, {}, ocnt, ooff, ocur, ov_count + 1, bpos, bW, grouped, gcls, Rsd(),
+    j->ov = OvArgs{ov_count, ov_idx, ov_key, fill, {}, ocnt, ooff, ov_count + 1, bpos, bW, grouped, gcls, Rsd(),
                    (int)ntiles};
     for (int c = 0; c < 8; ++c) j->ov.cap[c] = L.cap[c];
     j->tile_blocks = (unsigned)((ntiles + XCDS - 1) / XCDS * XCDS);

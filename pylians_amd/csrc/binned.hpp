@@ -20,7 +20,7 @@ struct BinArgs {
     long long CT;        // record slots per tile
     int cofs[8], cap[8]; // first slot and capacity of each class segment
     unsigned* ov_count;  // [1]
-    long long* ov_idx;   // [n]
+    unsigned long long* ov_idx;   // [n]
     unsigned* ov_key;    // [n]
     Rsd rsd;             // redshift-space shift of the positions (rsd.vel == nullptr: none)
     int agg = 0;         // runs of equal keys in consecutive lanes counted once (bin_agg)
@@ -50,13 +50,12 @@ struct TileArgs {
 
 struct OvArgs {
     const unsigned* ov_count;   // [1] records in the overflow list
-    const long long* ov_idx;    // particle index of each
+    const unsigned long long* ov_idx;   // particle index of each, its index beyond the segment's capacity << 32
     const unsigned* ov_key;     // (tile, class) key of each
     const unsigned* fill;       // [8 ntiles] records per (tile, class), overflow included
     int cap[8];                 // capacity of each class segment
     unsigned* ocnt;             // [ntiles] overflow records per tile
     unsigned* ooff;             // [ntiles] first grouped slot of each tile
-    unsigned* ocur;             // [ntiles] slots handed out
     unsigned* turn;             // [2] workgroups that arrived, 1 when the offsets are written
     const float* pos;
     const float* W;
