@@ -63,7 +63,7 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
     __shared__ int hkey[HT];
     __shared__ unsigned hcnt[HT];
     __shared__ int hused[BT * KP];   // slots that hold a key this step, in insertion order
-    __shared__ unsigned nused;
+    __shared__ unsigned nused, nov, ovbase;   // of the step: keys; records beyond their segments, and their first slot
     __shared__ int scap[8], scofs[8];
     const int tid = threadIdx.x;
     const bool grouped = a.sel && *a.sel;
@@ -77,7 +77,7 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
         hkey[i] = -1;
         hcnt[i] = 0u;
     }
-    if (tid == 0) nused = 0u;
+    if (tid == 0) nused = nov = 0u;
     __syncthreads();
     const long long nstep = (a.n + PS - 1) / PS;
     // particle k of this thread in a step: step * PS + k * BT + tid (coalesced for each k)
@@ -185,13 +185,21 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
         }
         __syncthreads();
         // one reservation per key of the step: its records go to [base, base + hcnt) of its segment;
-        // the base replaces the key in the slot
+        // the base replaces the key in the slot.  What lies beyond the segment gets consecutive slots of the
+        // overflow list, one reservation for the whole step (one atomic a record on that one counter took 1 ms for 4 M
+        // of 8 M clustered particles): the count becomes the key's first slot, less its first index there
         const unsigned nu = nused;
         for (unsigned i = tid; i < nu; i += BT) {
-            const int sl = hused[i];
-            hkey[sl] = (int)atomicAdd(&a.fill[hkey[sl]], hcnt[sl]);
+            const int sl = hused[i], k = hkey[sl];
+            const unsigned cnt = hcnt[sl], base = atomicAdd(&a.fill[k], cnt), first = max(base, (unsigned)scap[k & 7]);
+            hkey[sl] = (int)base;
+            if (base + cnt > first) hcnt[sl] = atomicAdd(&nov, base + cnt - first) - first;
         }
         __syncthreads();
+        if (nov) {
+            if (tid == 0) ovbase = atomicAdd(a.ov_count, nov);
+            __syncthreads();
+        }
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
             if (key[k] < 0) continue;
@@ -205,7 +213,7 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
                 r[2] = z[k];
                 if (HASW) r[3] = w[k];
             } else {
-                const unsigned o = atomicAdd(a.ov_count, 1u);
+                const unsigned o = ovbase + hcnt[slot[k]] + idx;
                 a.ov_idx[o] = (unsigned long long)(idx - (unsigned)scap[c]) << 32 | (unsigned long long)p;
                 a.ov_key[o] = (unsigned)key[k];
             }
@@ -216,7 +224,7 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
             hkey[sl] = -1;
             hcnt[sl] = 0u;
         }
-        if (tid == 0) nused = 0u;
+        if (tid == 0) nused = nov = 0u;
         __syncthreads();
     }
 }
