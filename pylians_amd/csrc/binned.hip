@@ -685,15 +685,16 @@ __global__ __launch_bounds__(TT) void k_tile_b(const TileArgs* __restrict__ tab,
 // ------------------------------------------------------------------ presort for unordered inputs
 // Particles in no spatial order give k_bin one key per particle: one global atomic each and 12-byte
 // scattered records.  The presort first groups them by supertile (whole columns of tiles, at most SUPMAX
-// groups): k_sup_count counts the groups of every workgroup's particles, k_sup_scan turns the counts into
-// each workgroup's first slot per group, and k_sup_scatter copies the particles there.  No global atomics:
+// groups): k_sup_count counts the groups of every workgroup's particles, k_sup_scatter turns the counts into
+// its workgroups' first slots per group and copies the particles there.  No global atomics:
 // with one global reservation per group and step instead, 3 M weighted particles took 46 + 46 us, most of
 // it in atomics on a hundred addresses.
 // k_bin then reads the grouped copy, where neighbouring particles share keys as in an ordered input.
 constexpr int PT = 1024;   // presort kernels: threads per workgroup
 constexpr int PKP = 8;    // particles per thread per step
-// particles from which the device looks for a spatial order (PRESORT_PROBE)
+// PRESORT_PROBE: particles, and (tile, class) keys of the grid, from which the device looks for a spatial order
 constexpr int64_t PROBE_MIN = 1 << 20;
+constexpr long long PROBE_KEYS = 512;
 // groups aimed at: more give k_bin fewer keys a step (3 M particles onto 320^3: 60 us with 128, 40 with 256, 29
 // with 512), fewer give the scatter longer runs (24 / 24 / 25 us)
 constexpr int SUPGROUPS = 512;
@@ -726,28 +727,36 @@ __device__ __forceinline__ void sup_range(const SupArgs& a, unsigned bx, long lo
 }
 
 // a.sel: the particles are grouped only when they are in no spatial order.  Every workgroup looks at
-// the same PT pairs of consecutive particles (read from L2 after the first) and takes them for unordered
-// when more than half of the pairs lie in different tiles (lattice order: 1 pair in TILE, or a few with large
-// displacements; unordered: all but one in ntiles).  Returns whether to group; workgroup 0 notes it.
+// the same PROBES pairs of consecutive particles and takes them for unordered
+// when more than half of the pairs lie in different tiles along two axes or three: in any order by cell a step goes
+// along one axis, also where the particles are so sparse that it leaves the tile (1 M onto 256^3 in cell order: with
+// one axis counted they were grouped, 98 us for 71).  The pairs are one from each of PROBES equal parts of the particles,
+// at a scattered place: equal distances fell on the ends of the rows of a lattice of 2^k a side.  (1024 pairs took
+// 2 us: every lane reads lines of its own.)  Returns whether to group; workgroup 0 notes it.
+constexpr int PROBES = 256;
 __device__ __forceinline__ bool sup_probe(const SupArgs& a, Blk B) {
     if (!a.sel) return true;
-    const long long p = (a.n - 1) * (long long)threadIdx.x / PT;   // pair (p, p + 1), p < n - 1
     const float inv = (float)a.inv;
-    bool diff = false;
-    if (p + 1 < a.n) {
+    int diff = 0;
+    if (threadIdx.x < PROBES) {
+        const unsigned long long lo = (a.n - 1) * (long long)threadIdx.x / PROBES,
+                                 hi = (a.n - 1) * (long long)(threadIdx.x + 1) / PROBES;
+        const unsigned long long p = lo + ((threadIdx.x * 2654435761u) * (hi - lo) >> 32);   // lo <= p < hi <= n - 1
         const float* r = a.pos + 3 * p;
 #pragma unroll
-        for (int c = 0; c < 3; ++c) diff |= sup_cell(r[c], inv, a.N) / TILE != sup_cell(r[3 + c], inv, a.N) / TILE;
+        for (int c = 0; c < 3; ++c) diff += sup_cell(r[c], inv, a.N) / TILE != sup_cell(r[3 + c], inv, a.N) / TILE ? 1 : 0;
     }
-    const bool group = 2 * __syncthreads_count(diff) > PT;
+    const bool group = 2 * __syncthreads_count(diff >= 2) > PROBES;
     if (B.x == 0 && threadIdx.x == 0) *a.sel = group ? 1u : 0u;
     return group;
 }
+static_assert(PROBE_MIN > PROBES, "a pair in every part");
 
 __device__ __forceinline__ void sup_count_body(const SupArgs& a, Blk B) {
     __shared__ unsigned h[SUPMAX];
-    if (!sup_probe(a, B) || (int)B.x >= a.nb) return;
     const int tid = threadIdx.x;
+    for (long long i = (long long)B.x * PT + tid; i < a.nclr; i += (long long)B.gx * PT) a.clr[i] = 0u;
+    if (!sup_probe(a, B) || (int)B.x >= a.nb) return;
     for (int i = tid; i < a.nsup; i += PT) h[i] = 0u;
     __syncthreads();
     long long s0, s1;
@@ -769,7 +778,7 @@ __device__ __forceinline__ void sup_count_body(const SupArgs& a, Blk B) {
             if (sp[k] >= 0) atomicAdd(&h[sp[k]], 1u);
     }
     __syncthreads();
-    for (int i = tid; i < a.nsup; i += PT) a.cnt[(long long)B.x * a.nsup + i] = h[i];
+    for (int i = tid; i < a.nsp; i += PT) a.cnt[(long long)B.x * a.nsp + i] = i < a.nsup ? h[i] : 0u;
 }
 
 __global__ __launch_bounds__(PT) void k_sup_count(SupArgs a) { sup_count_body(a, own_blk()); }
@@ -779,37 +788,32 @@ __global__ __launch_bounds__(PT) void k_sup_count_b(const SupArgs* __restrict__ 
     sup_count_body(tab[bj_], blk_);
 }
 
-// columns [64 bx, 64 bx + 64) of cnt: exclusive sums down the rows in place, and the column totals; the rows
-// are split over the 16 waves
-__device__ __forceinline__ void sup_scan_body(const SupArgs& a, unsigned bx) {
-    __shared__ unsigned wsum[16][64];
-    if (a.sel && !*a.sel) return;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int c = (int)bx * 64 + lane;
-    const int per = (a.nb + 15) / 16, r0 = min(a.nb, wv * per), r1 = min(a.nb, r0 + per);
-    constexpr int PER = SUPBLOCKS / 16;   // all rows of a wave are loaded before the first is used
-    unsigned s = 0u, v[PER];
-#pragma unroll
-    for (int j = 0; j < PER; ++j) v[j] = c < a.nsup && r0 + j < r1 ? a.cnt[(long long)(r0 + j) * a.nsup + c] : 0u;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) s += v[j];
-    wsum[wv][lane] = s;
-    __syncthreads();
-    if (c >= a.nsup) return;
-    unsigned run = 0u;
-    for (int j = 0; j < wv; ++j) run += wsum[j][lane];
-    if (wv == 15) a.tot[c] = run + s;
-#pragma unroll
-    for (int j = 0; j < PER; ++j) {
-        if (r0 + j < r1) a.cnt[(long long)(r0 + j) * a.nsup + c] = run;
-        run += v[j];
+// First slots of the groups for workgroup bx: where a group begins, plus what the workgroups before bx put there; thread
+// g's return value is group g's.  Every workgroup sums the whole table of counts (up to 1 MB, from L2): as long as a launch
+// of its own took, and ordered particles, which need none of this, save that launch.  sc: LDS for 2 x 32 x 4 PT / 4 words.
+__device__ __forceinline__ unsigned sup_first(const SupArgs& a, unsigned bx, unsigned* sc, unsigned* wsum) {
+    const int tid = threadIdx.x, q4 = a.nsp / 4, parts = min(PT / q4, 32);
+    const int part = tid / q4, c4 = tid % q4;
+    if (part < parts) {
+        uint4 t = make_uint4(0u, 0u, 0u, 0u), b = t;
+#pragma unroll 8
+        for (int r = part; r < a.nb; r += parts) {
+            const uint4 v = ((const uint4*)(a.cnt + (long long)r * a.nsp))[c4];
+            const unsigned m = r < (int)bx ? ~0u : 0u;
+            t.x += v.x, t.y += v.y, t.z += v.z, t.w += v.w;
+            b.x += v.x & m, b.y += v.y & m, b.z += v.z & m, b.w += v.w & m;
+        }
+        ((uint4*)sc)[part * q4 + c4] = t;
+        ((uint4*)sc)[(parts + part) * q4 + c4] = b;
     }
-}
-__global__ __launch_bounds__(1024) void k_sup_scan(SupArgs a) { sup_scan_body(a, blockIdx.x); }
-// batched: job blockIdx.y
-__global__ __launch_bounds__(1024) void k_sup_scan_b(const SupArgs* __restrict__ tab) {
-    const SupArgs& a = tab[blockIdx.y];
-    sup_scan_body(a, blockIdx.x);
+    __syncthreads();
+    unsigned tot = 0u, before = 0u;
+    if (tid < a.nsup)
+        for (int p = 0; p < parts; ++p) {
+            tot += sc[p * a.nsp + tid];
+            before += sc[(parts + p) * a.nsp + tid];
+        }
+    return block_exscan(tot, wsum) + before;
 }
 
 // A step's particles are put in group order in LDS and leave in runs of consecutive addresses (one store of
@@ -826,10 +830,8 @@ __device__ __forceinline__ void sup_scatter_body(const SupArgs& a, Blk B) {
     static_assert(SUPMAX == PT && PS <= 65536, "one group a thread");
     const int tid = threadIdx.x;
     if ((a.sel && !*a.sel) || (int)B.x >= a.nb) return;
-    // thread g's cursor: the first slot of group g (exclusive sum of the totals) plus what the workgroups before
-    // this one put there
-    unsigned cur = block_exscan(tid < a.nsup ? a.tot[tid] : 0u, wsum);
-    if (tid < a.nsup) cur += a.cnt[(long long)B.x * a.nsup + tid];
+    static_assert(PS * R >= 2 * 4 * PT, "the sums of the counts fit where the records come");
+    unsigned cur = sup_first(a, B.x, (unsigned*)rec, wsum);   // thread g's cursor: the workgroup's next slot in group g
     lc[tid] = 0u;
     long long s0, s1;
     sup_range(a, B.x, s0, s1);
@@ -916,6 +918,7 @@ struct Presort {
     const unsigned* sel = nullptr;
     const float* pos = nullptr;
     const float* W = nullptr;
+    bool cleared = false;   // the deposit's counters are cleared on the way
 };
 
 // Bucket layout of one deposit: class segment capacities of twice the expected count of a uniform
@@ -973,8 +976,7 @@ static int run_binned(const float* pos, const float* W, int64_t n, int dims, dou
     unsigned* ov_key = (unsigned*)(ov + 8 * (size_t)n);
     unsigned* gcls = (unsigned*)(ov + 12 * (size_t)n);
     float* grouped = (float*)(ov + 16 * (size_t)n + 64);
-    rc = zero_fill(cnt, sizeof(unsigned) * ncnt, st);
-    if (rc) return rc;
+    if (!ps.cleared && (rc = zero_fill(cnt, sizeof(unsigned) * ncnt, st))) return rc;
     {
         StageTimer tm("deposit_bin", st);
         BinArgs ba{pos, W, (long long)n, dims, nt, dims / BoxSize, fill, bucket, CT, {}, {}, ov_count, ov_idx, ov_key, rsd};
@@ -1062,7 +1064,7 @@ static int dispatch_s(const float* pos, const float* W, int64_t n, int dims, dou
 
 // supertiles: m whole tile columns (nt tiles along z) each, about SUPGROUPS of them and never more than
 // SUPMAX; sup_fill sets the geometry of a presort (everything but the buffers), sup_words the unsigned words
-// of its counters (counts, totals, the order word)
+// of its counters (counts, the order word)
 static void sup_fill(SupArgs* a, int64_t n, int dims) {
     a->nt = (dims + TILE - 1) / TILE;
     const long long cols = (long long)a->nt * a->nt;
@@ -1071,24 +1073,30 @@ static void sup_fill(SupArgs* a, int64_t n, int dims) {
     // v * ceil(2^32 / m) >> 32 = v / m for v < cols: the rounding adds less than cols / 2^32 < 1 / m
     a->cmul = m == 1 ? 0u : (unsigned)(((1ULL << 32) + m - 1) / m);
     a->nsup = (int)((cols + m - 1) / m);
+    a->nsp = (a->nsup + 3) / 4 * 4;
     a->N = dims;
     a->n = n;
     a->nb = (int)std::max<int64_t>(1, std::min<int64_t>(SUPBLOCKS, (n + PT * PKP - 1) / (PT * PKP)));
 }
-static size_t sup_words(const SupArgs& a) { return (size_t)(a.nb + 1) * a.nsup + 4; }
+static size_t sup_words(const SupArgs& a) { return (size_t)a.nb * a.nsp + 4; }
 static void sup_carve(SupArgs* a, unsigned* w) {
     a->cnt = w;
-    a->tot = w + (size_t)a->nb * a->nsup;
 }
 
 // groups the particles by supertile into library workspaces (ps->pos, ps->W); the redshift-space shift
 // is applied on the way, so the grouped copy is deposited without it.  probe: only when they are in no
-// spatial order, which the device decides (ps->sel)
-static int presort(const float* pos, const float* W, int64_t n, int dims, double BoxSize, const Rsd& rsd, bool probe,
-                   hipStream_t st, Presort* ps) {
-    int rc = OK;
+// spatial order, which the device decides (ps->sel).  The count clears the deposit's counters, so that ordered
+// particles cost no more launches than the clear, the three of the overflow grouping and the rest once did.
+static int presort(const float* pos, const float* W, int64_t n, int dims, double BoxSize, int scheme, const Rsd& rsd,
+                   bool probe, hipStream_t st, Presort* ps) {
     SupArgs a{};
     sup_fill(&a, n, dims);
+    Layout L;
+    int rc = layout_of(n, dims, scheme, W != nullptr, &L);
+    if (rc) return rc;
+    a.clr = (unsigned*)workspace(WS_BINS, L.cnt_bytes, &rc);
+    if (rc) return rc;
+    a.nclr = (long long)L.ncnt;
     unsigned* words = (unsigned*)workspace(WS_SUP, sizeof(unsigned) * sup_words(a), &rc);
     if (rc) return rc;
     float* sp = (float*)workspace(WS_STAGE, sizeof(float) * (size_t)n * (W ? 4 : 3) + 64, &rc);
@@ -1100,10 +1108,9 @@ static int presort(const float* pos, const float* W, int64_t n, int dims, double
     a.rsd = rsd;
     a.spos = sp;
     a.sw = W ? sp + 3 * n : nullptr;
-    a.sel = probe ? a.tot + a.nsup : nullptr;
+    a.sel = probe ? a.cnt + (size_t)a.nb * a.nsp : nullptr;
     StageTimer tm("deposit_presort", st);
     hipLaunchKernelGGL(k_sup_count, dim3((unsigned)a.nb), dim3(PT), 0, st, a);
-    hipLaunchKernelGGL(k_sup_scan, dim3((unsigned)((a.nsup + 63) / 64)), dim3(1024), 0, st, a);
     if (W)
         hipLaunchKernelGGL((k_sup_scatter<true>), dim3((unsigned)a.nb), dim3(PT), 0, st, a);
     else
@@ -1112,6 +1119,7 @@ static int presort(const float* pos, const float* W, int64_t n, int dims, double
     ps->sel = a.sel;
     ps->pos = sp;
     ps->W = a.sw;
+    ps->cleared = true;
     return OK;
 }
 
@@ -1129,9 +1137,10 @@ int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double
     PYL_CHECK(n < (1LL << 31), E_UNSUPPORTED, "binned deposit: at most 2^31 particles per call");
     Rsd rsd = rsd_in;
     Presort ps;
-    if (sorted == PRESORT_PROBE && (rsd.vel || n < PROBE_MIN)) sorted = PRESORT_NO;
+    const long long nt = (dims + TILE - 1) / TILE, keys = nt * nt * nt * (scheme > 1 ? 8 : 1);
+    if (sorted == PRESORT_PROBE && (rsd.vel || n < PROBE_MIN || keys < PROBE_KEYS)) sorted = PRESORT_NO;
     if (sorted) {
-        const int rc = presort(pos, W, n, dims, BoxSize, rsd_in, sorted == PRESORT_PROBE, st, &ps);
+        const int rc = presort(pos, W, n, dims, BoxSize, scheme, rsd_in, sorted == PRESORT_PROBE, st, &ps);
         if (rc && !(sorted == PRESORT_PROBE && rc == E_ALLOC)) return rc;
         if (rc) ps = Presort();   // no room for the grouped copy: deposit the particles as they are
         if (!rc && sorted == PRESORT_YES) {
@@ -1139,6 +1148,7 @@ int deposit_binned(const float* pos, const float* W, int64_t n, int dims, double
             W = ps.W;
             rsd = Rsd();
             ps = Presort();
+            ps.cleared = true;
         }
     }
     auto run = [&](const Presort& q) -> int {
@@ -1249,7 +1259,6 @@ static int batch_launch_s(bool sorted, const BinnedTables& t, hipStream_t st) {
     if (sorted) {
         StageTimer tm("deposit_presort", st);
         hipLaunchKernelGGL(k_sup_count_b, dim3(t.sup_total), dim3(PT), 0, st, t.sup, t.sup_start, t.nj);
-        hipLaunchKernelGGL(k_sup_scan_b, dim3(SUPMAX / 64, nj), dim3(1024), 0, st, t.sup);
         hipLaunchKernelGGL((k_sup_scatter_b<HASW>), dim3(t.sup_total), dim3(PT), 0, st, t.sup, t.sup_start, t.nj);
         PYL_HIP(hipGetLastError());
     }

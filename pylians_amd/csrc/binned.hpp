@@ -75,14 +75,16 @@ struct SupArgs {
     int N, nt;
     unsigned cmul;   // supertile of tile column v = tx * nt + ty: v * cmul >> 32 (cmul = 0: v itself)
     int nsup;
+    int nsp;         // nsup rounded up to 4: words of a row of counts
     int nb;          // workgroups of the count and of the scatter; each owns a contiguous range of the particles
     double inv;
     Rsd rsd;
-    unsigned* cnt;   // [nb][nsup] particles of each workgroup per supertile, then their exclusive sums down a column
-    unsigned* tot;   // [nsup] particles per supertile
+    unsigned* cnt;   // [nb][nsp] particles of each workgroup per supertile
     float* spos;     // [n * 3] grouped positions (redshift-space shift applied)
     float* sw;       // [n] grouped weights (HASW)
     unsigned* sel = nullptr;   // [1] nullable: written by the count, 1 = the particles were grouped
+    unsigned* clr = nullptr;   // [nclr] nullable: the deposit's counters, cleared by the count
+    long long nclr = 0;
 };
 
 // One job of a batched binned deposit (overdensity output): the arguments of every stage and
