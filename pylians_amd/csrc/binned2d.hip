@@ -278,15 +278,16 @@ __global__ __launch_bounds__(MT) void k_map_tile(MapArgs a) {
 // 96 with 32; 4 M onto 700^2, 121 tiles of 64: 99 with 64, 74 with 32)
 static int map_tile_edge(int N) { return N <= 256 ? 16 : (N <= 832 ? 32 : (N <= 2048 ? 64 : 128)); }
 
-constexpr double MAP_ATOMICS = 460e3;
-constexpr double MAP_CELL = 0.05;
-
-// The direct kernel takes n S^2 / 21e9 s; this route 22 us of launches and 2.4 ps a cell, and then 8 to 25 ps a
-// particle.  Measured, direct / this in us: 1000^2 CIC 2^16 20 / 24, 2^17 33 / 24, 2^23 1612 / 101; 1000^2 PCS 2^14
-// 23 / 28, 2^15 35 / 29; 4000^2 CIC 2^17 50 / 64, 2^18 75 / 65, 2^23 1628 / 146; 64^2 TSC 2^23 6412 / 1171.
+// The direct kernel takes n S^2 / 21e9 s for unordered particles, and down to a third of that in pixel order (several
+// share a line; one cell a particle: less again); this route 22 us of launches and 2.4 ps a cell, and then 8 to 25 ps a
+// particle.  The line lies where particles in pixel order are even.  Measured, in pixel order (unordered), direct / this in us:
+// 250^2 CIC 160 k 24 / 24 (35 / 21), 500^2 PCS 80 k 28 / 27 (72 / 27), 1000^2 CIC 2^18 22 / 25 (52 / 23), 357 k 28 / 26
+// (72 / 24), 4000^2 CIC 441 k 73 / 62 (88 / 64); NGP 500^2 1.9 M 46 / 42 (94 / 32), 1000^2 2.0 M 43 / 43 (100 / 35), 4000^2
+// 5.0 M 115 / 112 (245 / 103); 2^23 onto 1000^2, CIC 1528 / 192 (1612 / 101).
 bool map_supported(int64_t n, int dims, int scheme) {
     if (dims < 32 || dims > 4096 || n >= (1LL << 31)) return false;
-    return (double)n * scheme * scheme >= MAP_ATOMICS + MAP_CELL * dims * dims;
+    const double cells = (double)dims * dims;
+    return (double)n * scheme * scheme >= (scheme == 1 ? 2.0e6 + 0.3 * cells : 1.25e6 + 0.03 * cells);
 }
 
 template <int S, typename G, bool HASW>

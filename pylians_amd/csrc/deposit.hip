@@ -183,13 +183,17 @@ static int dispatch_scheme(const float* pos, const float* W, int64_t n, int axes
 }
 
 // Ragged grids: whether the binned deposit is taken without being asked for.  The direct kernel's global
-// atomics run at 21 G/s whatever the grid; the binned one costs about 28 us of small launches, 4 ps a cell
-// (every cell is read and written) and 30 ps a particle.  Measured at 33 to 399 cells an edge, 2^12 to 2^23
-// unordered particles, direct / binned in us: 100^3 CIC 2^15 18 / 29, 2^16 30 / 30, 2^20 407 / 102;
-// 250^3 CIC 2^17 55 / 71, 2^18 106 / 78, 2^23 3209 / 301; 399^3 PCS 2^16 210 / 321, 2^18 822 / 368.
+// atomics run at 21 G/s on unordered particles, and two to three times that on ordered ones, of which several share a
+// line; the binned deposit costs about 25 us of small launches and 4 ps a cell (every cell is read and written), and on a
+// few tiles, which leave most of the chip idle, more with the cells of the stencil.  The line lies where lattices with
+// displacements, the direct kernel's best case, are even; there unordered and clustered particles gain up to 3 times.
+// Measured at 33 to 399 cells an edge, direct / binned in us: lattice 33^3 TSC 2^16 37 / 38, PCS 53 k 70 / 65, 50^3 TSC 65 k
+// 28 / 27, 60^3 CIC 168 k 25 / 25, 72^3 TSC 34 k 23 / 22, 100^3 CIC 95 k 24 / 23, 399^3 PCS 114 k 345 / 329; unordered
+// 250^3 CIC 2^18 106 / 78, 2^23 3211 / 239; clustered 100^3 CIC 2^17 82 / 45.
 static bool ragged_worth(int64_t n, int dims, int scheme) {
     const double cells = (double)dims * dims * dims, stencil = (double)scheme * scheme * scheme;
-    return (double)n * (stencil - 0.63) >= 600e3 + 0.085 * cells;
+    const double nt = (dims + 15) / 16, few = (scheme == 1 ? 7e6 : 70e6) / (nt * nt * nt);
+    return (double)n * (stencil - 0.63) >= 600e3 + 0.095 * cells + few;
 }
 
 int deposit(const float* pos, const float* W, int64_t n, int axes, int dims, double BoxSize, int scheme, int flags,

@@ -70,3 +70,29 @@ def test_groups(gpu, dims, n, weighted):
     g = torch.zeros((dims,) * 3, device="cuda")
     MAS_library.MA(pos, g, L, "CIC", W=W)
     assert np.all(np.abs(g.cpu().numpy() - o) <= RTOL * np.abs(o))
+
+
+def _stages(axes, dims, scheme, n):
+    from pylians_amd import MAS_library, _lib
+    pos = torch.rand((n, axes), device="cuda", generator=torch.Generator("cuda").manual_seed(1)) * L
+    g = torch.zeros((dims,) * axes, device="cuda")
+    try:
+        _lib.profile(True)
+        MAS_library.MA(pos, g, L, scheme)
+        torch.cuda.synchronize()
+        return set(_lib.profile_read())
+    finally:
+        _lib.profile(False)
+
+
+@pytest.mark.parametrize("axes, dims, scheme, n", [(2, 1000, "CIC", 255000), (2, 250, "PCS", 40000), (2, 500, "NGP", 945000),
+                                                   (3, 33, "PCS", 19000), (3, 40, "CIC", 115000), (3, 399, "PCS", 96600)])
+def test_direct_kernel_below_the_line(gpu, axes, dims, scheme, n):
+    """Ordered particles so few are quicker there; whether they are ordered the host cannot tell."""
+    assert "deposit_atomic" in _stages(axes, dims, scheme, n)
+
+
+@pytest.mark.parametrize("axes, dims, scheme, n", [(2, 1000, "CIC", 330000), (2, 500, "NGP", 2100000), (3, 33, "PCS", 53000),
+                                                   (3, 100, "CIC", 131072), (3, 399, "PCS", 113600)])
+def test_without_global_atomics_above_it(gpu, axes, dims, scheme, n):
+    assert ("deposit_map" if axes == 2 else "deposit_tiles") in _stages(axes, dims, scheme, n)
