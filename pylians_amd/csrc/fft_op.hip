@@ -72,14 +72,17 @@ template <int N, int NL, int T> struct Last {
 };
 
 // Keeps the compiler from rearranging what made v with what uses it.  The contraction of a butterfly's products into
-// fused multiply-adds depends on its surroundings; with its outputs settled the pass rounds as the plain one does.
+// fused multiply-adds depends on its surroundings; with its outputs settled the pass rounds as the plain one does
+// (two stages and more, with the compiler in use: tests/test_gpu_mode_equal.py compares the two bit for bit; 8 points,
+// one stage, round in their own way).
 template <typename R> __device__ __forceinline__ cplx<R> settle(cplx<R> v) {
     asm volatile("" : "+v"(v.x), "+v"(v.y));
     return v;
 }
 
-// The radix-5 butterfly of fft_engine.hpp with the fused operations of its two sums written out, as the plain passes
-// have them (left to the compiler, the other product was fused here)
+// The radix-5 butterfly of fft_engine.hpp with the fused operations of its two sums written out, as the compiler makes them
+// in the plain passes (here it fused the other product).  Named in the plain one instead, they changed the last
+// bits of every transform with a factor 5.
 template <typename R> __device__ __forceinline__ void dft5(cplx<R>* a) {
     const R c1 = (R)0.30901699437494742410229341718282, c2 = (R)-0.80901699437494742410229341718282;
     const R s1 = (R)0.95105651629515357211643933337938, s2 = (R)0.58778525229247312916870595463907;
