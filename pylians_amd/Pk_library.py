@@ -144,7 +144,7 @@ def IFFT3Dr_d(a, threads=1):
     return _fft_c2r(a, _lib.F64T, _lib.C128T, _lib.F64)
 
 
-@functools.lru_cache(maxsize=64, typed=True)   # typed: 64.0 is refused whether 64 was asked for before or not
+@functools.lru_cache(maxsize=64)
 def pk_layout(dims):
     """(kmax_par, kmax_per, kmax, out_len) of the pyl_pk output vector."""
     import ctypes
