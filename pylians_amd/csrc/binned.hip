@@ -197,29 +197,33 @@ __device__ __forceinline__ void bin_body(const BinArgs& a, Blk B) {
             if (base + cnt > first) hcnt[sl] = atomicAdd(&nov, base + cnt - first) - first;
         }
         __syncthreads();
-        if (nov) {
-            if (tid == 0) ovbase = atomicAdd(a.ov_count, nov);
-            __syncthreads();
-        }
 #pragma unroll
         for (int k = 0; k < KP; ++k) {
             if (key[k] < 0) continue;
-            const long long p = step * PS + k * BT + tid;
             const int c = key[k] & 7;
-            const unsigned sl = sr[k] & 0xffffu, idx = (unsigned)hkey[sl] + (sr[k] >> 16);
-            if (idx < (unsigned)scap[c]) {
-                float* r = a.bucket + ((long long)(key[k] >> 3) * a.CT + scofs[c] + idx) * R;
-                r[0] = x[k];
-                r[1] = y[k];
-                r[2] = z[k];
-                if (HASW) r[3] = w[k];
-            } else {
-                const unsigned o = ovbase + hcnt[sl] + idx;
-                a.ov_idx[o] = (unsigned long long)(idx - (unsigned)scap[c]) << 32 | (unsigned long long)p;
-                a.ov_key[o] = (unsigned)key[k];
-            }
+            const unsigned idx = (unsigned)hkey[sr[k] & 0xffffu] + (sr[k] >> 16);
+            if (idx >= (unsigned)scap[c]) continue;
+            float* r = a.bucket + ((long long)(key[k] >> 3) * a.CT + scofs[c] + idx) * R;
+            r[0] = x[k];
+            r[1] = y[k];
+            r[2] = z[k];
+            if (HASW) r[3] = w[k];
         }
         __syncthreads();
+        if (nov) {   // (here, behind the stores, the look at it costs least)
+            if (tid == 0) ovbase = atomicAdd(a.ov_count, nov);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < KP; ++k) {
+                if (key[k] < 0) continue;
+                const unsigned sl = sr[k] & 0xffffu, idx = (unsigned)hkey[sl] + (sr[k] >> 16), cap = (unsigned)scap[key[k] & 7];
+                if (idx < cap) continue;
+                const unsigned o = ovbase + hcnt[sl] + idx;
+                a.ov_idx[o] = (unsigned long long)(idx - cap) << 32 | (unsigned long long)(step * PS + k * BT + tid);
+                a.ov_key[o] = (unsigned)key[k];
+            }
+            __syncthreads();
+        }
         for (unsigned i = tid; i < nu; i += BT) {
             const int sl = hused[i];
             hkey[sl] = -1;
