@@ -80,6 +80,7 @@ struct SupArgs {
     double inv;
     Rsd rsd;
     unsigned* cnt;   // [nb][nsp] particles of each workgroup per supertile
+    unsigned* tot;   // [nsp] nullable: particles per supertile; cnt then holds exclusive sums down its columns (batches)
     float* spos;     // [n * 3] grouped positions (redshift-space shift applied)
     float* sw;       // [n] grouped weights (HASW)
     unsigned* sel = nullptr;   // [1] nullable: written by the count, 1 = the particles were grouped
