@@ -696,7 +696,10 @@ __global__ __launch_bounds__(TT) void k_tile_b(const TileArgs* __restrict__ tab,
 // k_bin then reads the grouped copy, where neighbouring particles share keys as in an ordered input.
 constexpr int PT = 1024;   // presort kernels: threads per workgroup
 constexpr int PKP = 8;    // particles per thread per step
-// PRESORT_PROBE: particles, and (tile, class) keys of the grid, from which the device looks for a spatial order
+// PRESORT_PROBE: particles, and (tile, class) keys of the grid, from which the device looks for a spatial order.  Unordered
+// particles, grouped / as they are, us: CIC 128^3 2^17 35 / 27, 2^19 43 / 43, 2^20 50 / 64, 256^3 2^18 75 / 71, 2^20 85 / 109;
+// at 2^20 and more 32^3 CIC (64 keys) 267 / 250, 64^3 NGP (64) 52 / 41, 48^3 CIC (216) 113 / 109, 64^3 CIC (512) 71 / 87,
+// 128^3 NGP (512) 41 / 44.  A look that finds an order costs 2.
 constexpr int64_t PROBE_MIN = 1 << 20;
 constexpr long long PROBE_KEYS = 512;
 // groups aimed at: more give k_bin fewer keys a step (3 M particles onto 320^3: 60 us with 128, 40 with 256, 29
