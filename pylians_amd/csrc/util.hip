@@ -291,7 +291,7 @@ size_t ws_arena_bytes(const WsArena* a) {
 // Workspaces of the deposits that may run on several streams at once (StreamScope): at most STREAM_WS sets a device.  A
 // further stream takes over the set used longest ago: nothing is freed and the host does not wait, its kernels run
 // behind the event of that set's last call.  A stream's own calls run in order and need no event (it costs a call of
-// 87 us 3), and a handle comes back only after its work (hipStreamDestroy waits for it), so the handle names the queue --
+// 87 us 4.6), and a handle comes back only after its work (hipStreamDestroy waits for it), so the handle names the queue --
 // except hipStreamPerThread, which is another queue in every thread: there the thread counts too, and as a
 // thread's id may come back as well, its calls always have the event.
 constexpr size_t STREAM_WS = 4;
@@ -380,7 +380,7 @@ StreamScope::StreamScope(hipStream_t s) : st(s) {
     ws->mu.lock();
     const Queue q(st);
     hipError_t e = hipSuccess;
-    if (mark && !ws->done) e = hipEventCreateWithFlags(&ws->done, hipEventDisableTiming | hipEventDisableSystemFence);
+    if (mark && !ws->done) e = hipEventCreateWithFlags(&ws->done, hipEventDisableTiming);
     if (e == hipSuccess && ws->state != StreamWs::FREE && (!(ws->last == q) || st == hipStreamPerThread))
         // OPEN: the only set of its time when it was used last; the first to take it over waits
         e = ws->state == StreamWs::MARKED ? hipStreamWaitEvent(st, ws->done, 0) : hipDeviceSynchronize();
